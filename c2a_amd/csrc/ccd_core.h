@@ -144,7 +144,9 @@ struct Entry {           // 160 B stack entry: a considered-but-undecided pair
   int32_t b1, b2;        // node indices (replayed leaf pairs: triangle indices)
   int32_t sg;            // (generation << 8) | (slot + 1) of cached values, 0 = none
   int32_t flags;         // bit0 leaf1, bit1 leaf2, bit2 root (always visited),
-                         // bit3 replayed record
+                         // bit3 replayed record, bit4 leaf pair with its values
+                         // (b1, b2: triangles; R[0..5]: closest points), bit5
+                         // triangle features set
   double dTri, mleaf;    // replayed leaf pairs: triangle distance, leaf time
   int32_t ar, cp;        // replayed: record number, expansion index of its children
   int32_t nn, lvl;       // record number in this step's log (-1 = unlogged), depth
@@ -229,7 +231,6 @@ template <int K, int CAP>
 struct Wave {
   Entry stack[CAP];
   Slot slot[Shape<K>::NSLOT];
-  Entry X;                   // root of the pending round
   double Rrel[9], Trel[3];   // model 2 in model 1's frame (leaf tests)
   double r1[9], tt1[3];      // current pose of object 1 (world directions)
   Motion mo[2];
@@ -258,6 +259,9 @@ struct Wave {
   int32_t nmr;               // misses gathered (then: covered by that round)
   int32_t mrrec[MR_MAX];     // their replayed record numbers, in scan order
   int32_t mrb[MR_MAX][2];    // and node ids
+  int32_t perm[64];          // heap scan: the heap pair at each visiting position
+  int32_t hit[64][2];        // contact enumeration: triangles of a heap's contacts
+  double p1[3], p2[3];       // closest points of the last improving leaf
 };
 
 // A mesh-table entry held in LDS, made wavefront-uniform so that node and
@@ -296,7 +300,6 @@ struct Leader {
   int numCA;
   int64_t bv, tri;
   int last1, last2, seed1, seed2;
-  double p1[3], p2[3];
   int sp;
   double toc;
   int flags;
@@ -528,33 +531,27 @@ C2A_HD bool ca_on_rss(const Motion& mo1, const double* r1, const double* R, cons
   const double la[2] = {A1->l[0], A1->l[1]}, lb[2] = {A2->l[0], A2->l[1]};
   const double rr = A1->r + A2->r;
   const double angR = A1->angR;
-  double d = rect_dist(R, T, la, lb, S);
-  d -= rr;
-  d = (d < 0.0) ? 0.0 : d;
   mtxv(tmp, r1, mo1.cv);
   mtxv(Vel, RL, tmp);
-  if (d == 0.0) {
-    mint = 0.0;
-    distance = 0.0;
-    return true;
-  }
-  mxv(tmp, RL, S);
-  mxv(Sw, r1, tmp);
-  double tocf = conserv_d(d, delta) / motion_bound_leaf(mo1, angR, Sw);
-  double total = tocf;
-  int it = 1;
-  while ((d >= delta) && (total <= mint) && (it < 50)) {
-    for (int i = 0; i < 3; i++) T2[i] = T[i] + Vel[i] * (-total);
-    d = rect_dist(R, T2, la, lb, S);
+  double total = 0.0;
+  for (int it = 0;;) {   // it: advancements made
+    for (int i = 0; i < 3; i++) T2[i] = it == 0 ? T[i] : T[i] + Vel[i] * (-total);
+    double d = rect_dist(R, T2, la, lb, S);
     d -= rr;
     d = (d < 0.0) ? 0.0 : d;
-    if (d == 0) break;
+    if (d == 0.0) {
+      if (it > 0) break;
+      mint = 0.0;
+      distance = 0.0;
+      return true;
+    }
     mxv(tmp, RL, S);
     mxv(Sw, r1, tmp);
-    tocf = conserv_d(d, delta) / motion_bound_leaf(mo1, angR, Sw);
+    const double tocf = conserv_d(d, delta) / motion_bound_leaf(mo1, angR, Sw);
+    if (it > 0 && tocf < delta) break;
+    total = it == 0 ? tocf : total + tocf;
     it++;
-    if (tocf < delta) break;
-    total += tocf;
+    if (!((d >= delta) && (total <= mint) && (it < 50))) break;
   }
   if (total < 1.0) {
     mint = total;
@@ -571,33 +568,32 @@ C2A_HD bool ca_on_tris(const Motion& mo1, const double* r1, const double* A, con
                        double delta, double& mint, double& distance) {
   double Vel[3], p[3], q[3], n[3], At[9];
   mtxv(Vel, r1, mo1.cv);
-  double d = tri_dist(p, q, A, B, nullptr);
-  sub3(n, q, p);
-  normalize3(n);
-  double u = dot3(Vel, n);
-  if (u <= 0) u = 1e-30;
-  if (d == 0) {
-    mint = 0.0;
-    distance = 0.0;
-    return true;
-  }
-  const double dt = conserv_d(d, delta) / u;
-  int it = 1;
-  if (dt >= mint) return false;
-  double total = dt;
-  while ((d > delta) && (total <= mint) && (it < 50)) {
+  double total = 0.0;
+  for (int it = 0;;) {   // it: advancements made
     for (int v = 0; v < 3; v++)
-      for (int i = 0; i < 3; i++) At[3 * v + i] = A[3 * v + i] + Vel[i] * total;
-    d = tri_dist(p, q, At, B, nullptr);
-    if (d == 0.0) break;
+      for (int i = 0; i < 3; i++)
+        At[3 * v + i] = it == 0 ? A[3 * v + i] : A[3 * v + i] + Vel[i] * total;
+    const double d = tri_dist(p, q, At, B, nullptr);
+    if (it > 0 && d == 0.0) break;
+    if (d == 0) {
+      mint = 0.0;
+      distance = 0.0;
+      return true;
+    }
     sub3(n, q, p);
     normalize3(n);
-    u = dot3(Vel, n);
+    double u = dot3(Vel, n);
     if (u <= 0) u = 1e-30;
-    const double tofc = conserv_d(d, delta) / u;
+    const double dt = conserv_d(d, delta) / u;
+    if (it == 0) {
+      if (dt >= mint) return false;
+      total = dt;
+    } else {
+      if (dt < delta) break;
+      total += dt;
+    }
     it++;
-    if (tofc < delta) break;
-    total += tofc;
+    if (!((d > delta) && (total <= mint) && (it < 50))) break;
   }
   if (total <= mint && total >= 0.0) {
     mint = total;
@@ -607,17 +603,18 @@ C2A_HD bool ca_on_tris(const Motion& mo1, const double* r1, const double* A, con
   return false;
 }
 
-// Heap slot h of the depth-K subtree below X: the pair reached by the path
-// bits of h+1, its transform chained from X, and its values.
-template <int K, int CAP, class RT>
-C2A_HD void compute_slot_below(Wave<K, CAP>& g, const RT* xR, const RT* xT, int b1, int b2, int h,
-                               const MeshDev& M1, const MeshDev& M2, bool contact, Slot& s) {
+// Heap slot h of the subtree below the heap's root pair: the pair reached by
+// the path bits of h+1, its transform chained from the root's, and its values.
+template <int K, int CAP>
+C2A_HD void compute_slot_below(Wave<K, CAP>& g, const Slot& root, int h, const MeshDev& M1,
+                               const MeshDev& M2, bool contact, Slot& s) {
+  int b1 = root.b1, b2 = root.b2;
   node_ptr N1 = nodes_of(M1);
   node_ptr N2 = nodes_of(M2);
   const int lvl = 31 - clz32((unsigned)(h + 1));
   double R[9], T[3];
-  for (int i = 0; i < 9; i++) R[i] = xR[i];
-  for (int i = 0; i < 3; i++) T[i] = xT[i];
+  for (int i = 0; i < 9; i++) R[i] = root.R[i];
+  for (int i = 0; i < 3; i++) T[i] = root.T[i];
   NodeHead h1 = head_of(N1 + b1), h2 = head_of(N2 + b2);
   for (int lv = 0; lv < lvl; lv++) {
     const int bit = ((h + 1) >> (lvl - 1 - lv)) & 1;
@@ -652,18 +649,6 @@ C2A_HD void compute_slot_below(Wave<K, CAP>& g, const RT* xR, const RT* xT, int 
                      g.mo[1], contact);
 }
 
-template <int K, int CAP>
-C2A_HD void compute_slot_into(Wave<K, CAP>& g, int h, const MeshDev& M1, const MeshDev& M2,
-                              bool contact, Slot& s) {
-  compute_slot_below(g, g.X.R, g.X.T, g.X.b1, g.X.b2, h, M1, M2, contact, s);
-}
-
-template <int K, int CAP>
-C2A_HD void compute_slot(Wave<K, CAP>& g, int h, const MeshDev& M1, const MeshDev& M2,
-                         bool contact) {
-  compute_slot_into(g, h, M1, M2, contact, g.slot[h]);
-}
-
 // Heap slot h of the round written as arena record 2 * rpb + h, so that the
 // pair stays available for the rest of the step; slots above the last level
 // link their children (pair rpb + h).
@@ -671,7 +656,7 @@ template <int K, int CAP>
 C2A_HD void compute_slot_arena(Wave<K, CAP>& g, int h, const MeshDev& M1, const MeshDev& M2,
                                const ArenaView& av) {
   Slot s;
-  compute_slot_into(g, h, M1, M2, false, s);
+  compute_slot_below(g, g.slot[0], h, M1, M2, false, s);
   if (!s.valid) return;   // below a leaf pair: never referenced
   const int rpb = g.rpb;
   const int rec = 2 * rpb + h;
@@ -697,45 +682,37 @@ C2A_HD void compute_slot_arena(Wave<K, CAP>& g, int h, const MeshDev& M1, const 
   gp(av.hot)[rec] = hr;
 }
 
+// Arena-backed rounds: only the host-side harness runs them (the library
+// keeps them off), so the device code leaves the path out.
+C2A_HD bool arena_rounds_on(const KArgs& a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return false;
+#else
+  return a.arena_rounds != 0;
+#endif
+}
+
 // One lane's share of a round.
 template <int K, int CAP>
 C2A_HD void round_lane(Wave<K, CAP>& g, const Leader& L, int lane, int nl, const KArgs& a) {
   const MeshDev M1 = mesh_of(g, 0);
   const MeshDev M2 = mesh_of(g, 1);
   const bool contact = g.contact != 0;
-  if ((g.X.flags & 3) == 3) {
-    if (lane == 0) {
-      Slot& s = g.slot[0];
-      s.b1 = g.X.b1;
-      s.b2 = g.X.b2;
-      s.flags = 3;
-      s.valid = 1;
-      leaf_values(s, M1, M2, g.Rrel, g.Trel, g.r1, g.tt1, g.mo[0], g.mo[1], g.X.b1, g.X.b2,
-                  contact);
-    }
-    return;
-  }
-  if (g.rarena) {
+  if (arena_rounds_on(a) && g.rarena) {
     const ArenaView av = arena_view(L.ab, a.logcap);
     for (int h = lane + 1; h < Shape<K>::NSLOT; h += nl) compute_slot_arena(g, h, M1, M2, av);
     return;
   }
+  // one heap of g.rdepth levels below slot 0 (a leaf pair: its own values), or
+  // heap r in slots [r * mp, r * mp + mp - 1) below gathered miss r
   const int mp = g.mpage;
-  if (mp) {
-    // heap r (slots [r * mp, r * mp + mp - 1)) below gathered miss r, whose
-    // transform is its replayed record's
-    const ArenaView av = arena_view(L.ab, a.logcap);
-    const int nr = g.nmr;
-    for (int h = lane; h < nr * mp; h += nl) {
-      const int r = h / mp, l = h - r * mp;
-      if (l == 0 || l == mp - 1) continue;   // the miss itself; padding
-      const double C2A_GLOBAL* xf = gp(av.xf) + 12 * (int64_t)g.mrrec[r];
-      compute_slot_below(g, xf, xf + 9, g.mrb[r][0], g.mrb[r][1], l, M1, M2, contact, g.slot[h]);
-    }
-    return;
+  const bool own = !mp && (g.slot[0].flags & 3) == 3;
+  const int n = mp ? g.nmr * mp : (own ? 1 : (2 << g.rdepth) - 1);
+  for (int h = lane + (own ? 0 : 1); h < n; h += nl) {
+    const int l = mp ? h & (mp - 1) : h;
+    if (mp && (l == 0 || l == mp - 1)) continue;   // the miss itself; padding
+    compute_slot_below(g, g.slot[h - l], l, M1, M2, contact, g.slot[h]);
   }
-  const int nslot = (2 << g.rdepth) - 1;   // levels 0..rdepth of the heap
-  for (int h = lane + 1; h < nslot; h += nl) compute_slot(g, h, M1, M2, contact);
 }
 
 template <int K, int CAP>
@@ -747,60 +724,62 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
     gen = 1;
     if (lane == 0) g.mrgen = -1;
   }
-  const int flags = e.flags;
-  const int ar = e.ar;
+  const int flags = uni(e.flags);
+  const int ar = uni(e.ar);
   const int sg = (gen << 8) | 1;
-  lane_sync();
-  const uint64_t* s = reinterpret_cast<const uint64_t*>(&e);
-  uint64_t* x = reinterpret_cast<uint64_t*>(&g.X);
-  if (flags & 8) {
-    C2A_CHECK(ar >= 0 && ar < arena_records(a.logcap));
-    // replayed pair: the transform is in the arena
-    const uint64_t C2A_GLOBAL* xf = gp(reinterpret_cast<const uint64_t*>(
-        arena_view(L.ab, a.logcap).xf + 12 * (int64_t)ar));
-    for (int w = lane; w < 16; w += nl) x[w] = w < 12 ? xf[w] : s[w];
-  } else {
-    for (int w = lane; w < 16; w += nl) x[w] = s[w];
-  }
-  lane_sync();
   // internal pairs of a CA step go to the arena while it has room
   constexpr int NPAIR = (1 << K) - 1;
-  const bool to_arena = a.arena_rounds && !a.scorer.on && a.logcap > 0 && !g.contact &&
+  const bool to_arena = arena_rounds_on(a) && !a.scorer.on && a.logcap > 0 && !g.contact &&
                         (flags & 3) != 3 && L.napp + NPAIR <= 2 * a.logcap;
   // a miss the scan found with more misses after it in its window: one
   // shallow heap below each (the same slots a round below each would fill)
   const int mpage = 2 << L.kmiss;
+  const int nmr = uni(g.nmr);
   const bool multi = !to_arena && (flags & 8) && (flags & 3) != 3 && L.kmiss > 0 &&
-                     L.kmiss < L.kdepth && 2 * mpage <= Shape<K>::NSLOT + 1 && g.nmr > 1 &&
-                     ar == g.mrrec[0];
+                     L.kmiss < L.kdepth && 2 * mpage <= Shape<K>::NSLOT + 1 && nmr > 1 &&
+                     ar == uni(g.mrrec[0]);
+  const int cap = (Shape<K>::NSLOT + 1) / mpage;
+  const int nroot = nmr < cap ? nmr : cap;
   lane_sync();
+  // the heaps' root pairs into their slots; replayed pairs' transforms are in
+  // the arena
+  const uint64_t C2A_GLOBAL* xf =
+      gp(reinterpret_cast<const uint64_t*>(arena_view(L.ab, a.logcap).xf));
+  if (multi) {
+    for (int w = lane; w < 12 * nroot; w += nl) {
+      const int r = w / 12, k = w - 12 * r;
+      C2A_CHECK(g.mrrec[r] >= 0 && g.mrrec[r] < arena_records(a.logcap));
+      reinterpret_cast<uint64_t*>(&g.slot[r * mpage])[k] = xf[12 * (int64_t)g.mrrec[r] + k];
+    }
+    for (int r = lane; r < nroot; r += nl) {
+      g.slot[r * mpage].b1 = g.mrb[r][0];
+      g.slot[r * mpage].b2 = g.mrb[r][1];
+    }
+  } else {
+    C2A_CHECK(!(flags & 8) || (ar >= 0 && ar < arena_records(a.logcap)));
+    const uint64_t* s = reinterpret_cast<const uint64_t*>(&e);
+    uint64_t* x = reinterpret_cast<uint64_t*>(&g.slot[0]);
+    for (int w = lane; w < 15; w += nl)
+      x[w] = ((flags & 8) && w < 12) ? xf[12 * (int64_t)ar + w] : s[w];
+  }
   if (lane == 0) {
-    if (multi) {
-      g.rarena = 0;
-      e.sg = sg;               // heap 0, slot 0: the miss being walked
-      g.gen = gen;
-      g.mrgen = gen;
-      g.mpage = mpage;
-      g.rdepth = L.kmiss;
-      const int cap = (Shape<K>::NSLOT + 1) / mpage;
-      if (g.nmr > cap) g.nmr = cap;
-    } else if (to_arena) {
-      g.rarena = 1;
+    g.rarena = to_arena ? 1 : 0;
+    g.mpage = multi ? mpage : 0;
+    if (to_arena) {
       g.rpb = L.napp;
       e.cp = L.napp;
       e.flags = flags | 8;
     } else {
-      g.rarena = 0;
-      g.mpage = 0;
-      e.sg = sg;
-      Slot& s0 = g.slot[0];
-      s0.b1 = g.X.b1;
-      s0.b2 = g.X.b2;
-      s0.d = g.X.d;
-      s0.mt = g.X.mt;
-      s0.flags = flags & 3;
-      s0.valid = 1;
+      e.sg = sg;   // heap 0, slot 0
       g.gen = gen;
+    }
+    if (multi) {
+      g.mrgen = gen;
+      g.rdepth = L.kmiss;
+      g.nmr = nroot;
+    } else {
+      g.slot[0].flags = flags & 3;
+      g.slot[0].valid = 1;
       // a replayed pair that must now be expanded (a miss) usually needs
       // only a level or two: a shallow first round has a shorter chain of
       // dependent node loads
@@ -915,9 +894,26 @@ C2A_HD int lane_bcast(int v, int src) {
   return v;
 #endif
 }
-C2A_HD double lane_bcastd(double v, int src) {
+// v of lane `src`, the same in every lane (a scalar read, where lane_bcast
+// goes through the LDS crossbar).
+C2A_HD int lane_read(int v, int src) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  return __shfl(v, src);
+  return __builtin_amdgcn_readlane(v, __builtin_amdgcn_readfirstlane(src));
+#elif defined(C2A_EMU_SIMT)
+  return simt::bcast(v, src);
+#else
+  (void)src;
+  return v;
+#endif
+}
+C2A_HD double lane_readd(double v, int src) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int s = __builtin_amdgcn_readfirstlane(src);
+  union { double d; int32_t i[2]; } u;
+  u.d = v;
+  u.i[0] = __builtin_amdgcn_readlane(u.i[0], s);
+  u.i[1] = __builtin_amdgcn_readlane(u.i[1], s);
+  return u.d;
 #elif defined(C2A_EMU_SIMT)
   return simt::bcastd(v, src);
 #else
@@ -925,15 +921,43 @@ C2A_HD double lane_bcastd(double v, int src) {
   return v;
 #endif
 }
-// max over lanes below this one (0 for lane 0)
+// v of the neighbouring lane (lane ^ 1)
+C2A_HD double lane_xor1d(double v, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  (void)lane;
+  union { double d; int32_t i[2]; } u;
+  u.d = v;   // quad_perm [1, 0, 3, 2]
+  u.i[0] = __builtin_amdgcn_update_dpp(0, u.i[0], 0xB1, 0xf, 0xf, false);
+  u.i[1] = __builtin_amdgcn_update_dpp(0, u.i[1], 0xB1, 0xf, 0xf, false);
+  return u.d;
+#elif defined(C2A_EMU_SIMT)
+  return simt::bcastd(v, lane ^ 1);
+#else
+  (void)lane;
+  return v;
+#endif
+}
+#if defined(__HIP_DEVICE_COMPILE__)
+// Cross-lane data movement inside the vector ALU (DPP): a shuffle through
+// the LDS crossbar takes about 130 cycles, a DPP move about 8.  Six steps
+// reach all 64 lanes: row shifts by 1, 2, 4, 8 within 16 lanes, then lane 15
+// of each row to the next one and lane 31 to the upper half.  Lanes without
+// a source keep `old`.
+#define C2A_DPP_STEPS(X) \
+  X(0x111, 0xf) X(0x112, 0xf) X(0x114, 0xf) X(0x118, 0xf) X(0x142, 0xa) X(0x143, 0xc)
+#endif
+// max over lanes below this one (0 for lane 0); v >= 0
 C2A_HD int excl_prefix_max(int v, int lane) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(v, (unsigned)o);
-    if (lane >= o) v = v > u ? v : u;
+  (void)lane;
+#define C2A_STEP(ctrl, rows)                                            \
+  {                                                                     \
+    const int u = __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false); \
+    v = v > u ? v : u;                                                  \
   }
-  const int x = __shfl_up(v, 1u);
-  return lane == 0 ? 0 : x;
+  C2A_DPP_STEPS(C2A_STEP)
+#undef C2A_STEP
+  return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false);   // one lane up
 #elif defined(C2A_EMU_SIMT)
   (void)lane;
   return simt::excl_prefix_max(v);
@@ -943,23 +967,38 @@ C2A_HD int excl_prefix_max(int v, int lane) {
   return 0;
 #endif
 }
+// Smallest v of the wavefront, the same in every lane.  A NaN counts as no
+// value, as in the reference's sequential `if (v < min) min = v`.
 C2A_HD double wave_mind(double v) {
+  v = v < 1.0 / 0.0 ? v : 1.0 / 0.0;
 #if defined(__HIP_DEVICE_COMPILE__)
-  for (int o = 32; o >= 1; o >>= 1) {
-    const double u = __shfl_xor(v, o);
-    v = u < v ? u : v;
+#define C2A_STEP(ctrl, rows)                                                      \
+  {                                                                               \
+    union { double d; int32_t i[2]; } x, u;                                       \
+    x.d = v;                                                                      \
+    u.i[0] = __builtin_amdgcn_update_dpp(x.i[0], x.i[0], ctrl, rows, 0xf, false); \
+    u.i[1] = __builtin_amdgcn_update_dpp(x.i[1], x.i[1], ctrl, rows, 0xf, false); \
+    v = u.d < v ? u.d : v;                                                        \
   }
+  C2A_DPP_STEPS(C2A_STEP)
+#undef C2A_STEP
+  return lane_readd(v, 63);
 #elif defined(C2A_EMU_SIMT)
   v = simt::mind(v);
 #endif
   return v;
 }
+// Largest v of the wavefront (v >= 0), the same in every lane.
 C2A_HD int wave_maxi(int v) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  for (int o = 32; o >= 1; o >>= 1) {
-    const int u = __shfl_xor(v, o);
-    v = u > v ? u : v;
+#define C2A_STEP(ctrl, rows)                                            \
+  {                                                                     \
+    const int u = __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false); \
+    v = v > u ? v : u;                                                  \
   }
+  C2A_DPP_STEPS(C2A_STEP)
+#undef C2A_STEP
+  return lane_read(v, 63);
 #elif defined(C2A_EMU_SIMT)
   v = simt::maxi(v);
 #endif
@@ -1417,11 +1456,11 @@ C2A_HD int scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
     }
     lane_sync();
     if (stop < n) {
-      const double sd = lane_bcastd(E.d, stop), smt = lane_bcastd(E.mt, stop);
-      const double sdt = lane_bcastd(E.dTri, stop), sml = lane_bcastd(E.mleaf, stop);
-      const int sb1 = lane_bcast(E.b1, stop), sb2 = lane_bcast(E.b2, stop);
-      const int sinfo = lane_bcast(E.info, stop), srec = lane_bcast(E.rec, stop);
-      const int snn = lane_bcast(nn, stop);
+      const double sd = lane_readd(E.d, stop), smt = lane_readd(E.mt, stop);
+      const double sdt = lane_readd(E.dTri, stop), sml = lane_readd(E.mleaf, stop);
+      const int sb1 = lane_read(E.b1, stop), sb2 = lane_read(E.b2, stop);
+      const int sinfo = lane_read(E.info, stop), srec = lane_read(E.rec, stop);
+      const int snn = lane_read(nn, stop);
       L.spos = t0 + stop + 1;
       if ((sinfo & 3) == 3) {
         // improving leaf (C2A.cpp:1141-1183)
@@ -1566,9 +1605,11 @@ C2A_HD void push_back(Wave<K, CAP>& g, Leader& L, const Cur& c, int where, int c
 // a stack machine.  The pair being processed is held in registers; an
 // expansion pushes the child visited second and continues with the first,
 // so the stack holds exactly the reference's pending siblings.  Uniform
-// across lanes.  Returns true when a round has been requested.
+// across lanes.  Returns true when a round has been requested.  One pair at
+// a time: heaps of more than 64 pairs (K = 6) and the host-side harness's
+// one-lane and arena-round runs; the others take walk_heaps.
 template <int K, int CAP>
-C2A_HD bool walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+C2A_HD bool walk_pairs(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
   const int cmode = g.contact;
   const bool contact = cmode != 0;
   const bool learned = a.scorer.on && !contact;
@@ -1638,7 +1679,7 @@ C2A_HD bool walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
         if (imp) {
           L.D = dTri;
           L.pq_pending = 0;
-          for (int i = 0; i < 3; i++) { L.p1[i] = unid(sl.p[i]); L.p2[i] = unid(sl.q[i]); }
+          for (int i = lane; i < 3; i += nl) { g.p1[i] = sl.p[i]; g.p2[i] = sl.q[i]; }
           L.last1 = uni(sl.t1);
           L.last2 = uni(sl.t2);
         }
@@ -1647,7 +1688,7 @@ C2A_HD bool walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
         const double dTri = unid(sl.dTri);
         if (dTri < L.D) {
           L.D = dTri;
-          for (int i = 0; i < 3; i++) { L.p1[i] = unid(sl.p[i]); L.p2[i] = unid(sl.q[i]); }
+          for (int i = lane; i < 3; i += nl) { g.p1[i] = sl.p[i]; g.p2[i] = sl.q[i]; }
           L.last1 = uni(sl.t1);
           L.last2 = uni(sl.t2);
         }
@@ -1745,6 +1786,303 @@ C2A_HD bool walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
   }
 }
 
+// Whether the traversal enters a pair with RSS distance d and admissible
+// time mt at the current bound.  cmode: Wave::contact.
+C2A_HD bool enters(const Leader& L, int cmode, double d, double mt) {
+  if (cmode == 0)   // C2A.cpp:1284-1349
+    return mt < L.Up && ((d < (L.D - L.abs_err)) || (d * (1 + L.rel_err) < L.D));
+  if (L.mode == MODE_DISTANCE)   // C2A_PQP.cpp:594-617; C2A_Collide (:1068-1070):
+                                 // RectDist <= r1 + r2 exactly when the
+                                 // clamped RSS distance is 0
+    return ((d < (L.D - L.abs_err)) || (d * (1 + L.rel_err) < L.D)) && (cmode != 2 || d == 0.0);
+  return d < L.thr;   // contact enumeration, abs = rel = 0 (C2A.cpp:1760-1761)
+}
+
+// A tested leaf pair (C2A.cpp:1141-1183, C2A_PQP.cpp:493-520: strict <) with
+// triangle distance dTri; returns whether it becomes the closest one.
+C2A_HD bool leaf_update(Leader& L, int cmode, int strict, double dTri, double mleaf) {
+  if (cmode == 0) {
+    const bool imp = dTri <= L.D;
+    const double ml = leaf_time(dTri, mleaf, strict);
+    if ((imp || strict) && ml <= L.M) L.M = ml;
+    if (imp) L.D = dTri;
+    return imp;
+  }
+  const bool imp = dTri < L.D;
+  if (imp) L.D = dTri;
+  return imp;
+}
+
+// The reference DFS over the pairs of one speculative heap (slots base ..),
+// 64 decisions at a time: the walk of walk_pairs, decided like the scan.
+// x: the heap's root pair, which is being expanded.  Each lane takes one pair;
+// its visiting position follows from which child of each pair on its path
+// is the closer one (full subtree sizes: the heap is complete, pairs below a
+// leaf pair are invalid and decide nothing), and the pairs are permuted into
+// that order.  Decisions up to the first improving leaf or unexpanded pair
+// are final; after an improving leaf the rest is decided again with the new
+// bound.  Returns 1 when a pair at the heap's last level has to be expanded:
+// it and the pending siblings above it wait on the stack, as walk_pairs
+// would have left them.  Contact enumeration: nhit contacts in g.hit.
+//
+// Why: one pair at a time costs about 1.1 us on MI355X (some 2,600 cycles
+// of dependent LDS reads and uniform code, one useful lane), a heap of 62
+// pairs holds 8.6 visited ones on the heaviest knot query, and deciding the
+// heap takes two or three passes of about 400 instructions.
+template <int K, int CAP>
+C2A_HD int heap_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, const Cur& x, int base,
+                     int lane, int& nhit) {
+  const int cmode = uni(g.contact);
+  const bool counts = cmode != 0 && L.mode != MODE_DISTANCE;   // contact enumeration
+  const double inf = 1.0 / 0.0;
+  const int rd = uni(g.rdepth);
+  const int nloc = (2 << rd) - 2;   // pairs below x
+  const int j = lane & 63;
+  const bool in0 = j < nloc;
+  // heap index of this lane's pair: 1 .. nloc, odd = first child node
+  int loc = in0 ? j + 1 : 1;
+  int lv = 0, prank = 0;
+  {
+    C2A_CHECK(base + nloc < Shape<K>::NSLOT + 1);
+    const double d0 = g.slot[base + loc].d;
+    const double ds = lane_xor1d(d0, j);
+    const bool second = in0 && ((loc & 1) ? ds < d0 : !(d0 < ds));
+    const uint64_t sm = wave_ballot(second);
+    lv = 31 - clz32((unsigned)(loc + 1));
+    int r = 0;
+    for (int k = 1; k <= (K < 5 ? K : 5); k++) {
+      if (k <= lv) {
+        const int anc = ((loc + 1) >> (lv - k)) - 1;
+        const int late = (int)((sm >> (anc - 1)) & 1);
+        prank = r;
+        r += 1 + (late ? (2 << (rd - k)) - 1 : 0);
+      }
+    }
+    if (in0 && lane < 64) g.perm[r - 1] = loc | (prank << 8) | (lv << 16);
+    lane_sync();
+    if (in0) {
+      const int q = g.perm[j];
+      loc = q & 0xff;
+      prank = (q >> 8) & 0xff;
+      lv = q >> 16;
+    }
+  }
+  const Slot& s = g.slot[base + loc];
+  const bool valid = in0 && s.valid;
+  const double d = s.d, mt = s.mt;
+  const int b1 = s.b1, b2 = s.b2, fl = valid ? s.flags : 0;
+  const bool leaf = valid && (fl & 3) == 3;
+  const double dTri = leaf ? s.dTri : inf, mleaf = leaf ? s.mleaf : inf;
+  const int size = (2 << (rd - lv)) - 1;
+  const bool bottom = lv == rd;
+  // log the expansion of x for the next step's replay, then the heap's
+  const ArenaView av = arena_view(L.ab, a.logcap);
+  LogEnt C2A_GLOBAL* lw = gp(L.logbuf ? av.log1 : av.log0);
+  int enx = -1;
+  if (x.nn >= 0 && L.nlog < L.klog) {
+    enx = L.nlog++;
+    if (lane == 0) {
+      LogEnt v;
+      v.rec = x.nn;
+      v.b1 = x.b1;
+      v.b2 = x.b2;
+      v.level = x.lvl;
+      lw[enx] = v;
+    }
+  }
+  bool logging = enx >= 0;
+  if (!counts) L.bv += 2;
+  int en = -1, pos = 0, ret = 0;
+  for (;;) {
+    const bool live = valid && j >= pos;
+    const bool desc = live && enters(L, cmode, d, mt);
+    // a pruned pair's subtree is passed over (a leaf pair's is invalid)
+    const int covered = excl_prefix_max((live && !leaf && !desc) ? j + size : 0, j);
+    const bool active = live && j >= covered;
+    const bool miss = active && !leaf && desc && bottom;
+    const bool tested = active && leaf && desc;
+    const bool improving = tested && !counts && (cmode ? dTri < L.D : dTri <= L.D);
+    const uint64_t stopm = wave_ballot(miss || improving);
+    const int stop = stopm ? (int)__builtin_ctzll(stopm) : 64;
+    const bool in = active && j < stop;
+    const bool expand = in && !leaf && desc;
+    if (cmode == 0) {
+      // pruned pairs lower mint (C2A.cpp:1284-1349, `else if`); in strict
+      // mode so do the tested leaves
+      const double mc = wave_mind((in && !desc)                ? mt
+                                  : (a.strict && in && tested) ? leaf_time(dTri, mleaf, 1)
+                                                               : inf);
+      if (mc < L.M) L.M = mc;
+    }
+    const uint64_t em = wave_ballot(expand);
+    const int nexp = (int)__builtin_popcountll(em);
+    if (!counts) {
+      L.bv += 2 * nexp;
+      L.tri += (int)__builtin_popcountll(wave_ballot(in && tested));
+    } else {
+      const bool hit = in && tested && (fl & 4) && dTri <= L.thr;
+      const uint64_t hm = wave_ballot(hit);
+      if (hit && lane < 64) {
+        g.hit[lanes_below(hm, j)][0] = s.t1;
+        g.hit[lanes_below(hm, j)][1] = s.t2;
+      }
+      nhit = (int)__builtin_popcountll(hm);
+    }
+    if (logging && L.nlog + nexp > L.klog) logging = false;
+    if (expand && logging) en = L.nlog + lanes_below(em, j);
+    if (logging) L.nlog += nexp;
+    const int pen_in = lane_bcast(en, prank > 0 ? prank - 1 : 0);
+    const int pen = prank > 0 ? pen_in : enx;
+    const int nn = pen < 0 ? -1 : 2 * pen + 1 + ((loc - 1) & 1);
+    if (expand && logging && lane < 64) {
+      LogEnt v;
+      v.rec = nn;
+      v.b1 = b1;
+      v.b2 = b2;
+      v.level = x.lvl + lv;
+      lw[en] = v;
+    }
+    if (!stopm) break;
+    if (lane_read(leaf ? 1 : 0, stop)) {
+      const Slot& t = g.slot[base + lane_read(loc, stop)];
+      leaf_update(L, cmode, a.strict, unid(t.dTri), unid(t.mleaf));
+      L.pq_pending = 0;
+      if (lane < 3) { g.p1[lane] = t.p[lane]; g.p2[lane] = t.q[lane]; }
+      L.last1 = uni(t.t1);
+      L.last2 = uni(t.t2);
+      L.tri++;
+      pos = stop + 1;
+      continue;
+    }
+    // The second children whose sibling's subtree holds the pair that needs
+    // a round wait below it on the stack, the deepest on top.
+    const bool pend = valid && j > stop && prank - 1 < stop;
+    const uint64_t pm = wave_ballot(pend);
+    const int np = (int)__builtin_popcountll(pm);
+    if (L.sp + np + 1 > CAP) {
+      L.flags |= C2A_FLAG_STACK_OVERFLOW;
+      L.sp = 0;
+      ret = 2;
+      break;
+    }
+    if ((pend || j == stop) && lane < 64) {
+      Entry& o = g.stack[L.sp + (j == stop ? np : np - 1 - lanes_below(pm, j))];
+      if (leaf) {
+        for (int i = 0; i < 3; i++) { o.R[i] = s.p[i]; o.R[3 + i] = s.q[i]; }
+      } else {
+        for (int i = 0; i < 9; i++) o.R[i] = s.R[i];
+        for (int i = 0; i < 3; i++) o.T[i] = s.T[i];
+      }
+      Cur c;
+      c.d = d;
+      c.mt = mt;
+      c.b1 = leaf ? s.t1 : b1;
+      c.b2 = leaf ? s.t2 : b2;
+      c.sg = 0;
+      c.flags = leaf ? 3 | 16 | ((fl & 4) << 3) : fl & 3;
+      c.dTri = dTri;
+      c.mleaf = mleaf;
+      c.ar = -1;
+      c.cp = -1;
+      c.nn = nn;
+      c.lvl = x.lvl + lv;
+      *reinterpret_cast<Cur*>(&o.d) = c;
+    }
+    L.sp += np + 1;
+    ret = 1;
+    break;
+  }
+  L.nflush = L.nlog;
+  lane_sync();
+  return ret;
+}
+
+// The traversal below the pairs on the stack: a pair that has to be
+// expanded gets a round (a heap of pair values below it), and heap_scan
+// decides the heap.  Returns true when a round has been requested.
+template <int K, int CAP>
+C2A_HD bool walk_heaps(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+  const int cmode = uni(g.contact);
+  const bool counts = cmode != 0 && L.mode != MODE_DISTANCE;
+  int nhit = 0, next = 0;   // next: 1 a round for the top pair, 2 stack full
+  for (;;) {
+    if (nhit > 0) {   // contacts found last, in visiting order
+      const int at = L.num_contact + lane;
+      if (a.contacts && lane < nhit && at < a.contact_cap)
+        record_contact(g, a.contacts + L.qi * (int64_t)a.contact_cap + at, g.hit[lane][0],
+                       g.hit[lane][1]);
+      L.num_contact += nhit;
+      nhit = 0;
+      lane_sync();
+    }
+    if (next == 1) {
+      request_round(g, L, a, lane, nl);
+      return true;
+    }
+    if (next == 2 || L.sp == 0) return false;
+    const Entry& e = g.stack[L.sp - 1];
+    const Cur c = read_cur(e);
+    if (!(c.flags & 4) && !enters(L, cmode, c.d, c.mt)) {
+      if (cmode == 0 && c.mt < L.M) L.M = c.mt;
+      L.sp--;
+      continue;
+    }
+    const bool cached = (c.sg >> 8) == uni(g.gen) && (c.sg & 0xff) != 0;
+    const int base = (c.sg & 0xff) - 1;
+    const bool leaf = (c.flags & 3) == 3;
+    if (!cached && !(c.flags & 16)) {   // (the pair stays on the stack)
+      C2A_EMU_COUNT(leaf ? 0 : ((c.flags & 8) ? 1 : 3), L);
+      next = 1;
+      continue;
+    }
+    L.sp--;
+    if (leaf) {
+      // values from the entry (a heap's pending pair) or from its own round
+      const bool held = (c.flags & 16) != 0;
+      const Slot& sl = g.slot[held ? 0 : base];
+      const double dTri = held ? c.dTri : unid(sl.dTri);
+      const int t1 = held ? c.b1 : uni(sl.t1), t2 = held ? c.b2 : uni(sl.t2);
+      if (counts) {
+        const bool feat = held ? (c.flags & 32) != 0 : (uni(sl.flags) & 4) != 0;
+        if (feat && dTri <= L.thr) {
+          if (lane == 0) {
+            g.hit[0][0] = t1;
+            g.hit[0][1] = t2;
+          }
+          nhit = 1;
+          lane_sync();
+        }
+        continue;
+      }
+      if (leaf_update(L, cmode, a.strict, dTri, held ? c.mleaf : unid(sl.mleaf))) {
+        if (lane < 3) {
+          g.p1[lane] = held ? e.R[lane] : sl.p[lane];
+          g.p2[lane] = held ? e.R[3 + lane] : sl.q[lane];
+        }
+        lane_sync();
+        L.pq_pending = 0;
+        L.last1 = t1;
+        L.last2 = t2;
+      }
+      L.tri++;
+      continue;
+    }
+    next = heap_scan(g, L, a, c, base, lane, nhit);
+    if (next == 1) C2A_EMU_COUNT(2, L);
+  }
+}
+
+template <int K, int CAP>
+C2A_HD bool walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (K <= 5) return walk_heaps(g, L, a, lane, nl);
+  else return walk_pairs(g, L, a, lane, nl);
+#else
+  return (K <= 5 && nl >= 64 && !a.arena_rounds) ? walk_heaps(g, L, a, lane, nl)
+                                                 : walk_pairs(g, L, a, lane, nl);
+#endif
+}
+
 // After a step's walk: closest points of a replayed last improving leaf
 // (the same triangle-distance call a round would have made), and the log
 // hand-over to the next step.
@@ -1758,9 +2096,13 @@ C2A_HD void end_walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int n
     gdouble_ptr g2 = tris_of(M2) + 9 * (int64_t)L.last2;
     for (int i = 0; i < 9; i++) { ta[i] = g1[i]; tb[i] = g2[i]; Rrel[i] = g.Rrel[i]; }
     for (int i = 0; i < 3; i++) Trel[i] = g.Trel[i];
-    (void)tri_distance(Rrel, Trel, ta, tb, L.p1, L.p2, nullptr);
+    double p[3], q[3];
+    (void)tri_distance(Rrel, Trel, ta, tb, p, q, nullptr);
+    if (lane == 0)
+      for (int i = 0; i < 3; i++) { g.p1[i] = p[i]; g.p2[i] = q[i]; }
     L.pq_pending = 0;
   }
+  lane_sync();
   if (a.logcap > 0) {
     flush_log(g, L, arena_view(L.ab, a.logcap), lane, nl);
     L.nlog_prev = L.nlog;
@@ -1772,7 +2114,7 @@ template <int K, int CAP>
 C2A_HD void begin_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
   const MeshDev M1 = mesh_of(g, 0);
   const MeshDev M2 = mesh_of(g, 1);
-  if (L.mode != MODE_DISTANCE) {   // a distance query's traversal starts in fetch
+  if (L.mode == MODE_QUERY) {   // the other modes' traversals start in fetch
     double R1[9], T1[3], R2[9], T2[3];
     if (L.numCA == 0) {
       for (int i = 0; i < 9; i++) { R1[i] = g.mo[0].R0[i]; R2[i] = g.mo[1].R0[i]; }
@@ -1805,7 +2147,9 @@ C2A_HD void begin_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
   for (int i = 0; i < 3; i++) Trel[i] = g.Trel[i];
   L.D = tri_distance(Rrel, Trel, ta, tb, p, q, nullptr);
   if (L.mode == MODE_DISTANCE) {   // C2A_Distance's first bound (C2A_PQP.cpp:998-1005)
-    for (int i = 0; i < 3; i++) { L.p1[i] = p[i]; L.p2[i] = q[i]; }
+    if (lane == 0)
+      for (int i = 0; i < 3; i++) { g.p1[i] = p[i]; g.p2[i] = q[i]; }
+    lane_sync();
     L.state = ST_CONTACT_WALK;
     return;
   }
@@ -1835,7 +2179,7 @@ C2A_HD void finish_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, bool collis
     r->toc = L.toc;
     r->distance = L.D;
     r->mint = L.M;
-    for (int i = 0; i < 3; i++) { r->p1[i] = L.p1[i]; r->p2[i] = L.p2[i]; }
+    for (int i = 0; i < 3; i++) { r->p1[i] = g.p1[i]; r->p2[i] = g.p2[i]; }
     r->bv_tests = L.bv;
     r->tri_tests = L.tri;
     r->numCA = L.numCA;
@@ -1872,14 +2216,15 @@ C2A_HD void finish_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, bool collis
 // Saves the CA-loop state of a query about to start its next step and hands
 // the query to the tail pass (the next step starts there without a replay:
 // pair values do not depend on it).
-C2A_HD void hand_over(Leader& L, const KArgs& a, int lane) {
+template <int K, int CAP>
+C2A_HD void hand_over(const Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
   if (lane == 0) {
     TailRec& t = a.tail_rec[L.qi];
     t.lamda = L.lamda;
     t.lastLamda = L.lastLamda;
     t.Up = L.Up;
     t.M = L.M;
-    for (int i = 0; i < 3; i++) { t.p1[i] = L.p1[i]; t.p2[i] = L.p2[i]; }
+    for (int i = 0; i < 3; i++) { t.p1[i] = g.p1[i]; t.p2[i] = g.p2[i]; }
     t.bv = L.bv;
     t.tri = L.tri;
     t.nItrs = L.nItrs;
@@ -1907,7 +2252,7 @@ C2A_HD void after_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
       r->mint = L.M;
       r->abs_err = L.abs_err;
       r->rel_err = L.rel_err;
-      for (int i = 0; i < 3; i++) { r->p1[i] = L.p1[i]; r->p2[i] = L.p2[i]; }
+      for (int i = 0; i < 3; i++) { r->p1[i] = g.p1[i]; r->p2[i] = g.p2[i]; }
       r->bv_tests = L.bv;
       r->tri_tests = L.tri;
       r->last_tri[0] = L.last1;
@@ -1951,7 +2296,7 @@ C2A_HD void after_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
         L.numCA++;
         L.Up = 1.0 - L.lamda;
         L.state = ST_STEP;
-        if (a.tail_budget > 0 && !a.tail_pass && L.bv >= a.tail_budget) hand_over(L, a, lane);
+        if (a.tail_budget > 0 && !a.tail_pass && L.bv >= a.tail_budget) hand_over(g, L, a, lane);
         return;
       }
     }
@@ -1999,8 +2344,9 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
   L.bv = 0;
   L.tri = 0;
   L.num_contact = 0;
-  for (int i = 0; i < 3; i++) { L.p1[i] = 0.0; L.p2[i] = 0.0; }
   lane_sync();
+  if (lane == 0)
+    for (int i = 0; i < 3; i++) { g.p1[i] = 0.0; g.p2[i] = 0.0; }
   if (a.mode == MODE_STEP) {
     const StepDev& q = a.step_in[qi];
     if (lane == 0) {
@@ -2027,25 +2373,8 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
     for (int i = 0; i < 9; i++) { R1[i] = q.R1[i]; R2[i] = q.R2[i]; }
     for (int i = 0; i < 3; i++) { T1[i] = q.T1[i]; T2[i] = q.T2[i]; }
     start_traversal(g, L, M1, M2, R1, T1, R2, T2, -1, lane);
-    L.nlog = 0;
-    L.nflush = 0;
-    L.pq_pending = 0;
-    double p[3], qq[3], ta[9], tb[9], Rrel[9], Trel[3];
-    gdouble_ptr g1 = tris_of(M1) + 9 * (int64_t)L.seed1;
-    gdouble_ptr g2 = tris_of(M2) + 9 * (int64_t)L.seed2;
-    for (int i = 0; i < 9; i++) { ta[i] = g1[i]; tb[i] = g2[i]; Rrel[i] = g.Rrel[i]; }
-    for (int i = 0; i < 3; i++) Trel[i] = g.Trel[i];
-    L.D = tri_distance(Rrel, Trel, ta, tb, p, qq, nullptr);
-    if (L.numCA == 0) L.M = 1;
-    if (L.M <= 0.005 || L.D <= 0.5 || L.numCA > 5) {
-      L.abs_err = 0;
-      L.rel_err = 0;
-    } else {
-      L.abs_err = 1e+30;
-      L.rel_err = (L.numCA <= 2) ? 3 : 0.5;
-    }
-    L.M = 1;
-    L.state = ST_WALK;
+    L.nlog_prev = 0;
+    L.state = ST_STEP;
     return true;
   }
   if (a.mode == MODE_CONTACT || a.mode == MODE_DISTANCE) {
@@ -2163,7 +2492,10 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
     L.lastLamda = t.lastLamda;
     L.Up = t.Up;
     L.M = t.M;
-    for (int i = 0; i < 3; i++) { L.p1[i] = t.p1[i]; L.p2[i] = t.p2[i]; }
+    lane_sync();
+    if (lane == 0)
+      for (int i = 0; i < 3; i++) { g.p1[i] = t.p1[i]; g.p2[i] = t.p2[i]; }
+    lane_sync();
     L.bv = t.bv;
     L.tri = t.tri;
     L.nItrs = t.nItrs;
@@ -2205,48 +2537,51 @@ C2A_HD void translation_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, int la
   for (int i = 0; i < 9; i++) { Rrel[i] = g.Rrel[i]; r1[i] = R1[i]; }
   for (int i = 0; i < 3; i++) Trel[i] = g.Trel[i];
   int la = L.seed1, lb = L.seed2;
-  {
-    double A[9], tb[9], B[9];
-    load_tri(A, M1, la);
-    load_tri(tb, M2, lb);
-    for (int v = 0; v < 3; v++) mxvpv(B + 3 * v, Rrel, tb + 3 * v, Trel);
-    double mint = 1.0, dTri = 0.0;
-    if (ca_on_tris(g.mo[0], r1, A, B, delta, mint, dTri)) {
-      L.M = mint;
-      L.D = dTri;
-    } else {
-      L.M = 1.0;
-      L.D = 1e+30;
-    }
-  }
   L.abs_err = 0;
   L.rel_err = 0;
-  while (L.sp > 0) {
-    L.sp--;
-    const Entry& e = g.stack[L.sp];
+  bool seed = true;   // the first bound: the seed pair (C2A.cpp:1818-1852)
+  while (seed || L.sp > 0) {
     double R[9], T[3];
-    for (int i = 0; i < 9; i++) R[i] = unid(e.R[i]);
-    for (int i = 0; i < 3; i++) T[i] = unid(e.T[i]);
-    const int b1 = uni(e.b1), b2 = uni(e.b2), flags = uni(e.flags);
-    const double dv = unid(e.d), mv = unid(e.mt);
-    lane_sync();
-    if (!(flags & 4)) {   // the parent's deferred test (C2A.cpp:1477-1513)
-      if (!(mv < L.M && ((dv < (L.D - L.abs_err)) || (dv * (1 + L.rel_err) < L.D)))) continue;
+    int b1 = 0, b2 = 0, t1 = la, t2 = lb;
+    bool tris = seed;
+    if (!seed) {
+      L.sp--;
+      const Entry& e = g.stack[L.sp];
+      for (int i = 0; i < 9; i++) R[i] = unid(e.R[i]);
+      for (int i = 0; i < 3; i++) T[i] = unid(e.T[i]);
+      b1 = uni(e.b1);
+      b2 = uni(e.b2);
+      const int flags = uni(e.flags);
+      const double dv = unid(e.d), mv = unid(e.mt);
+      lane_sync();
+      if (!(flags & 4)) {   // the parent's deferred test (C2A.cpp:1477-1513)
+        if (!(mv < L.M && ((dv < (L.D - L.abs_err)) || (dv * (1 + L.rel_err) < L.D)))) continue;
+      }
+      node_ptr B1 = N1 + b1;
+      node_ptr B2 = N2 + b2;
+      if (node_leaf(B1) && node_leaf(B2)) {   // C2A.cpp:1395-1425
+        t1 = -B1->first_child - 1;
+        t2 = -B2->first_child - 1;
+        tris = true;
+      }
     }
-    node_ptr B1 = N1 + b1;
-    node_ptr B2 = N2 + b2;
-    const bool l1 = node_leaf(B1), l2 = node_leaf(B2);
-    if (l1 && l2) {   // C2A.cpp:1395-1425
-      const int t1 = -B1->first_child - 1, t2 = -B2->first_child - 1;
+    if (tris) {
       double A[9], tb[9], B[9];
       load_tri(A, M1, t1);
       load_tri(tb, M2, t2);
       for (int v = 0; v < 3; v++) mxvpv(B + 3 * v, Rrel, tb + 3 * v, Trel);
-      if (ca_on_tris(g.mo[0], r1, A, B, delta, L.M, L.D)) {
+      double mint = seed ? 1.0 : L.M, dTri = seed ? 0.0 : L.D;
+      if (ca_on_tris(g.mo[0], r1, A, B, delta, mint, dTri)) {
+        L.M = mint;
+        L.D = dTri;
         la = t1;
         lb = t2;
+      } else if (seed) {
+        L.M = 1.0;
+        L.D = 1e+30;
       }
-      L.tri++;
+      if (!seed) L.tri++;
+      seed = false;
       continue;
     }
     if (L.sp + 2 > CAP) {
@@ -2261,8 +2596,20 @@ C2A_HD void translation_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, int la
     descend(N1, N2, a1, a2, 0, RA, TA);
     descend(N1, N2, c1, c2, 1, RC, TC);
     double dA = 1e+30, dC = 1e+30, mA = L.M, mC = L.M;
-    ca_on_rss(g.mo[0], r1, RA, TA, N1 + a1, N2 + a2, delta, mA, dA);
-    ca_on_rss(g.mo[0], r1, RC, TC, N1 + c1, N2 + c2, delta, mC, dC);
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < 2; k++) {
+      double Rk[9], Tk[3], dk = 1e+30, mk = L.M;
+      for (int i = 0; i < 9; i++) Rk[i] = k ? RC[i] : RA[i];
+      for (int i = 0; i < 3; i++) Tk[i] = k ? TC[i] : TA[i];
+      ca_on_rss(g.mo[0], r1, Rk, Tk, N1 + (k ? c1 : a1), N2 + (k ? c2 : a2), delta, mk, dk);
+      if (k) {
+        mC = mk;
+        dC = dk;
+      } else {
+        mA = mk;
+        dA = dk;
+      }
+    }
     L.bv += 2;
     // closer child first (C2A.cpp:1478); both tests wait for their turn
     const bool c_first = dC < dA;
@@ -2298,9 +2645,12 @@ C2A_HD void translation_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, int la
     double ta[9], tb[9];
     load_tri(ta, M1, la);
     load_tri(tb, M2, lb);
-    L.D = tri_distance(Rrel, Trel, ta, tb, L.p1, L.p2, nullptr);
+    double p[3], q[3];
+    L.D = tri_distance(Rrel, Trel, ta, tb, p, q, nullptr);
+    lane_sync();
+    if (lane == 0)
+      for (int i = 0; i < 3; i++) { g.p1[i] = p[i]; g.p2[i] = q[i]; }
   }
-  lane_sync();
   if (lane == 0) {   // res->R, res->T at the advanced pose (C2A.cpp:1902-1904)
     for (int i = 0; i < 9; i++) g.Rrel[i] = Rrel[i];
     for (int i = 0; i < 3; i++) g.Trel[i] = Trel[i];
@@ -2380,10 +2730,11 @@ C2A_HD void leader_run(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
             double u[3], Rr[9], Tr[3], q2[3];
             for (int i = 0; i < 9; i++) Rr[i] = g.Rrel[i];
             for (int i = 0; i < 3; i++) Tr[i] = g.Trel[i];
-            sub3(u, L.p2, Tr);
+            const double p2[3] = {g.p2[0], g.p2[1], g.p2[2]};
+            sub3(u, p2, Tr);
             mtxv(q2, Rr, u);
             r->distance = L.D;
-            for (int i = 0; i < 3; i++) { r->p1[i] = L.p1[i]; r->p2[i] = q2[i]; }
+            for (int i = 0; i < 3; i++) { r->p1[i] = g.p1[i]; r->p2[i] = q2[i]; }
             r->bv_tests = L.bv;
             r->tri_tests = L.tri;
             r->last_tri[0] = L.last1;

@@ -54,8 +54,7 @@ __global__ void __launch_bounds__(64 * NW) ccd_kernel(KArgs a) {
       }
     }
     round_lane(g, L, lane, 64 * NW, a);
-    if (g.rarena) mem_sync();   // the walk reads the new records through the LDS window
-    else lane_sync();
+    lane_sync();
   }
 }
 
