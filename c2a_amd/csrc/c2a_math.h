@@ -308,31 +308,17 @@ C2A_HD void seg_params(double& t, double& u, double a, double b, double AB, doub
     clampd(t, 0, a);
   }
 }
-// InsideVoronoi (C2A_RectDist.h:123-154)
+// InsideVoronoi (C2A_RectDist.h:123-154), without branches.  The clamps by
+// min / max and the two ordered compares decide as the reference's nested
+// ifs do, a NaN included (every comparison with it is false).
 C2A_HD bool voronoi(double a, double b, double AnB, double AnT, double AB, double AT, double BT) {
-  if (fabs(AnB) < 1e-7) return false;
-  double u = -AnT / AnB;
-  clampd(u, 0, b);
-  double t = u * AB + AT;
-  clampd(t, 0, a);
-  double v = t * AB - BT;
-  if (AnB > 0) {
-    if (v > (u + 1e-7)) return true;
-  } else {
-    if (v < (u - 1e-7)) return true;
-  }
-  return false;
-}
-// edge-pair case epilogue: P on A's edge, Q = Tab + col_f*lf + col_v*u
-C2A_HD double rect_edge_tail(double P0, double P1, const double* Rab, const double* Tab, int cf,
-                             double lf, bool has_f, int cv, double u, double* S) {
-  double Q[3];
-  for (int i = 0; i < 3; i++) {
-    if (has_f) Q[i] = Tab[i] + Rab[3 * i + cf] * lf + Rab[3 * i + cv] * u;
-    else Q[i] = Tab[i] + Rab[3 * i + cv] * u;
-  }
-  S[0] = Q[0] - P0; S[1] = Q[1] - P1; S[2] = Q[2] - 0;
-  return sqrt(dot3(S, S));
+  const double u0 = -AnT / AnB;
+  const double u = __builtin_fmin(__builtin_fmax(u0, 0.0), b);
+  const double t0 = u * AB + AT;
+  const double t = __builtin_fmin(__builtin_fmax(t0, 0.0), a);
+  const double v = t * AB - BT;
+  const bool in = AnB > 0 ? v > (u + 1e-7) : v < (u - 1e-7);
+  return in & !(fabs(AnB) < 1e-7) & (u0 == u0) & (t0 == t0);
 }
 
 // True when any active lane of the wavefront holds p (host: the lane itself).
@@ -344,20 +330,98 @@ C2A_HD bool wave_any(bool p) {
 #endif
 }
 
-// Ordered (lo, hi) of two values the way the reference builds its edge
-// extents: hi/lo of (x, y) plus the matching pair (z, w).
-C2A_HD void order2(double x, double y, double z, double w, double& lo, double& hi, double& zlo,
-                   double& zhi) {
-  if (x < y) { lo = x; hi = y; zlo = z; zhi = w; }
-  else { lo = y; hi = x; zlo = w; zhi = z; }
+// One class of the rectangle distance's edge pairs: A's two edges along one
+// of its axes against B's two edges along one of its own.  f marks the fixed
+// axis of an edge, t the one it runs along.
+struct EdgeClass {
+  double at, af, bt, bf;       // sides
+  double ABtt, ABtf, ABft;     // direction cosines [A axis][B axis]
+  double aABff, aABft, bABff, bABtf;   // ... times af (aAB) or bf (bAB)
+  double Tat, Taf, Tbt, Tbf;   // Tab on A's axes, Tba on B's
+};
+// Which of two corner coordinates' tests holds for the reference's lo / hi
+// pair: first when x < y, else the second.
+C2A_HD bool sel(bool first, bool x, bool y) {
+  return (first & x) | (!first & y);
 }
 
-// The 16 edge-pair cases are tested in the reference's order; the first one
+// Corner coordinates of a rectangle against the other one's slab [0, m]:
+// below 0, above m.
+struct Side {
+  bool lo, hi;
+};
+C2A_HD Side side(double x, double m) {
+  Side r;
+  r.lo = x < 0;
+  r.hi = x > m;
+  return r;
+}
+
+// The winning edge pair of a lane.
+struct EdgeWin {
+  int w;           // 4 * class + case, -1 none
+  double AT, BT;   // segment parameters
+};
+
+// The four cases of a class in the reference's order: both edges at their
+// far side, A's far and B's near, A's near and B's far, both near.  Each lane
+// takes its own next case that passes the extent pre-test, so a wavefront
+// makes as many turns as its busiest lane has such cases (one or two, mostly)
+// instead of one per case, and the two Voronoi tests of a turn run side by
+// side.  x1, y1 / z1, w1: A's corners at B's near / far edge order (the
+// reference's lo / hi and ulo / uhi), o1 whether x1 < y1; x2 .. o2 the same for B's
+// corners.  first: class 0, whose far-far sums the reference associates
+// differently.
+C2A_HD void edge_class(EdgeWin& g, int cls, const EdgeClass& e, bool o1, Side x1, Side y1, Side z1,
+                       Side w1, bool o2, Side x2, Side y2, Side z2, Side w2) {
+  bool c0 = sel(o1, w1.hi, z1.hi) & sel(o2, w2.hi, z2.hi);   // uhi1 > bf, uhi2 > af
+  bool c1 = sel(o1, z1.lo, w1.lo) & sel(o2, y2.hi, x2.hi);   // ulo1 < 0, hi2 > af
+  bool c2 = sel(o1, y1.hi, x1.hi) & sel(o2, z2.lo, w2.lo);   // hi1 > bf, ulo2 < 0
+  bool c3 = sel(o1, x1.lo, y1.lo) & sel(o2, x2.lo, y2.lo);   // lo1 < 0, lo2 < 0
+  bool open = g.w < 0;
+  c0 = c0 & open;
+  c1 = c1 & open;
+  c2 = c2 & open;
+  c3 = c3 & open;
+  if (!wave_any(c0 | c1 | c2 | c3)) return;
+  const double q1 = e.aABft - e.Tbt, w1v = -e.Tat - e.bABtf;
+  const double n1hh = cls == 0 ? e.aABff - e.bf - e.Tbf : e.aABff - e.Tbf - e.bf;
+  const double n1hl = e.Tbf - e.aABff, n1lh = -e.Tbf - e.bf;
+  const double n2hh = cls == 0 ? e.Taf + e.bABff - e.af : e.Taf - e.af + e.bABff;
+  const double n2hl = e.Taf - e.af, n2lh = -e.Taf - e.bABff;
+  do {
+    const bool p0 = c0, p1 = c1 & !c0, p2 = c2 & !c0 & !c1, p3 = c3 & !c0 & !c1 & !c2;
+    const bool ah = p0 | p1, bh = p0 | p2;
+    // the far / near shortcuts past a Voronoi test
+    const bool s1 = (p0 & sel(o1, z1.hi, w1.hi)) | (p1 & sel(o1, w1.lo, z1.lo)) |
+                    (p2 & sel(o1, x1.hi, y1.hi)) | (p3 & sel(o1, y1.lo, x1.lo));
+    const bool s2 = (p0 & sel(o2, z2.hi, w2.hi)) | (p1 & sel(o2, x2.hi, y2.hi)) |
+                    (p2 & sel(o2, w2.lo, z2.lo)) | (p3 & sel(o2, y2.lo, x2.lo));
+    const double AT = ah ? q1 : -e.Tbt, BT = bh ? w1v : -e.Tat;
+    const double n1 = ah ? (bh ? n1hh : n1hl) : (bh ? n1lh : e.Tbf);
+    const double n2 = ah ? (bh ? n2hh : n2hl) : (bh ? n2lh : -e.Taf);
+    const bool v1 = voronoi(e.bt, e.at, bh ? e.ABtf : -e.ABtf, n1, e.ABtt, AT, BT);
+    const bool v2 = voronoi(e.at, e.bt, ah ? e.ABft : -e.ABft, n2, e.ABtt, -BT, -AT);
+    const bool ok = (p0 | p1 | p2 | p3) & (s1 | v1) & (s2 | v2);
+    if (ok) {
+      g.w = 4 * cls + (ah ? 0 : 2) + (bh ? 0 : 1);
+      g.AT = -BT;
+      g.BT = -AT;
+    }
+    c0 = false;
+    c1 = c1 & !p1 & !ok;
+    c2 = c2 & !p2 & !ok;
+    c3 = c3 & !p3 & !ok;
+  } while (wave_any(c1 | c2 | c3));
+}
+
+// The 16 edge-pair cases are decided in the reference's order; the first one
 // whose extent pre-test and two Voronoi tests hold gives the closest points.
-// The loop over cases is uniform across the wavefront (each case's
-// parameters are formed by a wave-uniform switch) and stops once every lane
-// has its case, so lanes working on different pairs do not serialize the
-// sixteen case bodies.  Each case's expressions are the reference's.
+// All pre-tests come from 40 comparisons of corner coordinates, kept as lane
+// masks.  What bounds it is the instruction stream of the one wavefront per
+// SIMD (FP64 divisions above all): 64 random pairs of a knot pair take 6,400
+// cycles on MI355X; trying the 16 cases one after another for the whole
+// wavefront took 15,300.
 C2A_HD double rect_dist(const double* Rab, const double* Tab, const double* a, const double* b,
                         double* S) {
   const double AB00 = Rab[0], AB01 = Rab[1], AB10 = Rab[3], AB11 = Rab[4];
@@ -385,169 +449,49 @@ C2A_HD double rect_dist(const double* Rab, const double* Tab, const double* a, c
   const double BULy = BLLy + bAB10;
   const double BUUy = BLUy + bAB10;
 
-  int win = -1;
-  double g_a = 0, g_b = 0, g_AB = 0, g_AT = 0, g_BT = 0;   // segment parameters
-  double g_p = 0;                                          // fixed coordinate of P
-  int g_tx = 0;                                            // 1: P = (t, p), 0: P = (p, t)
-  int g_cf = 0, g_cv = 0;
-  double g_lf = 0;
-  bool g_hf = false;
-  for (int c = 0; c < 16; c++) {
-    if (!wave_any(win < 0)) break;
-    double lo1, hi1, lo2, hi2, ulo1, uhi1, ulo2, uhi2;
-    bool pre = false, s1 = false, s2 = false;
-    double v1[7], v2[7], sg[5];
-    double pfix = 0;
-    int tx = 0, cf = 0, cv = 0;
-    double lf = 0;
-    bool hf = false;
-    if (c < 4) {
-      order2(ALLx, ALUx, AULx, AUUx, lo1, hi1, ulo1, uhi1);   // LA1 x-extent, UA1 x-extent
-      order2(BLLx, BLUx, BULx, BUUx, lo2, hi2, ulo2, uhi2);   // LB1, UB1
-    } else if (c < 8) {
-      order2(ALLy, ALUy, AULy, AUUy, lo1, hi1, ulo1, uhi1);   // LA1 y, UA1 y
-      order2(BLLx, BULx, BLUx, BUUx, lo2, hi2, ulo2, uhi2);   // LB0 x, UB0 x
-    } else if (c < 12) {
-      order2(ALLx, AULx, ALUx, AUUx, lo1, hi1, ulo1, uhi1);   // LA0 x, UA0 x
-      order2(BLLy, BLUy, BULy, BUUy, lo2, hi2, ulo2, uhi2);   // LB1 y, UB1 y
-    } else {
-      order2(ALLy, AULy, ALUy, AUUy, lo1, hi1, ulo1, uhi1);   // LA0 y, UA0 y
-      order2(BLLy, BULy, BLUy, BUUy, lo2, hi2, ulo2, uhi2);   // LB0 y, UB0 y
-    }
-#define C2A_V(o, A0, A1, A2, A3, A4, A5, A6) \
-  o[0] = (A0); o[1] = (A1); o[2] = (A2); o[3] = (A3); o[4] = (A4); o[5] = (A5); o[6] = (A6)
-#define C2A_G(A0, A1, A2, A3, A4) sg[0] = (A0); sg[1] = (A1); sg[2] = (A2); sg[3] = (A3); sg[4] = (A4)
-    switch (c) {
-      case 0:   // A x=a0 edge, B b0 edge (both along the 1-axes)
-        pre = (uhi1 > b[0]) && (uhi2 > a[0]); s1 = (ulo1 > b[0]); s2 = (ulo2 > a[0]);
-        C2A_V(v1, b[1], a[1], AB10, aAB00 - b[0] - Tba[0], AB11, aAB01 - Tba[1], -Tab[1] - bAB10);
-        C2A_V(v2, a[1], b[1], AB01, Tab[0] + bAB00 - a[0], AB11, Tab[1] + bAB10, Tba[1] - aAB01);
-        C2A_G(a[1], b[1], AB11, Tab[1] + bAB10, Tba[1] - aAB01);
-        pfix = a[0]; tx = 0; cf = 0; lf = b[0]; hf = true; cv = 1;
-        break;
-      case 1:
-        pre = (ulo1 < 0) && (hi2 > a[0]); s1 = (uhi1 < 0); s2 = (lo2 > a[0]);
-        C2A_V(v1, b[1], a[1], -AB10, Tba[0] - aAB00, AB11, aAB01 - Tba[1], -Tab[1]);
-        C2A_V(v2, a[1], b[1], AB01, Tab[0] - a[0], AB11, Tab[1], Tba[1] - aAB01);
-        C2A_G(a[1], b[1], AB11, Tab[1], Tba[1] - aAB01);
-        pfix = a[0]; tx = 0; cv = 1;
-        break;
-      case 2:
-        pre = (hi1 > b[0]) && (ulo2 < 0); s1 = (lo1 > b[0]); s2 = (uhi2 < 0);
-        C2A_V(v1, b[1], a[1], AB10, -Tba[0] - b[0], AB11, -Tba[1], -Tab[1] - bAB10);
-        C2A_V(v2, a[1], b[1], -AB01, -Tab[0] - bAB00, AB11, Tab[1] + bAB10, Tba[1]);
-        C2A_G(a[1], b[1], AB11, Tab[1] + bAB10, Tba[1]);
-        pfix = 0; tx = 0; cf = 0; lf = b[0]; hf = true; cv = 1;
-        break;
-      case 3:
-        pre = (lo1 < 0) && (lo2 < 0); s1 = (hi1 < 0); s2 = (hi2 < 0);
-        C2A_V(v1, b[1], a[1], -AB10, Tba[0], AB11, -Tba[1], -Tab[1]);
-        C2A_V(v2, a[1], b[1], -AB01, -Tab[0], AB11, Tab[1], Tba[1]);
-        C2A_G(a[1], b[1], AB11, Tab[1], Tba[1]);
-        pfix = 0; tx = 0; cv = 1;
-        break;
-      case 4:   // A 1-axis edges against B 0-axis edges
-        pre = (uhi1 > b[1]) && (uhi2 > a[0]); s1 = (ulo1 > b[1]); s2 = (ulo2 > a[0]);
-        C2A_V(v1, b[0], a[1], AB11, aAB01 - Tba[1] - b[1], AB10, aAB00 - Tba[0], -Tab[1] - bAB11);
-        C2A_V(v2, a[1], b[0], AB00, Tab[0] - a[0] + bAB01, AB10, Tab[1] + bAB11, Tba[0] - aAB00);
-        C2A_G(a[1], b[0], AB10, Tab[1] + bAB11, Tba[0] - aAB00);
-        pfix = a[0]; tx = 0; cf = 1; lf = b[1]; hf = true; cv = 0;
-        break;
-      case 5:
-        pre = (ulo1 < 0) && (hi2 > a[0]); s1 = (uhi1 < 0); s2 = (lo2 > a[0]);
-        C2A_V(v1, b[0], a[1], -AB11, Tba[1] - aAB01, AB10, aAB00 - Tba[0], -Tab[1]);
-        C2A_V(v2, a[1], b[0], AB00, Tab[0] - a[0], AB10, Tab[1], Tba[0] - aAB00);
-        C2A_G(a[1], b[0], AB10, Tab[1], Tba[0] - aAB00);
-        pfix = a[0]; tx = 0; cv = 0;
-        break;
-      case 6:
-        pre = (hi1 > b[1]) && (ulo2 < 0); s1 = (lo1 > b[1]); s2 = (uhi2 < 0);
-        C2A_V(v1, b[0], a[1], AB11, -Tba[1] - b[1], AB10, -Tba[0], -Tab[1] - bAB11);
-        C2A_V(v2, a[1], b[0], -AB00, -Tab[0] - bAB01, AB10, Tab[1] + bAB11, Tba[0]);
-        C2A_G(a[1], b[0], AB10, Tab[1] + bAB11, Tba[0]);
-        pfix = 0; tx = 0; cf = 1; lf = b[1]; hf = true; cv = 0;
-        break;
-      case 7:
-        pre = (lo1 < 0) && (lo2 < 0); s1 = (hi1 < 0); s2 = (hi2 < 0);
-        C2A_V(v1, b[0], a[1], -AB11, Tba[1], AB10, -Tba[0], -Tab[1]);
-        C2A_V(v2, a[1], b[0], -AB00, -Tab[0], AB10, Tab[1], Tba[0]);
-        C2A_G(a[1], b[0], AB10, Tab[1], Tba[0]);
-        pfix = 0; tx = 0; cv = 0;
-        break;
-      case 8:   // A 0-axis edges against B 1-axis edges
-        pre = (uhi1 > b[0]) && (uhi2 > a[1]); s1 = (ulo1 > b[0]); s2 = (ulo2 > a[1]);
-        C2A_V(v1, b[1], a[0], AB00, aAB10 - Tba[0] - b[0], AB01, aAB11 - Tba[1], -Tab[0] - bAB00);
-        C2A_V(v2, a[0], b[1], AB11, Tab[1] - a[1] + bAB10, AB01, Tab[0] + bAB00, Tba[1] - aAB11);
-        C2A_G(a[0], b[1], AB01, Tab[0] + bAB00, Tba[1] - aAB11);
-        pfix = a[1]; tx = 1; cf = 0; lf = b[0]; hf = true; cv = 1;
-        break;
-      case 9:
-        pre = (ulo1 < 0) && (hi2 > a[1]); s1 = (uhi1 < 0); s2 = (lo2 > a[1]);
-        C2A_V(v1, b[1], a[0], -AB00, Tba[0] - aAB10, AB01, aAB11 - Tba[1], -Tab[0]);
-        C2A_V(v2, a[0], b[1], AB11, Tab[1] - a[1], AB01, Tab[0], Tba[1] - aAB11);
-        C2A_G(a[0], b[1], AB01, Tab[0], Tba[1] - aAB11);
-        pfix = a[1]; tx = 1; cv = 1;
-        break;
-      case 10:
-        pre = (hi1 > b[0]) && (ulo2 < 0); s1 = (lo1 > b[0]); s2 = (uhi2 < 0);
-        C2A_V(v1, b[1], a[0], AB00, -b[0] - Tba[0], AB01, -Tba[1], -bAB00 - Tab[0]);
-        C2A_V(v2, a[0], b[1], -AB11, -Tab[1] - bAB10, AB01, Tab[0] + bAB00, Tba[1]);
-        C2A_G(a[0], b[1], AB01, Tab[0] + bAB00, Tba[1]);
-        pfix = 0; tx = 1; cf = 0; lf = b[0]; hf = true; cv = 1;
-        break;
-      case 11:
-        pre = (lo1 < 0) && (lo2 < 0); s1 = (hi1 < 0); s2 = (hi2 < 0);
-        C2A_V(v1, b[1], a[0], -AB00, Tba[0], AB01, -Tba[1], -Tab[0]);
-        C2A_V(v2, a[0], b[1], -AB11, -Tab[1], AB01, Tab[0], Tba[1]);
-        C2A_G(a[0], b[1], AB01, Tab[0], Tba[1]);
-        pfix = 0; tx = 1; cv = 1;
-        break;
-      case 12:  // A 0-axis edges against B 0-axis edges
-        pre = (uhi1 > b[1]) && (uhi2 > a[1]); s1 = (ulo1 > b[1]); s2 = (ulo2 > a[1]);
-        C2A_V(v1, b[0], a[0], AB01, aAB11 - Tba[1] - b[1], AB00, aAB10 - Tba[0], -Tab[0] - bAB01);
-        C2A_V(v2, a[0], b[0], AB10, Tab[1] - a[1] + bAB11, AB00, Tab[0] + bAB01, Tba[0] - aAB10);
-        C2A_G(a[0], b[0], AB00, Tab[0] + bAB01, Tba[0] - aAB10);
-        pfix = a[1]; tx = 1; cf = 1; lf = b[1]; hf = true; cv = 0;
-        break;
-      case 13:
-        pre = (ulo1 < 0) && (hi2 > a[1]); s1 = (uhi1 < 0); s2 = (lo2 > a[1]);
-        C2A_V(v1, b[0], a[0], -AB01, Tba[1] - aAB11, AB00, aAB10 - Tba[0], -Tab[0]);
-        C2A_V(v2, a[0], b[0], AB10, Tab[1] - a[1], AB00, Tab[0], Tba[0] - aAB10);
-        C2A_G(a[0], b[0], AB00, Tab[0], Tba[0] - aAB10);
-        pfix = a[1]; tx = 1; cv = 0;
-        break;
-      case 14:
-        pre = (hi1 > b[1]) && (ulo2 < 0); s1 = (lo1 > b[1]); s2 = (uhi2 < 0);
-        C2A_V(v1, b[0], a[0], AB01, -Tba[1] - b[1], AB00, -Tba[0], -Tab[0] - bAB01);
-        C2A_V(v2, a[0], b[0], -AB10, -Tab[1] - bAB11, AB00, Tab[0] + bAB01, Tba[0]);
-        C2A_G(a[0], b[0], AB00, Tab[0] + bAB01, Tba[0]);
-        pfix = 0; tx = 1; cf = 1; lf = b[1]; hf = true; cv = 0;
-        break;
-      default:
-        pre = (lo1 < 0) && (lo2 < 0); s1 = (hi1 < 0); s2 = (hi2 < 0);
-        C2A_V(v1, b[0], a[0], -AB01, Tba[1], AB00, -Tba[0], -Tab[0]);
-        C2A_V(v2, a[0], b[0], -AB10, -Tab[1], AB00, Tab[0], Tba[0]);
-        C2A_G(a[0], b[0], AB00, Tab[0], Tba[0]);
-        pfix = 0; tx = 1; cv = 0;
-        break;
-    }
-#undef C2A_V
-#undef C2A_G
-    if (win < 0 && pre) {
-      bool ok = s1 || voronoi(v1[0], v1[1], v1[2], v1[3], v1[4], v1[5], v1[6]);
-      ok = ok && (s2 || voronoi(v2[0], v2[1], v2[2], v2[3], v2[4], v2[5], v2[6]));
-      if (ok) {
-        win = c;
-        g_a = sg[0]; g_b = sg[1]; g_AB = sg[2]; g_AT = sg[3]; g_BT = sg[4];
-        g_p = pfix; g_tx = tx; g_cf = cf; g_cv = cv; g_lf = lf; g_hf = hf;
-      }
-    }
+  EdgeWin g;
+  g.w = -1;
+  g.AT = g.BT = 0.0;
+  {
+    const Side all = side(ALLx, b[0]), alu = side(ALUx, b[0]), aul = side(AULx, b[0]),
+               auu = side(AUUx, b[0]);
+    const Side ally = side(ALLy, b[1]), aluy = side(ALUy, b[1]), auly = side(AULy, b[1]),
+               auuy = side(AUUy, b[1]);
+    const Side bll = side(BLLx, a[0]), blu = side(BLUx, a[0]), bul = side(BULx, a[0]),
+               buu = side(BUUx, a[0]);
+    const Side blly = side(BLLy, a[1]), bluy = side(BLUy, a[1]), buly = side(BULy, a[1]),
+               buuy = side(BUUy, a[1]);
+    // A's 1-axis edges against B's 1-axis, then 0-axis edges; A's 0-axis edges likewise
+    const EdgeClass e0 = {a[1], a[0], b[1], b[0], AB11, AB10, AB01, aAB00, aAB01,
+                          bAB00, bAB10, Tab[1], Tab[0], Tba[1], Tba[0]};
+    edge_class(g, 0, e0, ALLx < ALUx, all, alu, aul, auu, BLLx < BLUx, bll, blu, bul, buu);
+    const EdgeClass e1 = {a[1], a[0], b[0], b[1], AB10, AB11, AB00, aAB01, aAB00,
+                          bAB01, bAB11, Tab[1], Tab[0], Tba[0], Tba[1]};
+    edge_class(g, 1, e1, ALLy < ALUy, ally, aluy, auly, auuy, BLLx < BULx, bll, bul, blu, buu);
+    const EdgeClass e2 = {a[0], a[1], b[1], b[0], AB01, AB00, AB11, aAB10, aAB11,
+                          bAB10, bAB00, Tab[0], Tab[1], Tba[1], Tba[0]};
+    edge_class(g, 2, e2, ALLx < AULx, all, aul, alu, auu, BLLy < BLUy, blly, bluy, buly, buuy);
+    const EdgeClass e3 = {a[0], a[1], b[0], b[1], AB00, AB01, AB10, aAB11, aAB10,
+                          bAB11, bAB01, Tab[0], Tab[1], Tba[0], Tba[1]};
+    edge_class(g, 3, e3, ALLy < AULy, ally, auly, aluy, auuy, BLLy < BULy, blly, buly, bluy, buuy);
   }
-  if (win >= 0) {
+  if (g.w >= 0) {
+    // P on A's edge, Q = Tab + (B's fixed side) + (B's edge) * u
+    const bool a1 = g.w < 8, b1 = (g.w & 4) == 0;   // the edges run along the 1-axes
+    const bool ah = (g.w & 2) == 0, bh = (g.w & 1) == 0;
     double t, u;
-    seg_params(t, u, g_a, g_b, g_AB, g_AT, g_BT);
-    return g_tx ? rect_edge_tail(t, g_p, Rab, Tab, g_cf, g_lf, g_hf, g_cv, u, S)
-                : rect_edge_tail(g_p, t, Rab, Tab, g_cf, g_lf, g_hf, g_cv, u, S);
+    seg_params(t, u, a1 ? a[1] : a[0], b1 ? b[1] : b[0],
+               a1 ? (b1 ? AB11 : AB10) : (b1 ? AB01 : AB00), g.AT, g.BT);
+    const double lf = b1 ? b[0] : b[1], p = ah ? (a1 ? a[0] : a[1]) : 0.0;
+    double Q[3];
+    for (int i = 0; i < 3; i++) {
+      const double cv = b1 ? Rab[3 * i + 1] : Rab[3 * i], cf = b1 ? Rab[3 * i] : Rab[3 * i + 1];
+      Q[i] = (bh ? Tab[i] + cf * lf : Tab[i]) + cv * u;
+    }
+    S[0] = Q[0] - (a1 ? p : t);
+    S[1] = Q[1] - (a1 ? t : p);
+    S[2] = Q[2] - 0;
+    return sqrt(dot3(S, S));
   }
 
   // face-normal separation (C2A_RectDist.h:855-933)
