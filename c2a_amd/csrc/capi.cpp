@@ -1288,10 +1288,9 @@ namespace {
 
 static_assert(sizeof(StaticOut) == sizeof(c2a_static_result), "static result layout");
 
-// The static queries of static_query.h: one thread per query over a
-// workspace of per-thread stacks / queues sized for the deepest pair of
-// hierarchies, with fewer threads when that would not fit in a quarter of
-// the free device memory.
+// The static queries of static_query.h and static_wave.h over a workspace of
+// stacks / queues sized for the deepest pair of hierarchies, with fewer
+// workgroups when that would not fit in a quarter of the free device memory.
 int static_queries(c2a_mesh* const* meshes, int32_t nmesh, int32_t kind, const double* poses,
                    const int32_t* mesh_pairs, const int32_t* seed_tris, const double* params,
                    double rel_err, double abs_err, int32_t qsize, int32_t flag, int64_t nq,
@@ -1331,22 +1330,26 @@ int static_queries(c2a_mesh* const* meshes, int32_t nmesh, int32_t kind, const d
     unpack_pose(poses + 24 * i + 12, q.R2, q.T2);
     q.param = params ? params[i] : 0.0;
   }
+  // one wavefront per query where the search allows it, else one thread
+  const bool wave = static_wave_ok(kind, qsize, pair_cap, depth_sum);
   const int64_t per_thread = sq_ws_entries(kind, qsize, depth_sum);
-  const size_t thread_bytes = (size_t)per_thread * sizeof(SqEntry);
+  // workspace of one workgroup: its wavefront's, or its threads'
+  const size_t group_bytes = wave ? (size_t)static_wave_bytes(kind, pair_cap, depth_sum)
+                                  : (size_t)kStaticBlock * per_thread * sizeof(SqEntry);
   size_t free_b = 0, total_b = 0;
   size_t budget = (size_t)1 << 30;
   if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b > 0) budget = free_b / 4;
-  int64_t blocks = (nq + kStaticBlock - 1) / kStaticBlock;
-  blocks = std::min<int64_t>(blocks, 4096);
-  while (blocks > 1 && (size_t)blocks * kStaticBlock * thread_bytes > budget) blocks /= 2;
-  if ((size_t)blocks * kStaticBlock * thread_bytes > budget)
+  int64_t blocks = wave ? nq : (nq + kStaticBlock - 1) / kStaticBlock;
+  blocks = std::min<int64_t>(blocks, wave ? 2048 : 4096);
+  while (blocks > 1 && (size_t)blocks * group_bytes > budget) blocks /= 2;
+  if ((size_t)blocks * group_bytes > budget)
     return fail(C2A_ERR_OOM, "search workspace for one workgroup exceeds the device budget");
   const size_t out_bytes = kind == SQ_DISTANCE_QUEUE ? sizeof(StaticOut) : sizeof(c2a_static_result);
   DevBuf dm, dq, dout, dc, dws, dp;
   if ((rc = dm.alloc(tab.size() * sizeof(MeshDev))) ||
       (rc = dq.alloc((size_t)nq * sizeof(StaticQueryDev))) ||
       (rc = dout.alloc((size_t)nq * out_bytes)) || (rc = dc.alloc(sizeof(int64_t))) ||
-      (rc = dws.alloc((size_t)blocks * kStaticBlock * thread_bytes)))
+      (rc = dws.alloc((size_t)blocks * group_bytes)))
     return rc;
   const size_t pair_bytes = kind == SQ_COLLIDE ? (size_t)nq * pair_cap * 2 * sizeof(int32_t) : 0;
   if (pair_bytes && (rc = dp.alloc(pair_bytes))) return rc;
@@ -1360,6 +1363,9 @@ int static_queries(c2a_mesh* const* meshes, int32_t nmesh, int32_t kind, const d
   a.out = (StaticOut*)dout.p;
   a.pairs = pair_bytes ? (int32_t*)dp.p : nullptr;
   a.ws = (SqEntry*)dws.p;
+  a.wave_ws = (unsigned char*)dws.p;
+  a.wave_bytes = (int64_t)group_bytes;
+  a.depth_sum = depth_sum;
   a.counter = (int64_t*)dc.p;
   a.nq = nq;
   a.ws_entries = per_thread;
@@ -1369,7 +1375,9 @@ int static_queries(c2a_mesh* const* meshes, int32_t nmesh, int32_t kind, const d
   a.pair_cap = kind == SQ_COLLIDE ? pair_cap : 0;
   a.rel_err = rel_err;
   a.abs_err = abs_err;
-  HIP_TRY(launch_static(a, (int)blocks, s));
+  // the list's places past a query's contacts hold -1
+  if (pair_bytes) HIP_TRY(hipMemsetAsync(dp.p, 0xff, pair_bytes, s));
+  HIP_TRY(wave ? launch_static_wave(a, (int)blocks, s) : launch_static(a, (int)blocks, s));
   if (kind == SQ_DISTANCE_QUEUE) {
     // the distance-query record: StaticOut's tri is the models' last_tri
     std::vector<StaticOut> h((size_t)nq);

@@ -2,7 +2,9 @@
 // best-first distance search (C2A_Distance with qsize > 2), the distance at
 // contact space, the tolerance query and the triangle-contact form of
 // C2A_Collide (C2A/src/C2A_PQP.cpp:624-968, :1282-1845).  Shared by the gfx950
-// kernel (static_kernel.hip) and the host-side test harness.
+// kernel (static_kernel.hip) and the host-side test harness.  The library
+// runs the best-first searches here, and of the others those that
+// static_wave.h does not take.
 //
 // These searches carry little state beyond a stack or a bounded priority
 // queue, and a batch of them is many short independent traversals, so each
@@ -72,6 +74,11 @@ struct StaticArgs {
   int32_t flag;            // SQ_COLLIDE: 2 = first contact only
   int32_t pair_cap;
   double rel_err, abs_err;
+  // one wavefront per query (static_wave.h)
+  unsigned char* wave_ws;  // per-wavefront workspace, wave_bytes each
+  int64_t wave_bytes;
+  int32_t depth_sum;       // deepest pair of hierarchies
+  int32_t pad;
 };
 
 C2A_HD bool sq_leaf(const GpuNode* n) { return n->first_child < 0; }

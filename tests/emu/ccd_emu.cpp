@@ -352,3 +352,65 @@ extern "C" int emu_static(const double* tris1, int64_t n1, const double* tris2, 
   for (int64_t i = 0; i < nq; i++) static_query(a, i, ws.data());
   return 0;
 }
+
+// The same queries through static_wave.h's wavefront, 64 lanes on fibers.
+#ifdef C2A_EMU_SIMT
+#include "../../c2a_amd/csrc/static_wave.h"
+namespace {
+struct SqCtx {
+  const StaticArgs* a;
+  SqWaveLds* g;
+  unsigned char* ws;
+  int64_t qi;
+};
+void sq_body(int lane, void* p) {
+  SqCtx& c = *(SqCtx*)p;
+  if (c.a->kind == SQ_COLLIDE) sq_wave_query<SQ_COLLIDE>(*c.a, c.qi, *c.g, c.ws, lane);
+  else if (c.a->kind == SQ_TOLERANCE) sq_wave_query<SQ_TOLERANCE>(*c.a, c.qi, *c.g, c.ws, lane);
+  else sq_wave_query<SQ_DISTANCE_CS>(*c.a, c.qi, *c.g, c.ws, lane);
+}
+}  // namespace
+extern "C" int emu_static_wave(const double* tris1, int64_t n1, const double* tris2, int64_t n2,
+                               int kind, const double* poses, const double* params, int flag,
+                               int64_t nq, int pair_cap, int32_t* pairs_out, c2a::StaticOut* out) {
+  Bvh b1, b2;
+  if (build_bvh(tris1, nullptr, nullptr, n1, &b1) || build_bvh(tris2, nullptr, nullptr, n2, &b2))
+    return 1;
+  MeshDev tab[2];
+  tab[0].nodes = b1.nodes.data(); tab[0].tris = b1.tris.data();
+  tab[0].ntri = (int32_t)n1; tab[0].depth = b1.max_depth;
+  tab[1].nodes = b2.nodes.data(); tab[1].tris = b2.tris.data();
+  tab[1].ntri = (int32_t)n2; tab[1].depth = b2.max_depth;
+  std::vector<StaticQueryDev> hq((size_t)nq);
+  for (int64_t i = 0; i < nq; i++) {
+    StaticQueryDev& q = hq[(size_t)i];
+    memset(&q, 0, sizeof(q));
+    q.mesh[1] = 1;
+    memcpy(q.R1, poses + 24 * i, 72); memcpy(q.T1, poses + 24 * i + 9, 24);
+    memcpy(q.R2, poses + 24 * i + 12, 72); memcpy(q.T2, poses + 24 * i + 21, 24);
+    q.param = params ? params[i] : 0.0;
+  }
+  StaticArgs a;
+  memset(&a, 0, sizeof(a));
+  a.meshes = tab;
+  a.q = hq.data();
+  a.out = out;
+  a.pairs = pairs_out;
+  a.nq = nq;
+  a.kind = kind;
+  a.qsize = 2;
+  a.flag = flag;
+  a.pair_cap = pair_cap;
+  a.depth_sum = b1.max_depth + b2.max_depth;
+  if (a.depth_sum > kSqWaveDepth) return 2;
+  // exactly the workspace the library gives it
+  std::vector<unsigned char> ws((size_t)sq_wave_bytes(kind, a.depth_sum, pair_cap));
+  SqWaveLds g;
+  for (int64_t i = 0; i < nq; i++) {
+    memset(&g, 0, sizeof(g));
+    SqCtx c{&a, &g, ws.data(), i};
+    if (simt::launch(sq_body, &c)) return 10;
+  }
+  return 0;
+}
+#endif
