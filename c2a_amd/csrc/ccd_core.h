@@ -134,6 +134,183 @@ C2A_HD T C2A_GLOBAL* gp(T* p) {
   return (T C2A_GLOBAL*)p;
 }
 
+// Wavefront primitives (the host harness runs one lane).
+C2A_HD uint64_t wave_ballot(bool p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint64_t)__ballot(p);
+#elif defined(C2A_EMU_SIMT)
+  return simt::ballot(p);
+#else
+  return p ? 1u : 0u;
+#endif
+}
+C2A_HD int lanes_below(uint64_t m, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  (void)lane;
+  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+#else
+  return __builtin_popcountll(m & ((1ull << lane) - 1));
+#endif
+}
+C2A_HD int lane_bcast(int v, int src) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __shfl(v, src);
+#elif defined(C2A_EMU_SIMT)
+  return simt::bcast(v, src);
+#else
+  (void)src;
+  return v;
+#endif
+}
+// v of lane `src`, the same in every lane (a scalar read, where lane_bcast
+// goes through the LDS crossbar).
+C2A_HD int lane_read(int v, int src) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_readlane(v, __builtin_amdgcn_readfirstlane(src));
+#elif defined(C2A_EMU_SIMT)
+  return simt::bcast(v, src);
+#else
+  (void)src;
+  return v;
+#endif
+}
+C2A_HD double lane_readd(double v, int src) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int s = __builtin_amdgcn_readfirstlane(src);
+  union { double d; int32_t i[2]; } u;
+  u.d = v;
+  u.i[0] = __builtin_amdgcn_readlane(u.i[0], s);
+  u.i[1] = __builtin_amdgcn_readlane(u.i[1], s);
+  return u.d;
+#elif defined(C2A_EMU_SIMT)
+  return simt::bcastd(v, src);
+#else
+  (void)src;
+  return v;
+#endif
+}
+// v of the neighbouring lane (lane ^ 1)
+C2A_HD double lane_xor1d(double v, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  (void)lane;
+  union { double d; int32_t i[2]; } u;
+  u.d = v;   // quad_perm [1, 0, 3, 2]
+  u.i[0] = __builtin_amdgcn_update_dpp(0, u.i[0], 0xB1, 0xf, 0xf, false);
+  u.i[1] = __builtin_amdgcn_update_dpp(0, u.i[1], 0xB1, 0xf, 0xf, false);
+  return u.d;
+#elif defined(C2A_EMU_SIMT)
+  return simt::bcastd(v, lane ^ 1);
+#else
+  (void)lane;
+  return v;
+#endif
+}
+#if defined(__HIP_DEVICE_COMPILE__)
+// Cross-lane data movement inside the vector ALU (DPP): a shuffle through
+// the LDS crossbar takes about 130 cycles, a DPP move about 8.  Six steps
+// reach all 64 lanes: row shifts by 1, 2, 4, 8 within 16 lanes, then lane 15
+// of each row to the next one and lane 31 to the upper half.  Lanes without
+// a source keep `old`.
+#define C2A_DPP_STEPS(X) \
+  X(0x111, 0xf) X(0x112, 0xf) X(0x114, 0xf) X(0x118, 0xf) X(0x142, 0xa) X(0x143, 0xc)
+#endif
+// max over lanes below this one (0 for lane 0); v >= 0
+C2A_HD int excl_prefix_max(int v, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  (void)lane;
+#define C2A_STEP(ctrl, rows)                                            \
+  {                                                                     \
+    const int u = __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false); \
+    v = v > u ? v : u;                                                  \
+  }
+  C2A_DPP_STEPS(C2A_STEP)
+#undef C2A_STEP
+  return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false);   // one lane up
+#elif defined(C2A_EMU_SIMT)
+  (void)lane;
+  return simt::excl_prefix_max(v);
+#else
+  (void)v;
+  (void)lane;
+  return 0;
+#endif
+}
+// Smallest v of the wavefront, the same in every lane.  A NaN counts as no
+// value, as in the reference's sequential `if (v < min) min = v`.
+C2A_HD double wave_mind(double v) {
+  v = v < 1.0 / 0.0 ? v : 1.0 / 0.0;
+#if defined(__HIP_DEVICE_COMPILE__)
+#define C2A_STEP(ctrl, rows)                                                      \
+  {                                                                               \
+    union { double d; int32_t i[2]; } x, u;                                       \
+    x.d = v;                                                                      \
+    u.i[0] = __builtin_amdgcn_update_dpp(x.i[0], x.i[0], ctrl, rows, 0xf, false); \
+    u.i[1] = __builtin_amdgcn_update_dpp(x.i[1], x.i[1], ctrl, rows, 0xf, false); \
+    v = u.d < v ? u.d : v;                                                        \
+  }
+  C2A_DPP_STEPS(C2A_STEP)
+#undef C2A_STEP
+  return lane_readd(v, 63);
+#elif defined(C2A_EMU_SIMT)
+  v = simt::mind(v);
+#endif
+  return v;
+}
+// Largest v of the wavefront (v >= 0), the same in every lane.
+C2A_HD int wave_maxi(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#define C2A_STEP(ctrl, rows)                                            \
+  {                                                                     \
+    const int u = __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false); \
+    v = v > u ? v : u;                                                  \
+  }
+  C2A_DPP_STEPS(C2A_STEP)
+#undef C2A_STEP
+  return lane_read(v, 63);
+#elif defined(C2A_EMU_SIMT)
+  v = simt::maxi(v);
+#endif
+  return v;
+}
+C2A_HD float unif(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+#else
+  return x;
+#endif
+}
+C2A_HD unsigned long long global_add_u64(unsigned long long* p, unsigned long long v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return atomicAdd(p, v);
+#else
+  const unsigned long long o = *p;
+  *p = o + v;
+  return o;
+#endif
+}
+C2A_HD long long lane0_bcast64(long long v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const unsigned long long u = (unsigned long long)v;
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32));
+  return (long long)(((unsigned long long)hi << 32) | lo);
+#elif defined(C2A_EMU_SIMT)
+  return simt::lane0(v);
+#else
+  return v;
+#endif
+}
+C2A_HD int lds_max(int32_t* p, int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return atomicMax(p, v);
+#else
+  int o = *p;
+  if (v > o) *p = v;
+  return o;
+#endif
+}
+
 C2A_HD node_ptr nodes_of(const MeshDev& m) { return (node_ptr)m.nodes; }
 C2A_HD gdouble_ptr tris_of(const MeshDev& m) { return (gdouble_ptr)m.tris; }
 
@@ -255,6 +432,7 @@ struct Wave {
   // Misses ahead in the scan's window share a round: each gets a heap of
   // `mpage` slots (mpage = 0: one heap below X).
   int32_t mpage;             // slots per heap of the current round
+  int32_t nheap;             // ... and its number of heaps
   int32_t mrgen;             // generation of the round below the gathered misses
   int32_t nmr;               // misses gathered (then: covered by that round)
   int32_t mrrec[MR_MAX];     // their replayed record numbers, in scan order
@@ -692,6 +870,30 @@ C2A_HD bool arena_rounds_on(const KArgs& a) {
 #endif
 }
 
+// Whether the traversal enters a pair with RSS distance d and admissible
+// time mt at the current bound.  cmode: Wave::contact.
+C2A_HD bool enters(const Leader& L, int cmode, double d, double mt) {
+  if (cmode == 0)   // C2A.cpp:1284-1349
+    return mt < L.Up && ((d < (L.D - L.abs_err)) || (d * (1 + L.rel_err) < L.D));
+  if (L.mode == MODE_DISTANCE)   // C2A_PQP.cpp:594-617; C2A_Collide (:1068-1070):
+                                 // RectDist <= r1 + r2 exactly when the
+                                 // clamped RSS distance is 0
+    return ((d < (L.D - L.abs_err)) || (d * (1 + L.rel_err) < L.D)) && (cmode != 2 || d == 0.0);
+  return d < L.thr;   // contact enumeration, abs = rel = 0 (C2A.cpp:1760-1761)
+}
+
+// Whether rounds are decided by heap_scan (walk_heaps) or one pair at a time
+// (walk_pairs): heaps of at most 64 pairs, a whole wavefront.
+template <int K>
+C2A_HD bool heaps_on(const KArgs& a, int nl) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return K <= 5;
+#else
+  return K <= 5 && nl >= 64 && !a.arena_rounds;
+#endif
+}
+constexpr int SHARE_MAX = 3;   // pending pairs that can share a round
+
 // One lane's share of a round.
 template <int K, int CAP>
 C2A_HD void round_lane(Wave<K, CAP>& g, const Leader& L, int lane, int nl, const KArgs& a) {
@@ -704,13 +906,14 @@ C2A_HD void round_lane(Wave<K, CAP>& g, const Leader& L, int lane, int nl, const
     return;
   }
   // one heap of g.rdepth levels below slot 0 (a leaf pair: its own values), or
-  // heap r in slots [r * mp, r * mp + mp - 1) below gathered miss r
+  // heap r in slots [r * mp, r * mp + mp - 1) below gathered miss or pending
+  // pair r
   const int mp = g.mpage;
   const bool own = !mp && (g.slot[0].flags & 3) == 3;
-  const int n = mp ? g.nmr * mp : (own ? 1 : (2 << g.rdepth) - 1);
+  const int n = mp ? g.nheap * mp : (own ? 1 : (2 << g.rdepth) - 1);
   for (int h = lane + (own ? 0 : 1); h < n; h += nl) {
     const int l = mp ? h & (mp - 1) : h;
-    if (mp && (l == 0 || l == mp - 1)) continue;   // the miss itself; padding
+    if (mp && (l == 0 || l == mp - 1)) continue;   // the root pair; padding
     compute_slot_below(g, g.slot[h - l], l, M1, M2, contact, g.slot[h]);
   }
 }
@@ -740,6 +943,25 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
                      ar == uni(g.mrrec[0]);
   const int cap = (Shape<K>::NSLOT + 1) / mpage;
   const int nroot = nmr < cap ? nmr : cap;
+  // Pending pairs below the top one that the current bound enters: each will
+  // need a round of its own unless an improving leaf prunes it first, so up
+  // to three of them share this one, each heap a level (two, with more than
+  // one) shallower.
+  int nshare = 0, share = 0;   // pairs sharing; this lane's heap (0: none)
+  if (heaps_on<K>(a, nl) && !multi && !(flags & 8) && (flags & 3) != 3) {
+    const int j = lane & 63, i = L.sp - 2 - j;
+    bool cand = false;
+    if (i >= 0) {
+      const Entry& o = g.stack[i];
+      cand = (o.flags & 3) != 3 && enters(L, g.contact, o.d, o.mt);
+    }
+    const uint64_t cm = wave_ballot(cand);
+    const int nc = (int)__builtin_popcountll(cm);
+    nshare = L.kdepth >= 3 ? (nc < SHARE_MAX ? nc : SHARE_MAX) : (L.kdepth == 2 && nc ? 1 : 0);
+    if (cand && lanes_below(cm, j) < nshare) share = 1 + lanes_below(cm, j);
+  }
+  const int sdepth = L.kdepth - (nshare == 0 ? 0 : (nshare == 1 ? 1 : 2));
+  const int spage = 2 << sdepth;
   lane_sync();
   // the heaps' root pairs into their slots; replayed pairs' transforms are in
   // the arena
@@ -762,9 +984,19 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
     for (int w = lane; w < 15; w += nl)
       x[w] = ((flags & 8) && w < 12) ? xf[12 * (int64_t)ar + w] : s[w];
   }
+  if (share && lane < 64) {
+    Entry& o = g.stack[L.sp - 2 - lane];
+    Slot& r = g.slot[share * spage];
+    for (int i = 0; i < 9; i++) r.R[i] = o.R[i];
+    for (int i = 0; i < 3; i++) r.T[i] = o.T[i];
+    r.b1 = o.b1;
+    r.b2 = o.b2;
+    o.sg = (gen << 8) | (share * spage + 1);
+  }
   if (lane == 0) {
     g.rarena = to_arena ? 1 : 0;
-    g.mpage = multi ? mpage : 0;
+    g.mpage = multi ? mpage : (nshare ? spage : 0);
+    g.nheap = multi ? nroot : 1 + nshare;
     if (to_arena) {
       g.rpb = L.napp;
       e.cp = L.napp;
@@ -783,7 +1015,7 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
       // a replayed pair that must now be expanded (a miss) usually needs
       // only a level or two: a shallow first round has a shorter chain of
       // dependent node loads
-      g.rdepth = ((flags & 8) && L.kmiss > 0 && L.kmiss < L.kdepth) ? L.kmiss : L.kdepth;
+      g.rdepth = ((flags & 8) && L.kmiss > 0 && L.kmiss < L.kdepth) ? L.kmiss : sdepth;
     }
   }
   if (to_arena) {
@@ -863,183 +1095,6 @@ inline double root_rss_distance(const GpuNode* r1n, const GpuNode* r2n, const do
   double d, mt;
   (void)pair_values((node_ptr)r1n, (node_ptr)r2n, 0, 0, R, T, R1, none, none, true, d, mt);
   return d;
-}
-
-// Wavefront primitives of the scan (the host harness runs one lane).
-C2A_HD uint64_t wave_ballot(bool p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return (uint64_t)__ballot(p);
-#elif defined(C2A_EMU_SIMT)
-  return simt::ballot(p);
-#else
-  return p ? 1u : 0u;
-#endif
-}
-C2A_HD int lanes_below(uint64_t m, int lane) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  (void)lane;
-  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                        __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-#else
-  return __builtin_popcountll(m & ((1ull << lane) - 1));
-#endif
-}
-C2A_HD int lane_bcast(int v, int src) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __shfl(v, src);
-#elif defined(C2A_EMU_SIMT)
-  return simt::bcast(v, src);
-#else
-  (void)src;
-  return v;
-#endif
-}
-// v of lane `src`, the same in every lane (a scalar read, where lane_bcast
-// goes through the LDS crossbar).
-C2A_HD int lane_read(int v, int src) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_readlane(v, __builtin_amdgcn_readfirstlane(src));
-#elif defined(C2A_EMU_SIMT)
-  return simt::bcast(v, src);
-#else
-  (void)src;
-  return v;
-#endif
-}
-C2A_HD double lane_readd(double v, int src) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const int s = __builtin_amdgcn_readfirstlane(src);
-  union { double d; int32_t i[2]; } u;
-  u.d = v;
-  u.i[0] = __builtin_amdgcn_readlane(u.i[0], s);
-  u.i[1] = __builtin_amdgcn_readlane(u.i[1], s);
-  return u.d;
-#elif defined(C2A_EMU_SIMT)
-  return simt::bcastd(v, src);
-#else
-  (void)src;
-  return v;
-#endif
-}
-// v of the neighbouring lane (lane ^ 1)
-C2A_HD double lane_xor1d(double v, int lane) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  (void)lane;
-  union { double d; int32_t i[2]; } u;
-  u.d = v;   // quad_perm [1, 0, 3, 2]
-  u.i[0] = __builtin_amdgcn_update_dpp(0, u.i[0], 0xB1, 0xf, 0xf, false);
-  u.i[1] = __builtin_amdgcn_update_dpp(0, u.i[1], 0xB1, 0xf, 0xf, false);
-  return u.d;
-#elif defined(C2A_EMU_SIMT)
-  return simt::bcastd(v, lane ^ 1);
-#else
-  (void)lane;
-  return v;
-#endif
-}
-#if defined(__HIP_DEVICE_COMPILE__)
-// Cross-lane data movement inside the vector ALU (DPP): a shuffle through
-// the LDS crossbar takes about 130 cycles, a DPP move about 8.  Six steps
-// reach all 64 lanes: row shifts by 1, 2, 4, 8 within 16 lanes, then lane 15
-// of each row to the next one and lane 31 to the upper half.  Lanes without
-// a source keep `old`.
-#define C2A_DPP_STEPS(X) \
-  X(0x111, 0xf) X(0x112, 0xf) X(0x114, 0xf) X(0x118, 0xf) X(0x142, 0xa) X(0x143, 0xc)
-#endif
-// max over lanes below this one (0 for lane 0); v >= 0
-C2A_HD int excl_prefix_max(int v, int lane) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  (void)lane;
-#define C2A_STEP(ctrl, rows)                                            \
-  {                                                                     \
-    const int u = __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false); \
-    v = v > u ? v : u;                                                  \
-  }
-  C2A_DPP_STEPS(C2A_STEP)
-#undef C2A_STEP
-  return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false);   // one lane up
-#elif defined(C2A_EMU_SIMT)
-  (void)lane;
-  return simt::excl_prefix_max(v);
-#else
-  (void)v;
-  (void)lane;
-  return 0;
-#endif
-}
-// Smallest v of the wavefront, the same in every lane.  A NaN counts as no
-// value, as in the reference's sequential `if (v < min) min = v`.
-C2A_HD double wave_mind(double v) {
-  v = v < 1.0 / 0.0 ? v : 1.0 / 0.0;
-#if defined(__HIP_DEVICE_COMPILE__)
-#define C2A_STEP(ctrl, rows)                                                      \
-  {                                                                               \
-    union { double d; int32_t i[2]; } x, u;                                       \
-    x.d = v;                                                                      \
-    u.i[0] = __builtin_amdgcn_update_dpp(x.i[0], x.i[0], ctrl, rows, 0xf, false); \
-    u.i[1] = __builtin_amdgcn_update_dpp(x.i[1], x.i[1], ctrl, rows, 0xf, false); \
-    v = u.d < v ? u.d : v;                                                        \
-  }
-  C2A_DPP_STEPS(C2A_STEP)
-#undef C2A_STEP
-  return lane_readd(v, 63);
-#elif defined(C2A_EMU_SIMT)
-  v = simt::mind(v);
-#endif
-  return v;
-}
-// Largest v of the wavefront (v >= 0), the same in every lane.
-C2A_HD int wave_maxi(int v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-#define C2A_STEP(ctrl, rows)                                            \
-  {                                                                     \
-    const int u = __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false); \
-    v = v > u ? v : u;                                                  \
-  }
-  C2A_DPP_STEPS(C2A_STEP)
-#undef C2A_STEP
-  return lane_read(v, 63);
-#elif defined(C2A_EMU_SIMT)
-  v = simt::maxi(v);
-#endif
-  return v;
-}
-C2A_HD float unif(float x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
-#else
-  return x;
-#endif
-}
-C2A_HD unsigned long long global_add_u64(unsigned long long* p, unsigned long long v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return atomicAdd(p, v);
-#else
-  const unsigned long long o = *p;
-  *p = o + v;
-  return o;
-#endif
-}
-C2A_HD long long lane0_bcast64(long long v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const unsigned long long u = (unsigned long long)v;
-  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(u >> 32));
-  return (long long)(((unsigned long long)hi << 32) | lo);
-#elif defined(C2A_EMU_SIMT)
-  return simt::lane0(v);
-#else
-  return v;
-#endif
-}
-C2A_HD int lds_max(int32_t* p, int v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return atomicMax(p, v);
-#else
-  int o = *p;
-  if (v > o) *p = v;
-  return o;
-#endif
 }
 
 // Training samples of one replayed step: every record below the root whose
@@ -1786,18 +1841,6 @@ C2A_HD bool walk_pairs(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
   }
 }
 
-// Whether the traversal enters a pair with RSS distance d and admissible
-// time mt at the current bound.  cmode: Wave::contact.
-C2A_HD bool enters(const Leader& L, int cmode, double d, double mt) {
-  if (cmode == 0)   // C2A.cpp:1284-1349
-    return mt < L.Up && ((d < (L.D - L.abs_err)) || (d * (1 + L.rel_err) < L.D));
-  if (L.mode == MODE_DISTANCE)   // C2A_PQP.cpp:594-617; C2A_Collide (:1068-1070):
-                                 // RectDist <= r1 + r2 exactly when the
-                                 // clamped RSS distance is 0
-    return ((d < (L.D - L.abs_err)) || (d * (1 + L.rel_err) < L.D)) && (cmode != 2 || d == 0.0);
-  return d < L.thr;   // contact enumeration, abs = rel = 0 (C2A.cpp:1760-1761)
-}
-
 // A tested leaf pair (C2A.cpp:1141-1183, C2A_PQP.cpp:493-520: strict <) with
 // triangle distance dTri; returns whether it becomes the closest one.
 C2A_HD bool leaf_update(Leader& L, int cmode, int strict, double dTri, double mleaf) {
@@ -2074,13 +2117,7 @@ C2A_HD bool walk_heaps(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
 
 template <int K, int CAP>
 C2A_HD bool walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (K <= 5) return walk_heaps(g, L, a, lane, nl);
-  else return walk_pairs(g, L, a, lane, nl);
-#else
-  return (K <= 5 && nl >= 64 && !a.arena_rounds) ? walk_heaps(g, L, a, lane, nl)
-                                                 : walk_pairs(g, L, a, lane, nl);
-#endif
+  return heaps_on<K>(a, nl) ? walk_heaps(g, L, a, lane, nl) : walk_pairs(g, L, a, lane, nl);
 }
 
 // After a step's walk: closest points of a replayed last improving leaf
