@@ -190,18 +190,41 @@ int auto_replay_log(const std::vector<MeshDev>& tab) {
   return cap;
 }
 
+int compute_units() {
+  int dev = 0, cus = 256;
+  (void)hipGetDevice(&dev);
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 256;
+  return cus;
+}
+
 // Resident workgroups: the kernel is persistent, so launching more than fit
 // at once only adds workgroups that find the queue empty.
 int grid_blocks(int K, int CAP, int NW, int64_t nq, bool learned = false) {
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  hipDeviceProp_t prop;
-  int cus = 256;
-  if (hipGetDeviceProperties(&prop, dev) == hipSuccess) cus = prop.multiProcessorCount;
+  const int cus = compute_units();
   int per_cu = kernel_blocks_per_cu(K, CAP, NW, learned);
   if (per_cu < 1) per_cu = 1;
   const int64_t cap = (int64_t)cus * per_cu;
   return (int)std::max<int64_t>(1, std::min<int64_t>(nq, cap));
+}
+
+// The four-wavefront shape (256 speculative slots): the tail pass's, and that
+// of small batches.
+constexpr int kWideK = 7;
+constexpr int kWideWaves = 4;
+
+// Small batches run four wavefronts per query: with one, most of the chip
+// idles while the longest queries finish; with four, the replay and the
+// rounds (up to eight heaps of pending pairs each) take four times the lanes,
+// and a compute unit holds one query instead of four.  The lines are where
+// the two met on MI355X (256 compute units), ms with one -> four wavefronts.
+// CCD, 8192-triangle knots: 1 query 127 -> 96, 256 queries 154 -> 107, 1024
+// 162 -> 127, 1536 176 -> 183, 2048 193 -> 201 (a line at 4 per compute unit).
+// Distance queries: 64 14.2 -> 9.8, 512 21.8 -> 19.6, 1024 22.4 -> 25.4 (2 per
+// compute unit).
+bool wide_batch(int64_t nq, int CAP, bool ccd) {
+  return nq <= (int64_t)compute_units() * (ccd ? 4 : 2) &&
+         kernel_shape_ok(kWideK, CAP, kWideWaves, false);
 }
 
 int prepare_queries(const std::vector<MeshDev>& tab, const c2a_query* q, int64_t nq,
@@ -315,10 +338,6 @@ int fill_args(c2a_batch* b, const c2a_params* p) {
   return C2A_OK;
 }
 
-// The tail pass's kernel shape.
-constexpr int kTailK = 5;
-constexpr int kTailWaves = 4;
-
 __global__ void zero_counter(int64_t* c) { *c = 0; }
 __global__ void zero_tail(int64_t* c, int32_t* n) {
   *c = 0;
@@ -343,7 +362,7 @@ int run_batch(const c2a_batch* b, hipStream_t s) {
   }
   int rc = run_kernel(b->args, b->K, b->CAP, b->NW, b->blocks, s);
   if (rc || !b->tail) return rc;
-  const hipError_t e = launch_ccd(b->args2, kTailK, b->CAP, kTailWaves, b->blocks2, s);
+  const hipError_t e = launch_ccd(b->args2, kWideK, b->CAP, kWideWaves, b->blocks2, s);
   if (e != hipSuccess) return hip_fail(e, "launch_ccd (tail pass)");
   return C2A_OK;
 }
@@ -353,7 +372,7 @@ int run_batch(const c2a_batch* b, hipStream_t s) {
 int setup_tail(c2a_batch* b, const c2a_params* p) {
   const int64_t budget = p->tail_budget;
   if (budget <= 0 || b->nq < 2 || b->scorer || b->sample_cap > 0 ||
-      !kernel_shape_ok(kTailK, b->CAP, kTailWaves, false))
+      !kernel_shape_ok(kWideK, b->CAP, kWideWaves, false))
     return C2A_OK;
   int rc;
   if ((rc = b->d_tail.alloc((size_t)b->nq * sizeof(TailRec))) ||
@@ -369,7 +388,7 @@ int setup_tail(c2a_batch* b, const c2a_params* p) {
   b->args2.tail_pass = 1;
   b->args2.counter = (int64_t*)b->d_tctr.p;
   // one replay arena per workgroup: no more workgroups than the first launch
-  b->blocks2 = std::min(grid_blocks(kTailK, b->CAP, kTailWaves, b->nq), b->blocks);
+  b->blocks2 = std::min(grid_blocks(kWideK, b->CAP, kWideWaves, b->nq), b->blocks);
   b->tail = true;
   return C2A_OK;
 }
@@ -473,6 +492,10 @@ int c2a_ccd_batch_noalloc(c2a_mesh* const* meshes, int32_t nmesh, const double* 
   const int CAP = need <= 48 ? 48 : (need <= 96 ? 96 : (need <= 192 ? 192 : -1));
   if (CAP < 0) return fail(C2A_ERR_UNSUPPORTED, "hierarchies too deep for the traversal stack");
   if (CAP == 192) K = 5;   // the deepest stack's one depth (no result depends on it)
+  if (p->spec_depth == 0 && p->waves_per_query == 0 && wide_batch(nq, CAP, true)) {
+    K = kWideK;
+    NW = kWideWaves;
+  }
   const int logcap = p->replay_log == -1 ? 1024 : p->replay_log;
   if (logcap < 0) return fail(C2A_ERR_BAD_ARG, "replay_log must be -1 (1024) or >= 0");
   const size_t room = kScratchBytes - kScratchArena;
@@ -815,7 +838,7 @@ int c2a_batch_create(c2a_mesh* const* meshes, int32_t nmesh, const c2a_query* q,
     delete b;
     return fail(C2A_ERR_BAD_ARG, "strict must be 0 or 1");
   }
-  if (params && params->tail_waves != 0 && params->tail_waves != kTailWaves) {
+  if (params && params->tail_waves != 0 && params->tail_waves != kWideWaves) {
     delete b;
     return fail(C2A_ERR_BAD_ARG, "tail_waves must be 0 or 4");
   }
@@ -859,6 +882,12 @@ int c2a_batch_create(c2a_mesh* const* meshes, int32_t nmesh, const c2a_query* q,
   }
   // the deepest stack is instantiated at one depth; the depth changes no result
   if (b->CAP == 192) b->K = 5;
+  if ((!params || (params->spec_depth == 0 && params->waves_per_query == 0 &&
+                   params->tail_budget <= 0)) &&
+      !b->scorer && b->sample_cap == 0 && wide_batch(nq, b->CAP, true)) {
+    b->K = kWideK;
+    b->NW = kWideWaves;
+  }
   b->blocks = grid_blocks(b->K, b->CAP, b->NW, nq, b->scorer != nullptr);
   const bool feats = b->scorer || b->sample_cap > 0;
   if (b->logcap > 0 && nq > 0) {
@@ -1092,7 +1121,8 @@ int c2a_ccd_step(c2a_mesh* const* meshes, int32_t nmesh, const c2a_step_query* q
   }
   int CAP = pick_cap(tab, pairs.data(), nq, 2);
   if (CAP < 0) return fail(C2A_ERR_UNSUPPORTED, "hierarchies too deep for the traversal stack");
-  const int K = 5;
+  const bool wide = wide_batch(nq, CAP, false);
+  const int K = wide ? kWideK : 5, NW = wide ? kWideWaves : 1;
   DevBuf dm, din, dout, dc;
   if ((rc = dm.alloc(tab.size() * sizeof(MeshDev))) || (rc = din.alloc((size_t)nq * sizeof(StepDev))) ||
       (rc = dout.alloc((size_t)nq * sizeof(c2a_step_result))) || (rc = dc.alloc(sizeof(int64_t))))
@@ -1109,7 +1139,7 @@ int c2a_ccd_step(c2a_mesh* const* meshes, int32_t nmesh, const c2a_step_query* q
   a.nq = nq;
   a.mode = MODE_STEP;
   a.max_iter = 150;
-  if ((rc = run_kernel(a, K, CAP, 1, grid_blocks(K, CAP, 1, nq), s))) return rc;
+  if ((rc = run_kernel(a, K, CAP, NW, grid_blocks(K, CAP, NW, nq), s))) return rc;
   HIP_TRY(hipMemcpyAsync(out, dout.p, (size_t)nq * sizeof(c2a_step_result), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   return C2A_OK;
@@ -1141,7 +1171,8 @@ static int contact_queries(c2a_mesh* const* meshes, int32_t nmesh, const double*
   }
   int CAP = pick_cap(tab, mesh_pairs, nq, 2);
   if (CAP < 0) return fail(C2A_ERR_UNSUPPORTED, "hierarchies too deep for the traversal stack");
-  const int K = 5;
+  const bool wide = wide_batch(nq, CAP, false);
+  const int K = wide ? kWideK : 5, NW = wide ? kWideWaves : 1;
   DevBuf dm, din, dout, dc, drec;
   if ((rc = dm.alloc(tab.size() * sizeof(MeshDev))) ||
       (rc = din.alloc((size_t)nq * sizeof(ContactDev))) ||
@@ -1161,7 +1192,7 @@ static int contact_queries(c2a_mesh* const* meshes, int32_t nmesh, const double*
   a.counter = (int64_t*)dc.p;
   a.nq = nq;
   a.mode = MODE_CONTACT;
-  if ((rc = run_kernel(a, K, CAP, 1, grid_blocks(K, CAP, 1, nq), s))) return rc;
+  if ((rc = run_kernel(a, K, CAP, NW, grid_blocks(K, CAP, NW, nq), s))) return rc;
   HIP_TRY(hipMemcpyAsync(counts_out, dout.p, (size_t)nq * sizeof(int32_t), hipMemcpyDeviceToHost, s));
   if (cap > 0)
     HIP_TRY(hipMemcpyAsync(out, drec.p, (size_t)nq * cap * sizeof(c2a_contact),
@@ -1245,7 +1276,8 @@ static int distance_queries(c2a_mesh* const* meshes, int32_t nmesh, const double
   }
   int CAP = pick_cap(tab, mesh_pairs, nq, 2);
   if (CAP < 0) return fail(C2A_ERR_UNSUPPORTED, "hierarchies too deep for the traversal stack");
-  const int K = 5;
+  const bool wide = wide_batch(nq, CAP, false);
+  const int K = wide ? kWideK : 5, NW = wide ? kWideWaves : 1;
   DevBuf dm, din, dout, dc;
   if ((rc = dm.alloc(tab.size() * sizeof(MeshDev))) ||
       (rc = din.alloc((size_t)nq * sizeof(ContactDev))) ||
@@ -1263,7 +1295,7 @@ static int distance_queries(c2a_mesh* const* meshes, int32_t nmesh, const double
   a.counter = (int64_t*)dc.p;
   a.nq = nq;
   a.mode = MODE_DISTANCE;
-  if ((rc = run_kernel(a, K, CAP, 1, grid_blocks(K, CAP, 1, nq), s))) return rc;
+  if ((rc = run_kernel(a, K, CAP, NW, grid_blocks(K, CAP, NW, nq), s))) return rc;
   HIP_TRY(hipMemcpyAsync(out, dout.p, (size_t)nq * sizeof(c2a_distance_result),
                          hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));

@@ -401,6 +401,10 @@ struct Slot {            // speculative pair values, heap-indexed below X
 template <int K>
 struct Shape {
   static constexpr int NSLOT = (1 << (K + 1)) - 1;
+  // Deepest heap a round makes: 62 pairs, which one wavefront decides at once
+  // (heap_scan); larger slot arrays (K = 7, four wavefronts) hold several.
+  // K = 6 walks its 126-pair heaps one pair at a time.
+  static constexpr int DEPTH = K == 7 ? 5 : K;
   static constexpr int PER_LANE = (NSLOT - 1 + 63) / 64;
 };
 
@@ -887,12 +891,11 @@ C2A_HD bool enters(const Leader& L, int cmode, double d, double mt) {
 template <int K>
 C2A_HD bool heaps_on(const KArgs& a, int nl) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  return K <= 5;
+  return K != 6;
 #else
-  return K <= 5 && nl >= 64 && !a.arena_rounds;
+  return K != 6 && nl >= 64 && !a.arena_rounds;
 #endif
 }
-constexpr int SHARE_MAX = 3;   // pending pairs that can share a round
 
 // One lane's share of a round.
 template <int K, int CAP>
@@ -944,9 +947,9 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
   const int cap = (Shape<K>::NSLOT + 1) / mpage;
   const int nroot = nmr < cap ? nmr : cap;
   // Pending pairs below the top one that the current bound enters: each will
-  // need a round of its own unless an improving leaf prunes it first, so up
-  // to three of them share this one, each heap a level (two, with more than
-  // one) shallower.
+  // need a round of its own unless an improving leaf prunes it first, so they
+  // share this one, up to four heaps (eight in the 256 slots of K = 7), each
+  // as deep as the slots allow.
   int nshare = 0, share = 0;   // pairs sharing; this lane's heap (0: none)
   if (heaps_on<K>(a, nl) && !multi && !(flags & 8) && (flags & 3) != 3) {
     const int j = lane & 63, i = L.sp - 2 - j;
@@ -957,10 +960,13 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
     }
     const uint64_t cm = wave_ballot(cand);
     const int nc = (int)__builtin_popcountll(cm);
-    nshare = L.kdepth >= 3 ? (nc < SHARE_MAX ? nc : SHARE_MAX) : (L.kdepth == 2 && nc ? 1 : 0);
+    const int most = K == 7 ? 7 : (L.kdepth >= 3 ? 3 : L.kdepth - 1);
+    nshare = nc < most ? nc : most;
     if (cand && lanes_below(cm, j) < nshare) share = 1 + lanes_below(cm, j);
   }
-  const int sdepth = L.kdepth - (nshare == 0 ? 0 : (nshare == 1 ? 1 : 2));
+  // heaps of depth d take 2 << d of the 2 << K slots
+  int sdepth = K - (nshare == 0 ? 0 : (nshare == 1 ? 1 : (nshare <= 3 ? 2 : 3)));
+  if (sdepth > L.kdepth) sdepth = L.kdepth;
   const int spage = 2 << sdepth;
   lane_sync();
   // the heaps' root pairs into their slots; replayed pairs' transforms are in
@@ -1893,7 +1899,7 @@ C2A_HD int heap_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, const Cur& x, i
     const uint64_t sm = wave_ballot(second);
     lv = 31 - clz32((unsigned)(loc + 1));
     int r = 0;
-    for (int k = 1; k <= (K < 5 ? K : 5); k++) {
+    for (int k = 1; k <= Shape<K>::DEPTH && k <= 5; k++) {
       if (k <= lv) {
         const int anc = ((loc + 1) >> (lv - k)) - 1;
         const int late = (int)((sm >> (anc - 1)) & 1);
@@ -2372,7 +2378,7 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
     return false;
   }
   L.qi = qi;
-  L.kdepth = K;
+  L.kdepth = Shape<K>::DEPTH;
   L.kmiss = a.miss_depth;
   L.klog = a.logcap;
   L.kext = a.ext_levels;
@@ -2506,7 +2512,7 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
     const int big = n1 > n2 ? n1 : n2;
     int b = 0;
     while (b + 1 < a.ntune && big > a.tune_ntri[b]) b++;
-    L.kdepth = a.tune_depth[b] < K ? a.tune_depth[b] : K;
+    L.kdepth = a.tune_depth[b] < Shape<K>::DEPTH ? a.tune_depth[b] : Shape<K>::DEPTH;
     L.kmiss = a.tune_miss[b];
     L.klog = a.tune_log[b] < a.logcap ? a.tune_log[b] : a.logcap;
     L.kext = a.tune_ext[b];

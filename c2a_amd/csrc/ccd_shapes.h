@@ -18,7 +18,7 @@
   X(1, 48, 1, 0) X(2, 48, 1, 0) X(3, 48, 1, 0) X(4, 48, 1, 0) X(5, 48, 1, 0)            \
   X(6, 48, 1, 0) X(1, 96, 1, 0) X(2, 96, 1, 0) X(3, 96, 1, 0) X(4, 96, 1, 0)            \
   X(5, 96, 1, 0) X(6, 96, 1, 0) X(5, 48, 1, 1) X(5, 96, 1, 1) X(5, 192, 1, 0)          \
-  X(5, 192, 1, 1) X(5, 48, 4, 0) X(5, 96, 4, 0)
+  X(5, 192, 1, 1) X(7, 48, 4, 0) X(7, 96, 4, 0)
 
 namespace c2a {
 

@@ -66,8 +66,9 @@ typedef struct {
   double contact_scale;
   double contact_offset;
   int32_t spec_depth;       /* speculative subtree depth per round, 0 = auto */
-  int32_t waves_per_query;  /* wavefronts cooperating on one query; this
-                               build provides 1 (0 = 1) */
+  int32_t waves_per_query;  /* wavefronts cooperating on one query: 1, or
+                               0 (default) = chosen from the batch size.  No
+                               result depends on it. */
   int32_t replay_log;       /* expansions logged per CA step for the next step's
                                replay; -1 (default) = from the largest mesh
                                (8192, or ntri / 8 rounded up to a power of

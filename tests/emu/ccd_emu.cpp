@@ -240,6 +240,7 @@ extern "C" int emu_ccd_batch(const double* tris1, int64_t n1, const double* tris
       case 3: return small ? run<3, 48>(ka) : run<3, 96>(ka);
       case 4: return small ? run<4, 48>(ka) : run<4, 96>(ka);
       case 5: return small ? run<5, 48>(ka) : run<5, 96>(ka);
+      case 7: return small ? run<7, 48>(ka) : run<7, 96>(ka);   // 256 slots
       default: return small ? run<6, 48>(ka) : run<6, 96>(ka);
     }
   };
@@ -261,7 +262,9 @@ extern "C" int emu_ccd_batch(const double* tris1, int64_t n1, const double* tris
   return run_shape(a);
 }
 
-// Static distance queries (MODE_DISTANCE) between two meshes, one lane.
+// Static distance queries (MODE_DISTANCE) between two meshes.
+static int emu_distance_k = 5;
+extern "C" void emu_set_distance_k(int k) { emu_distance_k = k; }
 extern "C" int emu_distance(const double* tris1, int64_t n1, const double* tris2, int64_t n2,
                             const double* poses, const int32_t* seeds, double rel_err,
                             double abs_err, int64_t nq, c2a_distance_result* out,
@@ -301,6 +304,7 @@ extern "C" int emu_distance(const double* tris1, int64_t n1, const double* tris2
   a.nq = nq;
   a.mode = MODE_DISTANCE;
   const bool small = b1.max_depth + b2.max_depth + 2 <= 48;
+  if (emu_distance_k == 7) return small ? run<7, 48>(a) : run<7, 96>(a);
   return small ? run<5, 48>(a) : run<5, 96>(a);
 }
 

@@ -1,6 +1,6 @@
 """The lane-parallel decision of a round's heap (heap_scan in ccd_core.h) with
 64 lanes on the CPU, against the FP64 oracle field by field: every heap depth
-(2 to 62 pairs), hierarchies that are a single leaf on one or both sides,
+(2 to 62 pairs; K = 7: 256 slots, up to eight heaps a round), hierarchies that are a single leaf on one or both sides,
 heaps cut short by leaf pairs, and each traversal that uses it (CCD steps,
 contact enumeration, distance and its overlap-only form)."""
 import ctypes as C
@@ -24,6 +24,7 @@ def emu64():
     L.emu_set_arena_rounds.argtypes = [C.c_int]
     L.emu_set_arena_rounds(0)
     yield L
+    L.emu_set_distance_k(5)
     L.emu_set_arena_rounds(1)
 
 
@@ -35,7 +36,7 @@ def mesh(kind):
     return W.torus_knot(n_seg=24, n_ring=5)[0].reshape(-1, 9)
 
 
-@pytest.mark.parametrize("K", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 7])
 @pytest.mark.parametrize("m1,m2", [("knot", "knot"), ("one", "knot"), ("three", "one")])
 def test_heaps_ccd_bit_exact(emu64, m1, m2, K):
     t1, t2 = mesh(m1), mesh(m2)
@@ -44,13 +45,16 @@ def test_heaps_ccd_bit_exact(emu64, m1, m2, K):
     ref = O.batch_toc(O.OModel(t1), O.OModel(t2), *P, 1e-3, 1e-4,
                       seeds=np.zeros((nq, 2), np.int32), with_contacts=True)
     got = run_emu(emu64, t1, t2, P,
-                  G.default_params(tol_d=1e-3, tol_t=1e-4, spec_depth=K, miss_depth=min(K, 3)), K)
+                  G.default_params(tol_d=1e-3, tol_t=1e-4, spec_depth=min(K, 6),
+                                   miss_depth=min(K, 3)), K)
     same(ref, got)
 
 
+@pytest.mark.parametrize("K", [5, 7])
 @pytest.mark.parametrize("rel,abs_,overlap", [(0.0, 0.0, 0), (0.5, 0.02, 0), (0.0, 0.0, 1)])
-def test_heaps_distance_bit_exact(emu64, rel, abs_, overlap):
+def test_heaps_distance_bit_exact(emu64, rel, abs_, overlap, K):
     t1, t2 = mesh("knot"), mesh("three")
+    emu64.emu_set_distance_k(K)
     for a, b in ((t1, t1), (t1, t2)):
         rng = np.random.default_rng(int(rel * 10 + 7))
         cases = [D.random_case(rng, s) for s in rng.uniform(0.0, 1.6, 8)]
