@@ -500,7 +500,9 @@ struct Leader {
   int kext;                      // levels of speculative extension in the replay
   int kx;                        // ... this step: kext, or 0 after a step with few misses
   int nmiss;                     // misses the scan met in this step
-  unsigned char* ab;             // this wavefront's replay arena
+  unsigned char* ab;             // the query's replay arena
+  unsigned char* own;            // this workgroup's replay arena
+  int fetched;                   // a query has been taken (and is done at the next fetch)
 };
 
 C2A_HD int node_leaf(node_ptr n) { return n->first_child < 0; }
@@ -2275,6 +2277,11 @@ C2A_HD void hand_over(const Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane
     t.flags = L.flags;
     t.last1 = L.last1;
     t.last2 = L.last2;
+    t.nlog = L.nlog_prev;
+    t.logbuf = L.logbuf;
+    t.nmiss = L.nmiss;
+    // a wavefront that takes further queries writes over its arena
+    t.ab = (a.tail_left > 0 && a.logcap > 0) ? L.ab : nullptr;
 #if defined(__HIP_DEVICE_COMPILE__)
     a.tail_list[atomicAdd(a.tail_count, 1)] = (int32_t)L.qi;
 #else
@@ -2282,6 +2289,18 @@ C2A_HD void hand_over(const Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane
 #endif
   }
   L.state = ST_FETCH;
+}
+
+// Whether every query has been taken and at most tail_left are unfinished.
+C2A_HD bool few_left(const KArgs& a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int64_t taken = __hip_atomic_load(a.counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int32_t done = __hip_atomic_load(a.finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+  const int64_t taken = *a.counter;
+  const int32_t done = *a.finished;
+#endif
+  return uni(taken >= a.nq && a.nq - done <= a.tail_left ? 1 : 0) != 0;
 }
 
 // End of a step in the CA loop (C2A.cpp:2029-2123): schedules the next step
@@ -2339,7 +2358,9 @@ C2A_HD void after_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
         L.numCA++;
         L.Up = 1.0 - L.lamda;
         L.state = ST_STEP;
-        if (a.tail_budget > 0 && !a.tail_pass && L.bv >= a.tail_budget) hand_over(g, L, a, lane);
+        if ((a.tail_budget > 0 && !a.tail_pass && L.bv >= a.tail_budget) ||
+            (a.tail_left > 0 && !a.tail_pass && few_left(a)))
+          hand_over(g, L, a, lane);
         return;
       }
     }
@@ -2366,6 +2387,14 @@ C2A_HD int64_t take_ticket(Wave<K, CAP>& g, int64_t* counter, int lane) {
 
 template <int K, int CAP>
 C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
+  if (a.tail_left > 0 && !a.tail_pass && L.fetched && lane == 0) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    atomicAdd(a.finished, 1);
+#else
+    (*a.finished)++;
+#endif
+  }
+  L.fetched = 1;
   int64_t qi = take_ticket(g, a.counter, lane);
   if (a.tail_pass) {   // the first launch's hand-overs
     if (qi >= *a.tail_count) {
@@ -2546,6 +2575,12 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
     L.flags = t.flags;
     L.last1 = t.last1;
     L.last2 = t.last2;
+    L.ab = t.ab ? t.ab : L.own;
+    if (t.ab) {
+      L.nlog_prev = t.nlog;
+      L.logbuf = t.logbuf;
+      L.nmiss = t.nmiss;
+    }
     L.state = ST_STEP;
   }
   return true;

@@ -44,6 +44,8 @@ __global__ void __launch_bounds__(64 * NW) ccd_kernel(KArgs a) {
   L.sp = 0;
   L.ab = a.logcap > 0 ? a.arena + (size_t)blockIdx.x * arena_bytes(a.logcap, a.feats != 0)
                       : nullptr;
+  L.own = L.ab;
+  L.fetched = 0;
   for (;;) {
     leader_run(g, L, a, lane, 64 * NW);
     if (L.state == ST_DONE) break;

@@ -37,7 +37,11 @@ struct TailRec {
   double lamda, lastLamda, Up, M;   // M: the last step's mint (error schedule)
   double p1[3], p2[3];              // closest points of the last improving leaf
   int64_t bv, tri;
-  int32_t nItrs, numCA, flags, last1, last2, pad[3];
+  int32_t nItrs, numCA, flags, last1, last2;
+  // The replay goes on in the first launch's arena slice, which its wavefront
+  // no longer uses (null: the next step starts without a replay).
+  int32_t nlog, logbuf, nmiss;
+  unsigned char* ab;
 };
 
 // One explicit CA step (backs C2A_TimeOfContactStep).
@@ -235,6 +239,11 @@ struct KArgs {
   int64_t tail_budget;     // 0: one launch
   int32_t tail_pass;       // 1 in the second launch: queries come from tail_list
   int32_t pad2;
+  // Or: once no more than tail_left queries are unfinished and none waits,
+  // every one of them is handed over at the end of its CA step (0: off).
+  int32_t tail_left;
+  int32_t pad3;
+  int32_t* finished;       // queries done (tail_left > 0)
   TailRec* tail_rec;       // per query
   int32_t* tail_list;      // queries handed over, in hand-over order
   int32_t* tail_count;     // their number

@@ -40,6 +40,9 @@ extern "C" void emu_set_arena_rounds(int on) { emu_arena_rounds = on; }
 // handed over and continued by a second run (0 = one run).
 static int64_t emu_tail_budget = 0;
 static int64_t emu_tail_handed = 0;
+// Hand-over of the last unfinished queries, the library's rule for batches.
+static int emu_tail_left = 0;
+extern "C" void emu_set_tail_left(int n) { emu_tail_left = n; }
 extern "C" void emu_set_tail_budget(int64_t b) { emu_tail_budget = b; }
 // The extension switched per step by the previous step's misses (the
 // library's mode for the autotuned levels).
@@ -111,7 +114,7 @@ static void simt_body(int lane, void* p) {
   Leader L;
   memset(&L, 0, sizeof(L));
   L.state = ST_FETCH;
-  L.ab = c.ab;
+  L.ab = L.own = c.ab;
   for (;;) {
     leader_run(g, L, a, lane, 64);
     if (L.state == ST_DONE) break;
@@ -131,7 +134,10 @@ static void simt_body(int lane, void* p) {
 
 template <int K, int CAP>
 static int run(const KArgs& a) {
-  std::vector<unsigned char> arena(a.logcap > 0 ? arena_bytes(a.logcap, a.feats != 0) : 1);
+  // (the tail pass of tail_left goes on in the first run's arena)
+  static std::vector<unsigned char> first, second;
+  std::vector<unsigned char>& arena = a.tail_pass ? second : first;
+  arena.assign(a.logcap > 0 ? arena_bytes(a.logcap, a.feats != 0) : 1, 0);
   std::unique_ptr<Wave<K, CAP>> gp(new Wave<K, CAP>());
   memset(gp.get(), 0, sizeof(Wave<K, CAP>));
   g_rounds = 0;
@@ -143,7 +149,10 @@ static int run(const KArgs& a) {
 #else
 template <int K, int CAP>
 static int run(const KArgs& a) {
-  std::vector<unsigned char> arena(a.logcap > 0 ? arena_bytes(a.logcap, a.feats != 0) : 1);
+  // (the tail pass of tail_left goes on in the first run's arena)
+  static std::vector<unsigned char> first, second;
+  std::vector<unsigned char>& arena = a.tail_pass ? second : first;
+  arena.assign(a.logcap > 0 ? arena_bytes(a.logcap, a.feats != 0) : 1, 0);
   using W = Wave<K, CAP>;
   std::unique_ptr<W> gp(new W());
   W& g = *gp;
@@ -151,7 +160,7 @@ static int run(const KArgs& a) {
   Leader L;
   memset(&L, 0, sizeof(L));
   L.state = ST_FETCH;
-  L.ab = a.logcap > 0 ? arena.data() : nullptr;
+  L.ab = L.own = a.logcap > 0 ? arena.data() : nullptr;
   g_rounds = 0;
   memset(g_kind, 0, sizeof(g_kind));
   g_scount = 0;
@@ -245,12 +254,15 @@ extern "C" int emu_ccd_batch(const double* tris1, int64_t n1, const double* tris
     }
   };
   emu_tail_handed = 0;
-  if (emu_tail_budget <= 0) return run_shape(a);
+  if (emu_tail_budget <= 0 && emu_tail_left <= 0) return run_shape(a);
   // two runs, as the library's two launches
   std::vector<TailRec> rec((size_t)nq);
   std::vector<int32_t> list((size_t)nq + 1);
   int32_t count = 0;
+  int32_t finished = 0;
   a.tail_budget = emu_tail_budget;
+  a.tail_left = emu_tail_left;
+  a.finished = &finished;
   a.tail_rec = rec.data();
   a.tail_list = list.data();
   a.tail_count = &count;

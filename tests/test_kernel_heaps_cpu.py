@@ -61,3 +61,22 @@ def test_heaps_distance_bit_exact(emu64, rel, abs_, overlap, K):
         seeds = np.stack([rng.integers(0, len(a), 8), rng.integers(0, len(b), 8)], 1)
         ref = D.oracle_batch(a, b, cases, rel, abs_, seeds, overlap_only=bool(overlap))
         D.check_same(ref, D.run_emu(emu64, a, b, cases, rel, abs_, seeds, overlap_only=overlap))
+
+
+@pytest.mark.parametrize("ext,log", [(0, -1), (1, -1), (1, 64), (0, 0)])
+def test_last_query_handed_over(emu64, ext, log):
+    """The last unfinished query goes on in a second run, with the replay log
+    of the first (or without one): same results."""
+    t = mesh("knot")
+    P = W.knot_queries(4, 3, 0.6)
+    kw = dict(tol_d=1e-3, tol_t=1e-4, ext_levels=ext, miss_depth=3, replay_log=log)
+    ref = run_emu(emu64, t, t, P, G.default_params(**kw), 5)
+    emu64.emu_tail_count.restype = C.c_int64
+    emu64.emu_set_tail_left(2)
+    try:
+        got = run_emu(emu64, t, t, P, G.default_params(**kw), 5)
+    finally:
+        emu64.emu_set_tail_left(0)
+    assert emu64.emu_tail_count() == 1
+    for f in ref.dtype.names:
+        assert np.array_equal(ref[f], got[f]), f
