@@ -21,7 +21,7 @@ typedef short bf16x8 __attribute__((ext_vector_type(8)));   // BF16 bit patterns
 typedef __bf16 bf16v8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-struct MlpLds {                 // per-wavefront scratch (20.5 KB)
+struct alignas(16) MlpLds {     // per-wavefront scratch (20.5 KB)
   uint16_t x[64][NF];           // input rows, BF16
   uint16_t h[64][NH];           // first hidden layer after ReLU, BF16
   uint16_t g[64][NH];           // gradient w.r.t. the second hidden layer, BF16
@@ -43,28 +43,17 @@ __device__ inline int crow(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >>
 // the row of accumulator register 8 s + i of this lane (k-slot i of step s)
 __device__ inline int krow(int s, int i, int lane) { return crow(8 * s + i, lane); }
 
+// eight consecutive BF16 values, 16-byte aligned
+__device__ inline bf16x8 ld8(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
+
 __device__ inline bf16x8 a_frag(const uint16_t* base, int ld, int lane, int kofs) {
   // A[m = lane % 32][k = kofs + 8 (lane / 32) + i] from a row-major BF16 tile
-  const uint16_t* p = base + (lane & 31) * ld + kofs + 8 * (lane >> 5);
-  bf16x8 v;
-  for (int i = 0; i < 8; i++) v[i] = (short)p[i];
-  return v;
-}
-
-__device__ inline bf16x8 b_frag(const uint16_t* w, int ld, int lane, int kofs, int nofs) {
-  // B[k = kofs + 8 (lane / 32) + i][n = nofs + lane % 32] from a row-major BF16 matrix
-  const uint16_t* p = w + (kofs + 8 * (lane >> 5)) * ld + nofs + (lane & 31);
-  bf16x8 v;
-  for (int i = 0; i < 8; i++) v[i] = (short)p[i * ld];
-  return v;
+  return ld8(base + (lane & 31) * ld + kofs + 8 * (lane >> 5));
 }
 
 __device__ inline bf16x8 bt_frag(const uint16_t* w, int ld, int lane, int kofs, int nofs) {
   // B[k][n] = W[n][k] (transposed): W row-major with leading dimension ld
-  const uint16_t* p = w + (nofs + (lane & 31)) * ld + kofs + 8 * (lane >> 5);
-  bf16x8 v;
-  for (int i = 0; i < 8; i++) v[i] = (short)p[i];
-  return v;
+  return ld8(w + (nofs + (lane & 31)) * ld + kofs + 8 * (lane >> 5));
 }
 
 __device__ inline f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
@@ -87,7 +76,7 @@ __device__ inline void mlp_forward64(const ScorerDev& S, MlpLds& m, int lane, f3
       f32x16 acc = {0};
       for (int ks = 0; ks < NF / 16; ks++)
         acc = mfma(a_frag(&m.x[32 * rt][0], NF, lane, 16 * ks),
-                   b_frag(S.w1, NH, lane, 16 * ks, 32 * ct), acc);
+                   bt_frag(S.w1t, NF, lane, 16 * ks, 32 * ct), acc);
       const int col = 32 * ct + (lane & 31);
       const float bias = S.b1[col];
       wave_lds_sync();
@@ -102,7 +91,7 @@ __device__ inline void mlp_forward64(const ScorerDev& S, MlpLds& m, int lane, f3
       f32x16 acc = {0};
       for (int ks = 0; ks < NH / 16; ks++)
         acc = mfma(a_frag(&m.h[32 * rt][0], NH, lane, 16 * ks),
-                   b_frag(S.w2, NH, lane, 16 * ks, 32 * ct), acc);
+                   bt_frag(S.w2t, NH, lane, 16 * ks, 32 * ct), acc);
       const float bias = S.b2[32 * ct + (lane & 31)];
       for (int r = 0; r < 16; r++) {
         const float v = acc[r] + bias;

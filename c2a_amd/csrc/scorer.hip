@@ -35,45 +35,47 @@ __global__ void __launch_bounds__(64) infer_kernel(ScorerDev S, const float* X, 
   }
 }
 
-// Scores of n feature rows through the training forward pass (FP32 in, one
-// wavefront per 64 rows).
-__global__ void __launch_bounds__(64) score_rows_kernel(ScorerDev S, const float* X, int64_t n,
-                                                        float* out) {
-  __shared__ MlpLds m;
-  const int lane = threadIdx.x;
-  for (int64_t base = (int64_t)blockIdx.x * 64; base < n; base += (int64_t)gridDim.x * 64) {
-    const int64_t row = base + lane;
-    for (int k = 0; k < NF; k++) m.x[lane][k] = f32_to_bf16(row < n ? X[row * NF + k] : 0.0f);
-    wave_lds_sync();
-    f32x16 h2[2][2];
-    mlp_forward64(S, m, lane, h2);
-    if (row < n) out[row] = m.s[lane];
-    wave_lds_sync();
-  }
+// Rows per workgroup of the gradient: one 64-row tile each (a batch of 2048
+// rows fills 32 workgroups; with four tiles one after another in each of
+// eight, the kernel took 83 us on MI355X), more once 512 workgroups are full.
+int grad_rows(int64_t n) {
+  const int64_t tiles = (n + 63) / 64;
+  return (int)(64 * ((tiles + 511) / 512));
 }
 
 // Partial gradients of rows [blockIdx.x * per_block, ...) written to
-// partial[blockIdx.x * (NPARAM + 1) ...] (the last entry is the squared error).
-__global__ void __launch_bounds__(64) grad_kernel(ScorerDev S, const float* X, const float* Y,
-                                                  const int32_t* idx, int64_t n, int per_block,
-                                                  float scale, float* partial) {
+// partial[blockIdx.x * (NPARAM + 1) ...] (the last entry is the squared
+// error).  b3 is read here, not by the host: it changes every step.
+__global__ void __launch_bounds__(64) grad_kernel(ScorerDev S, const float* b3, const float* X,
+                                                  const float* Y, const int32_t* idx, int64_t n,
+                                                  int per_block, float scale, float* partial) {
   __shared__ MlpLds m;
   const int lane = threadIdx.x;
   MlpGrad G;
   grad_zero(G);
-  const int64_t b0 = (int64_t)blockIdx.x * per_block;
-  const int64_t b1 = b0 + per_block < n ? b0 + per_block : n;
-  for (int64_t base = b0; base < b1; base += 64) {
+  S.b3 = *b3;
+  const int64_t r0 = (int64_t)blockIdx.x * per_block;
+  const int64_t r1 = r0 + per_block < n ? r0 + per_block : n;
+  for (int64_t base = r0; base < r1; base += 64) {
     const int64_t row = base + lane;
-    const bool v = row < b1;
+    const bool v = row < r1;
     const int64_t src = v ? (idx ? (int64_t)idx[row] : row) : 0;
-    for (int k = 0; k < NF; k++) m.x[lane][k] = f32_to_bf16(v ? X[src * NF + k] : 0.0f);
+    const float4* xr = reinterpret_cast<const float4*>(X + src * NF);
+    const float y = v ? Y[src] : 0.0f;
+    float4 f[NF / 4];
+    for (int k = 0; k < NF / 4; k++) f[k] = xr[k];
+    for (int k = 0; k < NF / 8; k++) {
+      bf16x8 q;
+      for (int i = 0; i < 8; i++)
+        q[i] = (short)f32_to_bf16(v ? (i < 4 ? (&f[2 * k].x)[i] : (&f[2 * k + 1].x)[i - 4]) : 0.0f);
+      *reinterpret_cast<bf16x8*>(&m.x[lane][8 * k]) = q;
+    }
     wave_lds_sync();
     f32x16 h2[2][2];
     mlp_forward64(S, m, lane, h2);
-    m.dy[lane] = v ? Y[src] : 0.0f;
+    m.dy[lane] = y;
     wave_lds_sync();
-    mlp_backward64(S, m, lane, h2, (int)(b1 - base), scale, G);
+    mlp_backward64(S, m, lane, h2, r1 - base < 64 ? (int)(r1 - base) : 64, scale, G);
   }
   float* o = partial + (int64_t)blockIdx.x * (NPARAM + 1);
   for (int nt = 0; nt < 2; nt++)
@@ -110,13 +112,22 @@ __global__ void reduce_kernel(const float* partial, int nblocks, float* grad) {
   grad[i] = s;
 }
 
-// Adam step on the FP32 master parameters; refreshes the BF16 weights.
-__global__ void adam_kernel(float* p, float* mom, float* vel, const float* grad, float lr,
-                            float b1, float b2, float eps, int step, uint16_t* w1,
-                            uint16_t* w2, uint16_t* w1t, uint16_t* w2t) {
+// The sum of the partials in block order and the Adam step on the FP32
+// master parameters in one launch; refreshes the BF16 weights.  The batch's
+// squared error goes to *loss.
+__global__ void __launch_bounds__(64) adam_kernel(float* p, float* mom, float* vel,
+                                                  const float* partial, int nblocks, float* loss,
+                                                  float lr, float b1, float b2, float eps, int step,
+                                                  uint16_t* w1, uint16_t* w2, uint16_t* w1t,
+                                                  uint16_t* w2t) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= NPARAM) return;
-  const float g = grad[i];
+  if (i > NPARAM) return;
+  float g = 0.0f;
+  for (int b = 0; b < nblocks; b++) g += partial[(int64_t)b * (NPARAM + 1) + i];
+  if (i == NPARAM) {
+    *loss = g;
+    return;
+  }
   const float mi = b1 * mom[i] + (1.0f - b1) * g;
   const float vi = b2 * vel[i] + (1.0f - b2) * g * g;
   mom[i] = mi;
@@ -350,8 +361,7 @@ int c2a_scorer_infer(const c2a_scorer* s, const float* feats, int64_t n, float* 
 int c2a_scorer_grad(const c2a_scorer* s, const float* feats, const float* labels, int64_t n,
                     float* grad_out, float* loss_out) {
   if (!s || n <= 0 || !feats || !labels || !grad_out) return bad_arg("bad scorer arguments");
-  const int per_block = 256;
-  const int nb = (int)((n + per_block - 1) / per_block);
+  const int rows = grad_rows(n), nb = (int)((n + rows - 1) / rows);
   DevArray<float> dx, dy, part, g;
   if (!dx.alloc((size_t)n * NF) || !dy.alloc((size_t)n) ||
       !part.alloc((size_t)nb * (NPARAM + 1)) || !g.alloc(NPARAM + 1))
@@ -359,9 +369,8 @@ int c2a_scorer_grad(const c2a_scorer* s, const float* feats, const float* labels
   hipError_t e = hipMemcpy(dx.p, feats, n * NF * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dy.p, labels, n * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(grad_kernel, dim3(nb), dim3(64), 0, 0, dev_view(s, read_b3(s)), dx.p,
-                       dy.p, (const int32_t*)nullptr, n, per_block, (float)(2.0 / (double)n),
-                       part.p);
+    hipLaunchKernelGGL(grad_kernel, dim3(nb), dim3(64), 0, 0, dev_view(s, 0.0f), s->p + P_B3,
+                       dx.p, dy.p, (const int32_t*)nullptr, n, rows, (float)(2.0 / (double)n), part.p);
     hipLaunchKernelGGL(reduce_kernel, dim3((NPARAM + 256) / 256), dim3(256), 0, 0, part.p, nb,
                        g.p);
     e = hipGetLastError();
@@ -380,20 +389,23 @@ int c2a_scorer_train(c2a_scorer* s, const float* feats, const float* labels, int
                      int32_t epochs, int32_t batch, float lr, uint64_t seed, float* loss_out) {
   if (!s || n <= 0 || !feats || !labels || epochs <= 0 || batch <= 0)
     return bad_arg("bad scorer training arguments");
-  const int per_block = 256;
-  const int nbmax = (batch + per_block - 1) / per_block;
-  DevArray<float> dx_, dy_, part_, g_;
+  const int rows = grad_rows(batch);
+  const int nbmax = (int)(((int64_t)batch + rows - 1) / rows);
+  const int64_t steps = (n + batch - 1) / batch;   // per epoch
+  DevArray<float> dx_, dy_, part_, loss_;
   DevArray<int32_t> didx_;
   if (!dx_.alloc((size_t)n * NF) || !dy_.alloc((size_t)n) || !didx_.alloc((size_t)n) ||
-      !part_.alloc((size_t)nbmax * (NPARAM + 1)) || !g_.alloc(NPARAM + 1))
+      !part_.alloc((size_t)nbmax * (NPARAM + 1)) || !loss_.alloc((size_t)steps))
     return oom("scorer training buffers");
-  float *dx = dx_.p, *dy = dy_.p, *part = part_.p, *g = g_.p;
+  float *dx = dx_.p, *dy = dy_.p, *part = part_.p;
   int32_t* didx = didx_.p;
   hipError_t e = hipMemcpy(dx, feats, n * NF * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dy, labels, n * sizeof(float), hipMemcpyHostToDevice);
   std::vector<int32_t> perm((size_t)n);
+  std::vector<float> lh((size_t)steps);
   uint64_t st = mix(seed ^ 0xA11CEull);
-  std::vector<float> gh(NPARAM + 1);
+  // Two launches per step and no host synchronisation inside an epoch (the
+  // output bias is read on the device, the squared errors at the epoch's end).
   for (int ep = 0; ep < epochs && e == hipSuccess; ep++) {
     for (int64_t i = 0; i < n; i++) perm[(size_t)i] = (int32_t)i;
     for (int64_t i = n - 1; i > 0; i--) {   // seeded Fisher-Yates shuffle
@@ -404,21 +416,22 @@ int c2a_scorer_train(c2a_scorer* s, const float* feats, const float* labels, int
       perm[(size_t)j] = t;
     }
     e = hipMemcpy(didx, perm.data(), n * sizeof(int32_t), hipMemcpyHostToDevice);
-    double eloss = 0.0;
-    for (int64_t b0 = 0; b0 < n && e == hipSuccess; b0 += batch) {
+    for (int64_t b = 0; b < steps && e == hipSuccess; b++) {
+      const int64_t b0 = b * batch;
       const int64_t nb_rows = b0 + batch < n ? batch : n - b0;
-      const int nb = (int)((nb_rows + per_block - 1) / per_block);
-      hipLaunchKernelGGL(grad_kernel, dim3(nb), dim3(64), 0, 0, dev_view(s, read_b3(s)), dx, dy,
-                         didx + b0, nb_rows, per_block, (float)(2.0 / (double)nb_rows), part);
-      hipLaunchKernelGGL(reduce_kernel, dim3((NPARAM + 256) / 256), dim3(256), 0, 0, part, nb, g);
+      const int nb = (int)((nb_rows + rows - 1) / rows);
+      hipLaunchKernelGGL(grad_kernel, dim3(nb), dim3(64), 0, 0, dev_view(s, 0.0f), s->p + P_B3, dx,
+                         dy, didx + b0, nb_rows, rows, (float)(2.0 / (double)nb_rows), part);
       s->step++;
-      hipLaunchKernelGGL(adam_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, 0, s->p, s->mom,
-                         s->vel, g, lr, 0.9f, 0.999f, 1e-8f, s->step, s->w1, s->w2, s->w1t, s->w2t);
+      hipLaunchKernelGGL(adam_kernel, dim3((NPARAM + 64) / 64), dim3(64), 0, 0, s->p, s->mom,
+                         s->vel, part, nb, loss_.p + b, lr, 0.9f, 0.999f, 1e-8f, s->step, s->w1,
+                         s->w2, s->w1t, s->w2t);
       e = hipGetLastError();
-      float l = 0.0f;
-      if (e == hipSuccess) e = hipMemcpy(&l, g + NPARAM, sizeof(float), hipMemcpyDeviceToHost);
-      eloss += l;
     }
+    if (e == hipSuccess)
+      e = hipMemcpy(lh.data(), loss_.p, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost);
+    double eloss = 0.0;
+    for (float l : lh) eloss += l;
     if (loss_out) loss_out[ep] = (float)(eloss / (double)n);
   }
   return hip_err(e);
