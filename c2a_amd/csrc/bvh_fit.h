@@ -192,14 +192,6 @@ C2A_HD void corner_grow(double px, double py, double pz, double cz, double radsq
   }
 }
 
-// A point can ever grow a corner only if it lies outside the rectangle in
-// both in-plane directions at the start of the corner pass (the rectangle
-// only grows, so the tests only get harder).
-C2A_HD bool corner_candidate(double px, double py, double minx, double maxx, double miny,
-                             double maxy) {
-  return (px > maxx || px < minx) && (py > maxy || py < miny);
-}
-
 // Rectangle corner, sides and radius of the fit (C2A_BV.cpp:608-635).
 C2A_HD void fit_finish(const double* R, double minx, double maxx, double miny, double maxy,
                        double cz, double r, double* Tr, double* l, double* rad) {

@@ -3,17 +3,22 @@
 // (C2A_Build.cpp:393-574, C2A_BV.cpp:71-111 and 354-635).
 //
 // Level by level, every node of a level at once, in three sizes: a
-// 256-thread workgroup per node above kWaveMax triangles, one wavefront per
-// node down to kThreadMax, one thread per node below.  A workgroup (or
-// wavefront) stages the node's per-triangle covariance terms through LDS and
-// nine lanes add them to the nine sums in triangle order (sums are
-// order-dependent: one dependent add per triangle and sum is the only
-// sequential part); every minimum, maximum and arg-extreme of the fit is
-// reduced across the lanes (exact in any order); the corner pass evaluates 64
-// points at a time against the current rectangle and advances to the first
-// one that grows it; and the in-place partition of the split is reproduced in
-// parallel from prefix counts (see the split below).  A one-thread node runs
-// the host's sequential code.
+// 1024-thread workgroup per node above kWaveMax triangles, one wavefront per
+// node down to kThreadMax, one thread per node below.  A workgroup stages the
+// node's per-triangle covariance terms through LDS and nine lanes add them to
+// the nine sums in triangle order (sums are order-dependent: one dependent add
+// per triangle and sum is the only sequential part) while other wavefronts
+// form the next terms; every minimum, maximum and arg-extreme of the fit is
+// reduced across the lanes (exact in any order); the corner pass evaluates
+// four points per thread at once against the current rectangle and goes on
+// behind the first one that grows it; and the in-place partition of the split
+// is reproduced in parallel from prefix counts (see the split below).  A
+// one-thread node runs the host's sequential code.
+//
+// What bounds it: the large nodes' latency, one workgroup each (the root of
+// 262,144 triangles first).  MI355X, the workgroup nodes of a build and a refit
+// at that size: 15 ms; with 256 threads, a point per turn and a sequential
+// corner pass over compacted candidates, 56 ms.
 // Node numbers follow the host's depth-first order through dfs_first_child.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -30,7 +35,8 @@ namespace c2a {
 
 namespace {
 
-constexpr int kWaveMax = 2048;   // nodes above this many triangles: 256 threads
+constexpr int kWaveMax = 2048;   // nodes above this many triangles: a workgroup
+constexpr int kGroup = 1024;     // its threads
 constexpr int kThreadMax = 24;   // nodes at most this large: one thread
 
 // node classes: 0 workgroup, 1 wavefront, 2 thread
@@ -47,7 +53,6 @@ struct BuildArgs {
   int32_t* perm;           // position -> caller triangle
   int32_t* perm_tmp;       // the split's output arrangement
   int32_t* tape;           // 2n: the partition's queue tape
-  int32_t* cand;           // 3n: corner candidates
   GpuNode* nodes;          // 2n - 1, zeroed
   const BuildJob* jobs[3];  // this level's nodes of each class
   BuildJob* next[3];        // the next level's nodes of each class
@@ -152,9 +157,35 @@ __device__ int block_scan(int v, int* sh, int& total) {
 
 // ---- one large node per workgroup -----------------------------------------
 
+// Sum k of the m staged terms, in triangle order, onto sk: sixteen terms are
+// read ahead of the dependent adds.
+__device__ inline double add_terms(const double* chunk, int m, int k, double sk) {
+  double t[16];
+  int j = 0;
+  if (m >= 16) {
+#pragma unroll
+    for (int u = 0; u < 16; u++) t[u] = chunk[9 * u + k];
+    for (; j + 32 <= m; j += 16) {
+      double n[16];
+#pragma unroll
+      for (int u = 0; u < 16; u++) n[u] = chunk[9 * (j + 16 + u) + k];
+#pragma unroll
+      for (int u = 0; u < 16; u++) sk += t[u];
+#pragma unroll
+      for (int u = 0; u < 16; u++) t[u] = n[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; u++) sk += t[u];
+    j += 16;
+  }
+  for (; j < m; j++) sk += chunk[9 * j + k];
+  return sk;
+}
+
 template <int B>
 __global__ void __launch_bounds__(B) build_node(BuildArgs a, int cls) {
-  __shared__ double chunk[B * 9];
+  constexpr int CH = B < 256 ? B : 256;   // triangles staged at a time
+  __shared__ double chunk[2][CH * 9];
   __shared__ double shv[B / 64];
   __shared__ int shi[B / 64];
   __shared__ int shs[B / 64];
@@ -165,29 +196,21 @@ __global__ void __launch_bounds__(B) build_node(BuildArgs a, int cls) {
   const int32_t first = job.first, num = job.num;
   const int np = 3 * num;
 
-  // covariance sums, in triangle order (C2A_Build.cpp:279-335): every
-  // thread computes its triangle's nine terms into LDS, then lane k < 9 adds
-  // term k of each triangle, in order, to sum k (one dependent add per
-  // triangle and sum)
+  // covariance sums, in triangle order (C2A_Build.cpp:279-335): the threads
+  // behind wavefront 0 (of a one-wavefront node: its own) compute the next
+  // triangles' nine terms into LDS while lane k < 9 of wavefront 0 adds term k
+  // of each staged triangle, in order, to sum k
+  constexpr int P0 = B > 64 ? 64 : 0;   // first producing thread
+  const int nch = (num + CH - 1) / CH;
   double run = 0.0;
-  for (int base = 0; base < num; base += B) {
-    const int i = base + tid;
-    if (i < num) cov_terms(tri_at(a, first + i), chunk + 9 * tid);
-    __syncthreads();
-    if (tid < 9) {
-      const int m = num - base < B ? num - base : B;
-      double sk = run;
-      int j = 0;
-      for (; j + 8 <= m; j += 8) {
-        double t[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) t[u] = chunk[9 * (j + u) + tid];
-#pragma unroll
-        for (int u = 0; u < 8; u++) sk += t[u];
-      }
-      for (; j < m; j++) sk += chunk[9 * j + tid];
-      run = sk;
-    }
+  for (int c = 0; c <= nch; c++) {
+    const int i = c * CH + tid - P0;
+    if (c < nch && tid >= P0 && tid - P0 < CH && i < num)
+      cov_terms(tri_at(a, first + i), chunk[c & 1] + 9 * (tid - P0));
+    if (B == 64) __syncthreads();
+    const int d = B == 64 ? c : c - 1;   // the chunk to add
+    if (tid < 9 && d >= 0 && d < nch)
+      run = add_terms(chunk[d & 1], num - d * CH < CH ? num - d * CH : CH, tid, run);
     __syncthreads();
   }
   if (tid < 9) acc[tid] = run;
@@ -204,22 +227,28 @@ __global__ void __launch_bounds__(B) build_node(BuildArgs a, int cls) {
   double Rr[9];
   for (int k = 0; k < 9; k++) Rr[k] = R[k];
 
-  // angular radius, slab (z) extent, then the in-plane arg-extremes
+  // angular radius, slab (z) extent, then the in-plane arg-extremes; a
+  // triangle per thread and turn
   double amax = 0.0, zmin = INFINITY, zmax = -INFINITY;
   double xmn = INFINITY, xmx = -INFINITY, ymn = INFINITY, ymx = -INFINITY;
   int ixmn = 0x7fffffff, ixmx = 0x7fffffff, iymn = 0x7fffffff, iymx = 0x7fffffff;
-  for (int i = tid; i < np; i += B) {
-    const double* v = tri_at(a, first + i / 3) + 3 * (i % 3);
-    const double d = vertex_radius(v);
-    amax = d > amax ? d : amax;
-    double P[3];
-    mtxv(P, Rr, v);
-    zmin = P[2] < zmin ? P[2] : zmin;
-    zmax = P[2] > zmax ? P[2] : zmax;
-    if (P[0] < xmn) { xmn = P[0]; ixmn = i; }
-    if (P[0] > xmx) { xmx = P[0]; ixmx = i; }
-    if (P[1] < ymn) { ymn = P[1]; iymn = i; }
-    if (P[1] > ymx) { ymx = P[1]; iymx = i; }
+  for (int t = tid; t < num; t += B) {
+    const double* tv = tri_at(a, first + t);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const double* v = tv + 3 * k;
+      const int i = 3 * t + k;
+      const double d = vertex_radius(v);
+      amax = d > amax ? d : amax;
+      double P[3];
+      mtxv(P, Rr, v);
+      zmin = P[2] < zmin ? P[2] : zmin;
+      zmax = P[2] > zmax ? P[2] : zmax;
+      if (P[0] < xmn) { xmn = P[0]; ixmn = i; }
+      if (P[0] > xmx) { xmx = P[0]; ixmx = i; }
+      if (P[1] < ymn) { ymn = P[1]; iymn = i; }
+      if (P[1] > ymx) { ymx = P[1]; iymx = i; }
+    }
   }
   const double angR = block_max<B>(amax, shv);
   const double minz = block_min<B>(zmin, shv);
@@ -241,70 +270,83 @@ __global__ void __launch_bounds__(B) build_node(BuildArgs a, int cls) {
   proj(a, Rr, first, iymx, P);
   const double hiy0 = extent_hi(P[1], P[2], cz, radsqr);
   double lox = lox0, hix = hix0, loy = loy0, hiy = hiy0;
-  for (int i = tid; i < np; i += B) {
-    proj(a, Rr, first, i, P);
-    if (P[0] < lox0) { const double x = extent_lo(P[0], P[2], cz, radsqr); lox = x < lox ? x : lox; }
-    if (P[0] > hix0) { const double x = extent_hi(P[0], P[2], cz, radsqr); hix = x > hix ? x : hix; }
-    if (P[1] < loy0) { const double x = extent_lo(P[1], P[2], cz, radsqr); loy = x < loy ? x : loy; }
-    if (P[1] > hiy0) { const double x = extent_hi(P[1], P[2], cz, radsqr); hiy = x > hiy ? x : hiy; }
+  for (int t = tid; t < num; t += B) {
+    const double* tv = tri_at(a, first + t);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      mtxv(P, Rr, tv + 3 * k);
+      if (P[0] < lox0) { const double x = extent_lo(P[0], P[2], cz, radsqr); lox = x < lox ? x : lox; }
+      if (P[0] > hix0) { const double x = extent_hi(P[0], P[2], cz, radsqr); hix = x > hix ? x : hix; }
+      if (P[1] < loy0) { const double x = extent_lo(P[1], P[2], cz, radsqr); loy = x < loy ? x : loy; }
+      if (P[1] > hiy0) { const double x = extent_hi(P[1], P[2], cz, radsqr); hiy = x > hiy ? x : hiy; }
+    }
   }
   double minx = block_min<B>(lox, shv), maxx = block_max<B>(hix, shv);
   double miny = block_min<B>(loy, shv), maxy = block_max<B>(hiy, shv);
 
-  // corner pass: the candidates in point order, then one lane in sequence
-  int ncand = 0;
-  int32_t* cand = a.cand + 3 * (int64_t)first;
-  for (int base = 0; base < np; base += B) {
-    const int i = base + tid;
-    int f = 0;
-    if (i < np) {
-      proj(a, Rr, first, i, P);
-      f = corner_candidate(P[0], P[1], minx, maxx, miny, maxy) ? 1 : 0;
+  // Corner pass.  The host grows the rectangle point by point
+  // (C2A_BV.cpp:542-606); a point changes it only when it lies outside the
+  // current rounded corner.  Every thread evaluates its four points of the
+  // next 4 B (point base + q B + tid) against the current rectangle: the points
+  // before the first one that changes it are no-ops in sequence too, that one's
+  // result is the next rectangle, and the points behind it are evaluated again.
+  constexpr int NQ = 4;
+  for (int base = 0; base < np; base += NQ * B) {
+    double Q[NQ][3];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const int i = base + q * B + tid;
+      proj(a, Rr, first, i < np ? i : np - 1, Q[q]);
     }
-    int tot;
-    const int at = block_scan<B>(f, shs, tot);
-    if (f) cand[ncand + at] = i;
-    ncand += tot;
-  }
-  // The host grows the rectangle point by point (C2A_BV.cpp:542-606); a
-  // point changes it only when it lies outside the current rounded corner.
-  // Wavefront 0 evaluates 64 candidates at once against the current
-  // rectangle: the points before the first one that changes it are no-ops
-  // in sequence too, and that one's result is the next rectangle.  Each
-  // chunk's projected points are staged in LDS by the whole workgroup.
-  __syncthreads();
-  double* cp = chunk;
-  for (int base = 0; base < ncand; base += B) {
-    const int m = ncand - base < B ? ncand - base : B;
-    if (tid < m) proj(a, Rr, first, cand[base + tid], cp + 3 * tid);
-    __syncthreads();
-    if (tid < 64) {
-      int pos = 0;
-      while (pos < m) {
-        const int j = pos + tid;
+    int from = base;
+    for (;;) {
+      int hit = 0x7fffffff;
+      double g0 = 0.0, g1 = 0.0, g2 = 0.0, g3 = 0.0;
+#pragma unroll
+      for (int q = NQ - 1; q >= 0; q--) {
+        const int i = base + q * B + tid;
         double x0 = minx, x1 = maxx, y0 = miny, y1 = maxy;
-        bool changed = false;
-        if (j < m) {
-          corner_grow(cp[3 * j], cp[3 * j + 1], cp[3 * j + 2], cz, radsqr, x0, x1, y0, y1);
-          changed = __double_as_longlong(x0) != __double_as_longlong(minx) ||
-                    __double_as_longlong(x1) != __double_as_longlong(maxx) ||
-                    __double_as_longlong(y0) != __double_as_longlong(miny) ||
-                    __double_as_longlong(y1) != __double_as_longlong(maxy);
+        corner_grow(Q[q][0], Q[q][1], Q[q][2], cz, radsqr, x0, x1, y0, y1);
+        const bool changed = __double_as_longlong(x0) != __double_as_longlong(minx) ||
+                             __double_as_longlong(x1) != __double_as_longlong(maxx) ||
+                             __double_as_longlong(y0) != __double_as_longlong(miny) ||
+                             __double_as_longlong(y1) != __double_as_longlong(maxy);
+        if (changed && i >= from && i < np) {
+          hit = i;
+          g0 = x0;
+          g1 = x1;
+          g2 = y0;
+          g3 = y1;
         }
-        const unsigned long long hit = __ballot(changed);
-        if (hit == 0) {
-          pos += 64;
-          continue;
-        }
-        const int f = __ffsll(hit) - 1;
-        minx = __shfl(x0, f);
-        maxx = __shfl(x1, f);
-        miny = __shfl(y0, f);
-        maxy = __shfl(y1, f);
-        pos += f + 1;
       }
+      int f = hit;
+      for (int o = 32; o > 0; o >>= 1) {
+        const int w = __shfl_xor(f, o);
+        f = w < f ? w : f;
+      }
+      if (B > 64) {
+        if ((tid & 63) == 0) shi[tid >> 6] = f;
+        __syncthreads();
+        for (int k = 0; k < B / 64; k++) f = shi[k] < f ? shi[k] : f;
+      }
+      if (f == 0x7fffffff) {
+        if (B > 64) __syncthreads();   // shi is read before it is written again
+        break;
+      }
+      if (hit == f) {
+        box[0] = g0;
+        box[1] = g1;
+        box[2] = g2;
+        box[3] = g3;
+      }
+      __syncthreads();
+      minx = box[0];
+      maxx = box[1];
+      miny = box[2];
+      maxy = box[3];
+      from = f + 1;
+      __syncthreads();
     }
-    __syncthreads();
   }
   if (tid == 0) {
     GpuNode& nd = a.nodes[job.bn];
@@ -563,18 +605,17 @@ inline unsigned grid_of(int64_t n, int b) { return (unsigned)((n + b - 1) / b); 
 
 hipError_t build_bvh_device(const double* xyz9, const int32_t* ids, const int32_t* vidx3,
                             int64_t n, Bvh* out, void** nodes_dev, void** tris_dev,
-                            hipStream_t s) {
+                            hipStream_t s, const std::function<void()>& before_out) {
   *nodes_dev = nullptr;
   *tris_dev = nullptr;
   const int64_t nn = 2 * n - 1;
-  Dev src, dids, dvidx, perm, perm_tmp, tape, cand, counts, mRT, parent, tris, ids_out, vidx_out;
+  Dev src, dids, dvidx, perm, perm_tmp, tape, counts, mRT, parent, tris, ids_out, vidx_out;
   Dev lists[2][3];   // ping-pong job lists of the three node classes
   GpuNode* nodes = nullptr;
   BVH_TRY(src.alloc((size_t)n * 9 * sizeof(double)));
   BVH_TRY(perm.alloc((size_t)n * 4));
   BVH_TRY(perm_tmp.alloc((size_t)n * 4));
   BVH_TRY(tape.alloc((size_t)n * 8));
-  BVH_TRY(cand.alloc((size_t)n * 12));
   for (int l = 0; l < 2; l++)
     for (int c = 0; c < 3; c++) BVH_TRY(lists[l][c].alloc((size_t)n * sizeof(BuildJob)));
   BVH_TRY(counts.alloc(4 * sizeof(int32_t)));
@@ -601,7 +642,6 @@ hipError_t build_bvh_device(const double* xyz9, const int32_t* ids, const int32_
   a.perm = (int32_t*)perm.p;
   a.perm_tmp = (int32_t*)perm_tmp.p;
   a.tape = (int32_t*)tape.p;
-  a.cand = (int32_t*)cand.p;
   a.nodes = nodes;
   a.counts = (int32_t*)counts.p;
   const BuildJob root{0, 0, (int32_t)n, 0, 0, {0, 0, 0}};
@@ -619,7 +659,7 @@ hipError_t build_bvh_device(const double* xyz9, const int32_t* ids, const int32_
     }
     BVH_TRY(hipMemsetAsync(a.counts, 0, 3 * sizeof(int32_t), s));
     if (cnt[0] > 0)
-      hipLaunchKernelGGL(build_node<256>, dim3((unsigned)cnt[0]), dim3(256), 0, s, a, 0);
+      hipLaunchKernelGGL(build_node<kGroup>, dim3((unsigned)cnt[0]), dim3(kGroup), 0, s, a, 0);
     if (cnt[1] > 0)
       hipLaunchKernelGGL(build_node<64>, dim3((unsigned)cnt[1]), dim3(64), 0, s, a, 1);
     if (cnt[2] > 0)
@@ -645,6 +685,7 @@ hipError_t build_bvh_device(const double* xyz9, const int32_t* ids, const int32_
                      (const int32_t*)dids.p, (const int32_t*)dvidx.p, a.perm, n,
                      (double*)tris.p, (int32_t*)ids_out.p, (int32_t*)vidx_out.p);
   BVH_TRY(hipGetLastError());
+  before_out();
   out->nodes.resize((size_t)nn);
   out->tris.resize((size_t)n * 9);
   out->tri_id.resize((size_t)n);
@@ -669,8 +710,8 @@ hipError_t build_bvh_device(const double* xyz9, const int32_t* ids, const int32_
   return hipSuccess;
 }
 
-// Refit on the device: the tree is known, so each depth's nodes go in one
-// launch per size class (no host round trip between levels), then the
+// Refit on the device: the tree is known and a node's fit depends on its
+// triangles alone, so all nodes of a size class go in one launch, then the
 // parent-relative frames and the triangles in build order.  Copies the
 // result back into *b.
 hipError_t refit_bvh_device(const double* xyz9, Bvh* b, void* nodes_dev, void* tris_dev,
@@ -681,39 +722,27 @@ hipError_t refit_bvh_device(const double* xyz9, Bvh* b, void* nodes_dev, void* t
     return hipErrorInvalidValue;
   std::vector<int32_t> first, num, depth;
   node_ranges(b->nodes, first, num, depth);
-  // level by level: a node's corner candidates live in its triangle range of
-  // a.cand, which its descendants' ranges overlap, so only nodes of one
-  // depth (disjoint ranges) may run together
-  int max_depth = 0;
-  for (int64_t v = 0; v < nn; v++) max_depth = std::max(max_depth, (int)depth[(size_t)v]);
+  // the nodes of each class, larger ones first (nodes near the root come first
+  // in the numbering); no node's fit depends on another's
   std::vector<BuildJob> jobs[3];
-  // jobs of each class ordered by depth, with per-depth offsets
-  std::vector<std::vector<int32_t>> cnt(3, std::vector<int32_t>((size_t)max_depth + 1, 0));
-  for (int64_t v = 0; v < nn; v++) cnt[node_class(num[(size_t)v])][(size_t)depth[(size_t)v]]++;
-  std::vector<std::vector<int32_t>> off(3, std::vector<int32_t>((size_t)max_depth + 2, 0));
-  for (int c = 0; c < 3; c++) {
-    for (int d = 0; d <= max_depth; d++) off[c][(size_t)d + 1] = off[c][(size_t)d] + cnt[c][(size_t)d];
-    jobs[c].resize((size_t)off[c][(size_t)max_depth + 1]);
-  }
-  {
-    std::vector<std::vector<int32_t>> fill = off;
-    for (int64_t v = 0; v < nn; v++) {
-      const int c = node_class(num[(size_t)v]);
-      jobs[c][(size_t)fill[c][(size_t)depth[(size_t)v]]++] =
-          BuildJob{(int32_t)v, first[(size_t)v], num[(size_t)v], depth[(size_t)v], 0, {0, 0, 0}};
-    }
-  }
-  Dev src, perm, cand, mRT, parent, lists[3];
+  size_t cnt[3] = {0, 0, 0};
+  for (int64_t v = 0; v < nn; v++) cnt[node_class(num[(size_t)v])]++;
+  for (int c = 0; c < 3; c++) jobs[c].reserve(cnt[c]);
+  for (int64_t v = 0; v < nn; v++)
+    jobs[node_class(num[(size_t)v])].push_back(
+        BuildJob{(int32_t)v, first[(size_t)v], num[(size_t)v], depth[(size_t)v], 0, {0, 0, 0}});
+  for (int c = 0; c < 2; c++)
+    std::stable_sort(jobs[c].begin(), jobs[c].end(),
+                     [](const BuildJob& x, const BuildJob& y) { return x.num > y.num; });
+  Dev src, perm, mRT, parent, lists[3];
   BVH_TRY(src.alloc((size_t)n * 9 * sizeof(double)));
   BVH_TRY(perm.alloc((size_t)n * 4));
-  BVH_TRY(cand.alloc((size_t)n * 12));
   BVH_TRY(hipMemcpyAsync(src.p, xyz9, (size_t)n * 9 * sizeof(double), hipMemcpyHostToDevice, s));
   BVH_TRY(hipMemcpyAsync(perm.p, b->src_index.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
   BuildArgs a;
   memset(&a, 0, sizeof(a));
   a.src = (const double*)src.p;
   a.perm = (int32_t*)perm.p;
-  a.cand = (int32_t*)cand.p;
   a.nodes = (GpuNode*)nodes_dev;
   a.refit = 1;
   for (int c = 0; c < 3; c++) {
@@ -722,16 +751,14 @@ hipError_t refit_bvh_device(const double* xyz9, Bvh* b, void* nodes_dev, void* t
     BVH_TRY(hipMemcpyAsync(lists[c].p, jobs[c].data(), jobs[c].size() * sizeof(BuildJob),
                            hipMemcpyHostToDevice, s));
   }
-  for (int d = 0; d <= max_depth; d++) {
-    for (int c = 0; c < 3; c++)
-      a.jobs[c] = (const BuildJob*)lists[c].p + off[c][(size_t)d];
-    const int32_t n0 = cnt[0][(size_t)d], n1 = cnt[1][(size_t)d], n2 = cnt[2][(size_t)d];
-    if (n0 > 0) hipLaunchKernelGGL(build_node<256>, dim3((unsigned)n0), dim3(256), 0, s, a, 0);
-    if (n1 > 0) hipLaunchKernelGGL(build_node<64>, dim3((unsigned)n1), dim3(64), 0, s, a, 1);
-    if (n2 > 0)
-      hipLaunchKernelGGL(build_thread, dim3(grid_of((int64_t)n2, 64)), dim3(64), 0, s, a, n2);
-    BVH_TRY(hipGetLastError());
-  }
+  for (int c = 0; c < 3; c++) a.jobs[c] = (const BuildJob*)lists[c].p;
+  if (cnt[0] > 0)
+    hipLaunchKernelGGL(build_node<kGroup>, dim3((unsigned)cnt[0]), dim3(kGroup), 0, s, a, 0);
+  if (cnt[1] > 0) hipLaunchKernelGGL(build_node<64>, dim3((unsigned)cnt[1]), dim3(64), 0, s, a, 1);
+  if (cnt[2] > 0)
+    hipLaunchKernelGGL(build_thread, dim3(grid_of((int64_t)cnt[2], 64)), dim3(64), 0, s, a,
+                       (int32_t)cnt[2]);
+  BVH_TRY(hipGetLastError());
   BVH_TRY(mRT.alloc((size_t)nn * 12 * sizeof(double)));
   BVH_TRY(parent.alloc((size_t)nn * 4));
   hipLaunchKernelGGL(model_frames, dim3(grid_of(nn, 256)), dim3(256), 0, s, a.nodes, nn,
