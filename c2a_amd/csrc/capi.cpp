@@ -278,22 +278,27 @@ void params_to_args(KArgs& a, const c2a_params* p) {
 // The extension levels are tuned for the plain order only: under the learned
 // order, and when the batch logs training samples (which are drawn from the
 // replayed records), they stay at 0 unless given.
+void tune_args(KArgs& t, int replay_log, int ext_levels, bool ext) {
+  const int rows = std::min(kTuneRows, C2A_TUNE_MAX);
+  t.ntune = rows;
+  for (int r = 0; r < rows; r++) {
+    t.tune_ntri[r] = kTune[r][0];
+    t.tune_depth[r] = std::min(6, std::max(1, kTune[r][1]));
+    // the learned order's replays hold fewer misses: three levels below one
+    // (2048 knot queries, MI355X: 206 ms; four levels 214)
+    t.tune_miss[r] = std::max(0, ext ? kTune[r][2] : std::min(3, kTune[r][2]));
+    t.tune_log[r] = replay_log >= 0 ? replay_log : kTune[r][3];
+    t.tune_ext[r] = ext_levels >= 0 ? std::min(8, ext_levels)
+                                    : (ext ? std::min(8, std::max(0, kTune[r][4])) : 0);
+  }
+}
+
 void apply_tuning(c2a_batch* b, const std::vector<int32_t>& pairs, int replay_log,
                   int ext_levels) {
   if (kTuneRows <= 0) return;
   const int rows = std::min(kTuneRows, C2A_TUNE_MAX);
   KArgs& t = b->tune;
-  t.ntune = rows;
-  for (int r = 0; r < rows; r++) {
-    t.tune_ntri[r] = kTune[r][0];
-    t.tune_depth[r] = std::min(6, std::max(1, kTune[r][1]));
-    t.tune_miss[r] = std::max(0, kTune[r][2]);
-    t.tune_log[r] = replay_log >= 0 ? replay_log : kTune[r][3];
-    t.tune_ext[r] = ext_levels >= 0 ? std::min(8, ext_levels)
-                                    : ((b->scorer || b->sample_cap > 0)
-                                           ? 0
-                                           : std::min(8, std::max(0, kTune[r][4])));
-  }
+  tune_args(t, replay_log, ext_levels, !b->scorer && b->sample_cap <= 0);
   // the kernel's depth and arena are sized for the buckets the batch uses
   int kmax = 1, logmax = 0;
   for (size_t i = 0; i + 1 < pairs.size(); i += 2) {
@@ -537,6 +542,7 @@ int c2a_ccd_batch_noalloc(c2a_mesh* const* meshes, int32_t nmesh, const double* 
   a.nq = nq;
   a.logcap = logcap;
   a.arena = logcap > 0 ? sp + kScratchArena : nullptr;
+  if (p->spec_depth == 0) tune_args(a, logcap, p->ext_levels, true);
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(write_mesh_table, dim3(1), dim3(C2A_NOALLOC_MAX_MESHES), 0, s,
                      (MeshDev*)(sp + kScratchTable), tab, nmesh);
