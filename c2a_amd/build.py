@@ -42,7 +42,7 @@ def _run(cmd):
 
 
 def kernel_shapes():
-    """(K, CAP, NW, LRN) of every shape in ccd_shapes.h's C2A_SHAPES list."""
+    """(K, CAP, NW, V) of every shape in ccd_shapes.h's C2A_SHAPES list."""
     text = open(os.path.join(CSRC, "ccd_shapes.h")).read()
     body = text[text.index("#define C2A_SHAPES(X)"):]
     body = body[:body.index("\n\n")]

@@ -363,6 +363,10 @@ struct EdgeWin {
   double AT, BT;   // segment parameters
 };
 
+#if defined(__clang__)   // lane masks are combined without branches on purpose
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Wbitwise-instead-of-logical"
+#endif
 // The four cases of a class in the reference's order: both edges at their
 // far side, A's far and B's near, A's near and B's far, both near.  Each lane
 // takes its own next case that passes the extent pre-test, so a wavefront
@@ -414,6 +418,9 @@ C2A_HD void edge_class(EdgeWin& g, int cls, const EdgeClass& e, bool o1, Side x1
     c3 = c3 & !p3 & !ok;
   } while (wave_any(c1 | c2 | c3));
 }
+#if defined(__clang__)
+#pragma clang diagnostic pop
+#endif
 
 // The 16 edge-pair cases are decided in the reference's order; the first one
 // whose extent pre-test and two Voronoi tests hold gives the closest points.

@@ -173,9 +173,9 @@ int pick_shape(const c2a_params* p, int& K, int& NW) {
     return fail(C2A_ERR_BAD_ARG, "order must be C2A_ORDER_PLAIN or C2A_ORDER_LEARNED");
   if (learned && !p->scorer) return fail(C2A_ERR_BAD_ARG, "learned order needs a scorer");
   if (K < 1 || K > 6) return fail(C2A_ERR_BAD_ARG, "spec_depth must be 1..6");
-  if (NW != 1 || !kernel_shape_ok(K, 48, NW, false))
+  if (NW != 1 || !kernel_shape_ok(K, 48, NW, 0))
     return fail(C2A_ERR_BAD_ARG, "waves_per_query must be 0 or 1");
-  if (learned && !kernel_shape_ok(K, 48, NW, true))
+  if (learned && !kernel_shape_ok(K, 48, NW, 1))
     return fail(C2A_ERR_BAD_ARG, "learned order runs at spec_depth 0 or 5");
   return C2A_OK;
 }
@@ -203,9 +203,9 @@ int compute_units() {
 
 // Resident workgroups: the kernel is persistent, so launching more than fit
 // at once only adds workgroups that find the queue empty.
-int grid_blocks(int K, int CAP, int NW, int64_t nq, bool learned = false) {
+int grid_blocks(int K, int CAP, int NW, int64_t nq, int variant = 0) {
   const int cus = compute_units();
-  int per_cu = kernel_blocks_per_cu(K, CAP, NW, learned);
+  int per_cu = kernel_blocks_per_cu(K, CAP, NW, variant);
   if (per_cu < 1) per_cu = 1;
   const int64_t cap = (int64_t)cus * per_cu;
   return (int)std::max<int64_t>(1, std::min<int64_t>(nq, cap));
@@ -227,7 +227,7 @@ constexpr int kWideWaves = 4;
 // compute unit).
 bool wide_batch(int64_t nq, int CAP, bool ccd) {
   return nq <= (int64_t)compute_units() * (ccd ? 4 : 2) &&
-         kernel_shape_ok(kWideK, CAP, kWideWaves, false);
+         kernel_shape_ok(kWideK, CAP, kWideWaves, 0);
 }
 
 int prepare_queries(const std::vector<MeshDev>& tab, const c2a_query* q, int64_t nq,
@@ -377,9 +377,9 @@ int run_batch(const c2a_batch* b, hipStream_t s) {
   return C2A_OK;
 }
 
-// Sets up the tail pass when the batch can take it: plain order, no sample
-// logging, a stack the four-wavefront shapes cover.  With tail_budget, long
-// queries are handed over by their BV tests.  Without, a batch that is too
+// Sets up the tail pass when the batch can take it: no sample logging, a stack
+// the four-wavefront shapes cover.  With tail_budget (plain order), long
+// queries are handed over by their BV tests, without their replay log.  Without, a batch that is too
 // large for four wavefronts per query hands over the last unfinished ones, one
 // per compute unit at most: at that point they are the batch's longest queries
 // and three quarters of the chip has nothing left to do, and the step costs
@@ -390,8 +390,8 @@ int run_batch(const c2a_batch* b, hipStream_t s) {
 int setup_tail(c2a_batch* b, const c2a_params* p) {
   const int64_t budget = p->tail_budget;
   const bool last = budget <= 0 && p->spec_depth == 0 && p->waves_per_query == 0 && b->NW == 1;
-  if ((budget <= 0 && !last) || b->nq < 2 || b->scorer || b->sample_cap > 0 ||
-      !kernel_shape_ok(kWideK, b->CAP, kWideWaves, false))
+  if ((budget <= 0 && !last) || b->nq < 2 || (b->scorer && !last) || b->sample_cap > 0 ||
+      !kernel_shape_ok(kWideK, b->CAP, kWideWaves, 0))
     return C2A_OK;
   int rc;
   if ((rc = b->d_tail.alloc((size_t)b->nq * sizeof(TailRec))) ||
@@ -947,11 +947,11 @@ int c2a_batch_create(c2a_mesh* const* meshes, int32_t nmesh, const c2a_query* q,
   if (b->CAP == 192) b->K = 5;
   if ((!params || (params->spec_depth == 0 && params->waves_per_query == 0 &&
                    params->tail_budget <= 0)) &&
-      !b->scorer && b->sample_cap == 0 && wide_batch(nq, b->CAP, true)) {
+      b->sample_cap == 0 && wide_batch(nq, b->CAP, true)) {
     b->K = kWideK;
     b->NW = kWideWaves;
   }
-  b->blocks = grid_blocks(b->K, b->CAP, b->NW, nq, b->scorer != nullptr);
+  b->blocks = grid_blocks(b->K, b->CAP, b->NW, nq, b->scorer ? 1 : 0);
   const bool feats = b->scorer || b->sample_cap > 0;
   if (b->logcap > 0 && nq > 0) {
     // one replay arena per resident workgroup: fewer workgroups when the
@@ -1009,7 +1009,8 @@ int c2a_batch_run(c2a_batch* b, void* stream) {
   if (!b) return fail(C2A_ERR_BAD_ARG, "null batch");
   if (b->nq == 0) return C2A_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (b->scorer) b->args.scorer = scorer_view(b->scorer);   // current parameters
+  if (b->scorer)   // current parameters
+    b->args.scorer = b->args2.scorer = scorer_view(b->scorer);
   if (b->sample_cap > 0) {
     hipLaunchKernelGGL(zero_counter, dim3(1), dim3(1), 0, s, (int64_t*)b->d_scount.p);
     HIP_TRY(hipGetLastError());
@@ -1255,7 +1256,7 @@ static int contact_queries(c2a_mesh* const* meshes, int32_t nmesh, const double*
   a.counter = (int64_t*)dc.p;
   a.nq = nq;
   a.mode = MODE_CONTACT;
-  if ((rc = run_kernel(a, K, CAP, NW, grid_blocks(K, CAP, NW, nq), s))) return rc;
+  if ((rc = run_kernel(a, K, CAP, NW, grid_blocks(K, CAP, NW, nq, CAP == 192 ? 0 : 2), s))) return rc;
   HIP_TRY(hipMemcpyAsync(counts_out, dout.p, (size_t)nq * sizeof(int32_t), hipMemcpyDeviceToHost, s));
   if (cap > 0)
     HIP_TRY(hipMemcpyAsync(out, drec.p, (size_t)nq * cap * sizeof(c2a_contact),
@@ -1358,7 +1359,7 @@ static int distance_queries(c2a_mesh* const* meshes, int32_t nmesh, const double
   a.counter = (int64_t*)dc.p;
   a.nq = nq;
   a.mode = MODE_DISTANCE;
-  if ((rc = run_kernel(a, K, CAP, NW, grid_blocks(K, CAP, NW, nq), s))) return rc;
+  if ((rc = run_kernel(a, K, CAP, NW, grid_blocks(K, CAP, NW, nq, CAP == 192 ? 0 : 2), s))) return rc;
   HIP_TRY(hipMemcpyAsync(out, dout.p, (size_t)nq * sizeof(c2a_distance_result),
                          hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));

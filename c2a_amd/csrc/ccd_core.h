@@ -408,7 +408,13 @@ struct Shape {
   static constexpr int PER_LANE = (NSLOT - 1 + 63) / 64;
 };
 
-template <int K, int CAP>
+// The query's state in LDS.  ST: the kernel for contact and distance queries
+// only (no motions, replay, scan or CA loop).  The full kernel takes 512
+// registers per lane, one wavefront per SIMD; without that code 256 do, two per
+// SIMD, and its LDS is a seventh of a compute unit's.  16,384 distance queries
+// between two 8192-triangle knots on MI355X, host to host: 106 ms in the
+// full kernel, 62 ms in this one.
+template <int K, int CAP, bool ST = false>
 struct Wave {
   Entry stack[CAP];
   Slot slot[Shape<K>::NSLOT];
@@ -421,18 +427,18 @@ struct Wave {
                              // enumeration, distance query); 2: a distance
                              // query entering only overlapping RSS pairs
   int32_t gen;
-  HotRec win[WIN];           // replayed records [L.wbase, L.wbase + WIN)
-  LogEnt lbuf[LBUF];         // log entries [L.nflush, L.nlog) not yet in the arena
-  int32_t anc[CAP + 2];      // scan: log index of the last event at each depth
-  int32_t lastlane[CAP + 2]; // scan: scratch for the per-depth last event
+  HotRec win[ST ? 1 : WIN];           // replayed records [L.wbase, L.wbase + WIN)
+  LogEnt lbuf[ST ? 1 : LBUF];         // log entries [L.nflush, L.nlog) not yet in the arena
+  int32_t anc[ST ? 1 : CAP + 2];      // scan: log index of the last event at each depth
+  int32_t lastlane[ST ? 1 : CAP + 2]; // scan: scratch for the per-depth last event
   int32_t nleafq;            // replay: leaf records queued for the triangle pass
   int32_t next;              // replay: pairs queued for the speculative extension
   int64_t ticket;            // work-queue ticket shared by the wavefronts
   int32_t rarena;            // the pending round writes its subtree to the arena
   int32_t rdepth;            // levels of the slot heap the current round filled
   int32_t rpb;               // ... as pairs [rpb, rpb + 2^K - 1)
-  int32_t lh[CAP + 2];       // replay: expansions per level, then fill cursors
-  int32_t ls[CAP + 3];       // replay: first sorted expansion of each level
+  int32_t lh[ST ? 1 : CAP + 2];       // replay: expansions per level, then fill cursors
+  int32_t ls[ST ? 1 : CAP + 3];       // replay: first sorted expansion of each level
   // Misses ahead in the scan's window share a round: each gets a heap of
   // `mpage` slots (mpage = 0: one heap below X).
   int32_t mpage;             // slots per heap of the current round
@@ -448,8 +454,8 @@ struct Wave {
 
 // A mesh-table entry held in LDS, made wavefront-uniform so that node and
 // triangle addresses use scalar base registers.
-template <int K, int CAP>
-C2A_HD MeshDev mesh_of(const Wave<K, CAP>& g, int k) {
+template <int K, int CAP, bool ST>
+C2A_HD MeshDev mesh_of(const Wave<K, CAP, ST>& g, int k) {
   MeshDev m = g.md[k];
 #if defined(__HIP_DEVICE_COMPILE__)
   const uint64_t pn = (uint64_t)m.nodes, pt = (uint64_t)m.tris;
@@ -789,8 +795,8 @@ C2A_HD bool ca_on_tris(const Motion& mo1, const double* r1, const double* A, con
 
 // Heap slot h of the subtree below the heap's root pair: the pair reached by
 // the path bits of h+1, its transform chained from the root's, and its values.
-template <int K, int CAP>
-C2A_HD void compute_slot_below(Wave<K, CAP>& g, const Slot& root, int h, const MeshDev& M1,
+template <int K, int CAP, bool ST>
+C2A_HD void compute_slot_below(Wave<K, CAP, ST>& g, const Slot& root, int h, const MeshDev& M1,
                                const MeshDev& M2, bool contact, Slot& s) {
   int b1 = root.b1, b2 = root.b2;
   node_ptr N1 = nodes_of(M1);
@@ -836,8 +842,8 @@ C2A_HD void compute_slot_below(Wave<K, CAP>& g, const Slot& root, int h, const M
 // Heap slot h of the round written as arena record 2 * rpb + h, so that the
 // pair stays available for the rest of the step; slots above the last level
 // link their children (pair rpb + h).
-template <int K, int CAP>
-C2A_HD void compute_slot_arena(Wave<K, CAP>& g, int h, const MeshDev& M1, const MeshDev& M2,
+template <int K, int CAP, bool ST>
+C2A_HD void compute_slot_arena(Wave<K, CAP, ST>& g, int h, const MeshDev& M1, const MeshDev& M2,
                                const ArenaView& av) {
   Slot s;
   compute_slot_below(g, g.slot[0], h, M1, M2, false, s);
@@ -900,12 +906,12 @@ C2A_HD bool heaps_on(const KArgs& a, int nl) {
 }
 
 // One lane's share of a round.
-template <int K, int CAP>
-C2A_HD void round_lane(Wave<K, CAP>& g, const Leader& L, int lane, int nl, const KArgs& a) {
+template <int K, int CAP, bool ST>
+C2A_HD void round_lane(Wave<K, CAP, ST>& g, const Leader& L, int lane, int nl, const KArgs& a) {
   const MeshDev M1 = mesh_of(g, 0);
   const MeshDev M2 = mesh_of(g, 1);
-  const bool contact = g.contact != 0;
-  if (arena_rounds_on(a) && g.rarena) {
+  const bool contact = ST || g.contact != 0;
+  if (!ST && arena_rounds_on(a) && g.rarena) {
     const ArenaView av = arena_view(L.ab, a.logcap);
     for (int h = lane + 1; h < Shape<K>::NSLOT; h += nl) compute_slot_arena(g, h, M1, M2, av);
     return;
@@ -923,8 +929,8 @@ C2A_HD void round_lane(Wave<K, CAP>& g, const Leader& L, int lane, int nl, const
   }
 }
 
-template <int K, int CAP>
-C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD void request_round(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   Entry& e = g.stack[L.sp - 1];
   int gen = g.gen + 1;
   if (gen >= 0x7fffff) {   // generation wrap: forget every cached link
@@ -932,18 +938,18 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
     gen = 1;
     if (lane == 0) g.mrgen = -1;
   }
-  const int flags = uni(e.flags);
+  const int flags = ST ? uni(e.flags) & ~8 : uni(e.flags);   // (no replayed pairs)
   const int ar = uni(e.ar);
   const int sg = (gen << 8) | 1;
   // internal pairs of a CA step go to the arena while it has room
   constexpr int NPAIR = (1 << K) - 1;
-  const bool to_arena = arena_rounds_on(a) && !a.scorer.on && a.logcap > 0 && !g.contact &&
+  const bool to_arena = !ST && arena_rounds_on(a) && !a.scorer.on && a.logcap > 0 && !g.contact &&
                         (flags & 3) != 3 && L.napp + NPAIR <= 2 * a.logcap;
   // a miss the scan found with more misses after it in its window: one
   // shallow heap below each (the same slots a round below each would fill)
   const int mpage = 2 << L.kmiss;
   const int nmr = uni(g.nmr);
-  const bool multi = !to_arena && (flags & 8) && (flags & 3) != 3 && L.kmiss > 0 &&
+  const bool multi = !ST && !to_arena && (flags & 8) && (flags & 3) != 3 && L.kmiss > 0 &&
                      L.kmiss < L.kdepth && 2 * mpage <= Shape<K>::NSLOT + 1 && nmr > 1 &&
                      ar == uni(g.mrrec[0]);
   const int cap = (Shape<K>::NSLOT + 1) / mpage;
@@ -1037,8 +1043,8 @@ C2A_HD void request_round(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
 // Root pair of a traversal at absolute poses (C2A.cpp:1793-1806).  `nn` is
 // the root's record number in this step's log (0), or -1 when the traversal
 // is not logged.
-template <int K, int CAP>
-C2A_HD void start_traversal(Wave<K, CAP>& g, Leader& L, const MeshDev& M1, const MeshDev& M2,
+template <int K, int CAP, bool ST>
+C2A_HD void start_traversal(Wave<K, CAP, ST>& g, Leader& L, const MeshDev& M1, const MeshDev& M2,
                             const double* R1, const double* T1, const double* R2,
                             const double* T2, int nn, int lane) {
   double Tt[3], Rt[9], R[9], T[3], Rrel[9], Trel[3], C1R[9], C2R[9], C1T[3], C2T[3];
@@ -1139,8 +1145,8 @@ C2A_HD void write_samples(const LeaderT& L, const KArgs& a, const ArenaView& av,
 // values, features, and a queue entry for the triangle pass if it is a leaf
 // pair.  `fresh`: the record lies beyond the previous step's records (its
 // child link starts empty).
-template <int K, int CAP>
-C2A_HD void replay_record(Wave<K, CAP>& g, const Leader& L, const KArgs& a, const ArenaView& av,
+template <int K, int CAP, bool ST>
+C2A_HD void replay_record(Wave<K, CAP, ST>& g, const Leader& L, const KArgs& a, const ArenaView& av,
                           node_ptr N1, node_ptr N2, const LogEnt le, int e, int side, bool fresh) {
   double C2A_GLOBAL* xf = gp(av.xf);
   int32_t C2A_GLOBAL* cpa = gp(av.cpa);
@@ -1187,8 +1193,8 @@ C2A_HD void replay_record(Wave<K, CAP>& g, const Leader& L, const KArgs& a, cons
 // computed as a child of an expansion (C2A.cpp:1195-1276 per pair), level by
 // level so that each record's parent transform is ready before it is needed.
 // Lanes take one record each.
-template <int K, int CAP>
-C2A_HD void replay(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD void replay(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   const ArenaView av = arena_view(L.ab, a.logcap, a.feats != 0);
   const LogEnt C2A_GLOBAL* lg = gp(L.logbuf ? av.log0 : av.log1);
   double C2A_GLOBAL* xf = gp(av.xf);
@@ -1332,8 +1338,8 @@ C2A_HD void replay(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl)
 // child first, C2A.cpp:1281, or the lower score under the learned order),
 // then the records scattered into that order.  Training samples of the
 // replayed pairs are written on the way up.
-template <int K, int CAP>
-C2A_HD void replay_layout(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD void replay_layout(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   const ArenaView av = arena_view(L.ab, a.logcap, a.feats != 0);
   const LogEnt C2A_GLOBAL* lg = gp(L.logbuf ? av.log0 : av.log1);
   int32_t C2A_GLOBAL* order = gp(av.order);
@@ -1409,8 +1415,8 @@ C2A_HD void replay_layout(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, 
 
 // Starts the scan of a replayed step: the root pair is always expanded
 // (C2A.cpp:1920 -> 1279) and logged first.
-template <int K, int CAP>
-C2A_HD void start_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD void start_scan(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   const ArenaView av = arena_view(L.ab, a.logcap);
   if (lane == 0) {
     LogEnt v;
@@ -1441,8 +1447,8 @@ C2A_HD void start_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
 // handed to the sequential walk.  A pruned pair the previous step expanded
 // skips its replayed subtree.  Returns 1 when such a pair waits on the
 // stack, 0 when the step is complete.
-template <int K, int CAP>
-C2A_HD int scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD int scan(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   const ArenaView av = arena_view(L.ab, a.logcap);
   const Event C2A_GLOBAL* ev = gp(av.ev);
   LogEnt C2A_GLOBAL* lw = gp(L.logbuf ? av.log1 : av.log0);
@@ -1591,8 +1597,8 @@ C2A_HD int scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
 }
 
 // Stages replayed records [rec, rec + WIN) in LDS.
-template <int K, int CAP>
-C2A_HD void load_window(Wave<K, CAP>& g, Leader& L, const ArenaView& av, int rec, int nrec_max,
+template <int K, int CAP, bool ST>
+C2A_HD void load_window(Wave<K, CAP, ST>& g, Leader& L, const ArenaView& av, int rec, int nrec_max,
                         int lane, int nl) {
   const HotRec C2A_GLOBAL* hot = gp(av.hot);
   C2A_CHECK(rec >= 0 && rec + 1 < nrec_max);
@@ -1606,8 +1612,8 @@ C2A_HD void load_window(Wave<K, CAP>& g, Leader& L, const ArenaView& av, int rec
 // Copies the staged log entries to the arena (lane-parallel).  Keeping
 // global stores out of the per-expansion path matters: a store's completion
 // is waited for wherever the walk next waits on vector memory.
-template <int K, int CAP>
-C2A_HD void flush_log(Wave<K, CAP>& g, Leader& L, const ArenaView& av, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD void flush_log(Wave<K, CAP, ST>& g, Leader& L, const ArenaView& av, int lane, int nl) {
   const int n = L.nlog - L.nflush;
   if (n <= 0) return;
   LogEnt C2A_GLOBAL* lw = gp(L.logbuf ? av.log1 : av.log0) + L.nflush;
@@ -1621,8 +1627,8 @@ C2A_HD void flush_log(Wave<K, CAP>& g, Leader& L, const ArenaView& av, int lane,
 // contact traversal's pose: the features and closest points of the same
 // triangle distance the leaf test made.  Feature ids are the vertex slots
 // 0..2 of the triangle; the host maps them to the caller's vertex ids.
-template <int K, int CAP>
-C2A_HD void record_contact(const Wave<K, CAP>& g, c2a_contact* out, int t1, int t2) {
+template <int K, int CAP, bool ST>
+C2A_HD void record_contact(const Wave<K, CAP, ST>& g, c2a_contact* out, int t1, int t2) {
   const MeshDev M1 = mesh_of(g, 0);
   const MeshDev M2 = mesh_of(g, 1);
   double ta[9], tb[9], Rrel[9], Trel[3], p[3], q[3], u[3], pb[3];
@@ -1650,8 +1656,8 @@ C2A_HD void record_contact(const Wave<K, CAP>& g, c2a_contact* out, int t1, int 
 // Puts the pair being processed back on the stack (a round will be rooted
 // at it).  where: 0 = its full entry is still at stack[sp] (it was just
 // popped), 1 = it is slot `csl` of the current round, 2 = a replayed record.
-template <int K, int CAP>
-C2A_HD void push_back(Wave<K, CAP>& g, Leader& L, const Cur& c, int where, int csl, int lane,
+template <int K, int CAP, bool ST>
+C2A_HD void push_back(Wave<K, CAP, ST>& g, Leader& L, const Cur& c, int where, int csl, int lane,
                       int nl) {
   if (where == 1) {
     lane_sync();
@@ -1671,8 +1677,8 @@ C2A_HD void push_back(Wave<K, CAP>& g, Leader& L, const Cur& c, int where, int c
 // across lanes.  Returns true when a round has been requested.  One pair at
 // a time: heaps of more than 64 pairs (K = 6) and the host-side harness's
 // one-lane and arena-round runs; the others take walk_heaps.
-template <int K, int CAP>
-C2A_HD bool walk_pairs(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD bool walk_pairs(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   const int cmode = g.contact;
   const bool contact = cmode != 0;
   const bool learned = a.scorer.on && !contact;
@@ -1880,10 +1886,10 @@ C2A_HD bool leaf_update(Leader& L, int cmode, int strict, double dTri, double ml
 // of dependent LDS reads and uniform code, one useful lane), a heap of 62
 // pairs holds 8.6 visited ones on the heaviest knot query, and deciding the
 // heap takes two or three passes of about 400 instructions.
-template <int K, int CAP>
-C2A_HD int heap_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, const Cur& x, int base,
+template <int K, int CAP, bool ST>
+C2A_HD int heap_scan(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, const Cur& x, int base,
                      int lane, int& nhit) {
-  const int cmode = uni(g.contact);
+  const int cmode = ST ? (uni(g.contact) == 2 ? 2 : 1) : uni(g.contact);
   const bool counts = cmode != 0 && L.mode != MODE_DISTANCE;   // contact enumeration
   const double inf = 1.0 / 0.0;
   const int rd = uni(g.rdepth);
@@ -1930,7 +1936,7 @@ C2A_HD int heap_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, const Cur& x, i
   const ArenaView av = arena_view(L.ab, a.logcap);
   LogEnt C2A_GLOBAL* lw = gp(L.logbuf ? av.log1 : av.log0);
   int enx = -1;
-  if (x.nn >= 0 && L.nlog < L.klog) {
+  if (!ST && x.nn >= 0 && L.nlog < L.klog) {
     enx = L.nlog++;
     if (lane == 0) {
       LogEnt v;
@@ -1979,13 +1985,18 @@ C2A_HD int heap_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, const Cur& x, i
       }
       nhit = (int)__builtin_popcountll(hm);
     }
-    if (logging && L.nlog + nexp > L.klog) logging = false;
-    if (expand && logging) en = L.nlog + lanes_below(em, j);
-    if (logging) L.nlog += nexp;
+    // the log takes the first klog expansions of a step in depth-first order
+    const int at = L.nlog + lanes_below(em, j);
+    const bool logs = expand && logging && at < L.klog;
+    if (logs) en = at;
+    if (logging) {
+      L.nlog = L.nlog + nexp < L.klog ? L.nlog + nexp : L.klog;
+      logging = L.nlog < L.klog;
+    }
     const int pen_in = lane_bcast(en, prank > 0 ? prank - 1 : 0);
     const int pen = prank > 0 ? pen_in : enx;
     const int nn = pen < 0 ? -1 : 2 * pen + 1 + ((loc - 1) & 1);
-    if (expand && logging && lane < 64) {
+    if (logs && lane < 64) {
       LogEnt v;
       v.rec = nn;
       v.b1 = b1;
@@ -2051,9 +2062,9 @@ C2A_HD int heap_scan(Wave<K, CAP>& g, Leader& L, const KArgs& a, const Cur& x, i
 // The traversal below the pairs on the stack: a pair that has to be
 // expanded gets a round (a heap of pair values below it), and heap_scan
 // decides the heap.  Returns true when a round has been requested.
-template <int K, int CAP>
-C2A_HD bool walk_heaps(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
-  const int cmode = uni(g.contact);
+template <int K, int CAP, bool ST>
+C2A_HD bool walk_heaps(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
+  const int cmode = ST ? (uni(g.contact) == 2 ? 2 : 1) : uni(g.contact);
   const bool counts = cmode != 0 && L.mode != MODE_DISTANCE;
   int nhit = 0, next = 0;   // next: 1 a round for the top pair, 2 stack full
   for (;;) {
@@ -2123,16 +2134,17 @@ C2A_HD bool walk_heaps(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
   }
 }
 
-template <int K, int CAP>
-C2A_HD bool walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
-  return heaps_on<K>(a, nl) ? walk_heaps(g, L, a, lane, nl) : walk_pairs(g, L, a, lane, nl);
+template <int K, int CAP, bool ST>
+C2A_HD bool walk(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
+  if constexpr (ST) return walk_heaps(g, L, a, lane, nl);
+  else return heaps_on<K>(a, nl) ? walk_heaps(g, L, a, lane, nl) : walk_pairs(g, L, a, lane, nl);
 }
 
 // After a step's walk: closest points of a replayed last improving leaf
 // (the same triangle-distance call a round would have made), and the log
 // hand-over to the next step.
-template <int K, int CAP>
-C2A_HD void end_walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD void end_walk(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   if (L.pq_pending) {
     const MeshDev M1 = mesh_of(g, 0);
     const MeshDev M2 = mesh_of(g, 1);
@@ -2155,11 +2167,11 @@ C2A_HD void end_walk(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int n
   }
 }
 
-template <int K, int CAP>
-C2A_HD void begin_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
+template <int K, int CAP, bool ST>
+C2A_HD void begin_step(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
   const MeshDev M1 = mesh_of(g, 0);
   const MeshDev M2 = mesh_of(g, 1);
-  if (L.mode == MODE_QUERY) {   // the other modes' traversals start in fetch
+  if (!ST && L.mode == MODE_QUERY) {   // the other modes' traversals start in fetch
     double R1[9], T1[3], R2[9], T2[3];
     if (L.numCA == 0) {
       for (int i = 0; i < 9; i++) { R1[i] = g.mo[0].R0[i]; R2[i] = g.mo[1].R0[i]; }
@@ -2191,7 +2203,7 @@ C2A_HD void begin_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
   for (int i = 0; i < 9; i++) Rrel[i] = g.Rrel[i];
   for (int i = 0; i < 3; i++) Trel[i] = g.Trel[i];
   L.D = tri_distance(Rrel, Trel, ta, tb, p, q, nullptr);
-  if (L.mode == MODE_DISTANCE) {   // C2A_Distance's first bound (C2A_PQP.cpp:998-1005)
+  if (ST || L.mode == MODE_DISTANCE) {   // C2A_Distance's first bound (C2A_PQP.cpp:998-1005)
     if (lane == 0)
       for (int i = 0; i < 3; i++) { g.p1[i] = p[i]; g.p2[i] = q[i]; }
     lane_sync();
@@ -2214,8 +2226,8 @@ C2A_HD void begin_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
 
 // Finishes the CA loop (C2A.cpp:2125-2143) and optionally starts the contact
 // traversal at the TOC pose (C2A_Solve, C2A.cpp:2411-2435).
-template <int K, int CAP>
-C2A_HD void finish_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, bool collisionfree,
+template <int K, int CAP, bool ST>
+C2A_HD void finish_query(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, bool collisionfree,
                          int lane) {
   double Rt[9], Tt[3];
   if (!collisionfree) motion_integrate(g.mo[0], L.toc, Rt, Tt, nullptr);
@@ -2261,8 +2273,8 @@ C2A_HD void finish_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, bool collis
 // Saves the CA-loop state of a query about to start its next step and hands
 // the query to the tail pass (the next step starts there without a replay:
 // pair values do not depend on it).
-template <int K, int CAP>
-C2A_HD void hand_over(const Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
+template <int K, int CAP, bool ST>
+C2A_HD void hand_over(const Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
   if (lane == 0) {
     TailRec& t = a.tail_rec[L.qi];
     t.lamda = L.lamda;
@@ -2305,8 +2317,8 @@ C2A_HD bool few_left(const KArgs& a) {
 
 // End of a step in the CA loop (C2A.cpp:2029-2123): schedules the next step
 // (state ST_STEP) or finishes the query.
-template <int K, int CAP>
-C2A_HD void after_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
+template <int K, int CAP, bool ST>
+C2A_HD void after_step(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
   if (L.mode == MODE_STEP) {
     if (lane == 0) {
       c2a_step_result* r = a.step_out + L.qi;
@@ -2372,8 +2384,8 @@ C2A_HD void after_step(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
 }
 
 // Takes the next query from the work queue (one atomic per workgroup).
-template <int K, int CAP>
-C2A_HD int64_t take_ticket(Wave<K, CAP>& g, int64_t* counter, int lane) {
+template <int K, int CAP, bool ST>
+C2A_HD int64_t take_ticket(Wave<K, CAP, ST>& g, int64_t* counter, int lane) {
 #if defined(__HIP_DEVICE_COMPILE__)
   if (lane == 0) g.ticket = (int64_t)atomicAdd((unsigned long long*)counter, 1ull);
 #else
@@ -2385,8 +2397,8 @@ C2A_HD int64_t take_ticket(Wave<K, CAP>& g, int64_t* counter, int lane) {
   return t;
 }
 
-template <int K, int CAP>
-C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
+template <int K, int CAP, bool ST>
+C2A_HD bool fetch(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
   if (a.tail_left > 0 && !a.tail_pass && L.fetched && lane == 0) {
 #if defined(__HIP_DEVICE_COMPILE__)
     atomicAdd(a.finished, 1);
@@ -2419,7 +2431,7 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
   lane_sync();
   if (lane == 0)
     for (int i = 0; i < 3; i++) { g.p1[i] = 0.0; g.p2[i] = 0.0; }
-  if (a.mode == MODE_STEP) {
+  if (!ST && a.mode == MODE_STEP) {
     const StepDev& q = a.step_in[qi];
     if (lane == 0) {
       g.mo[0] = q.mo[0];
@@ -2449,7 +2461,7 @@ C2A_HD bool fetch(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
     L.state = ST_STEP;
     return true;
   }
-  if (a.mode == MODE_CONTACT || a.mode == MODE_DISTANCE) {
+  if (ST || a.mode == MODE_CONTACT || a.mode == MODE_DISTANCE) {
     // contact enumeration, or C2A_Distance with qsize <= 2 (C2A_PQP.cpp:970-1057):
     // both walk pair distances without motion bounds
     const ContactDev& c = a.contact_in[qi];
@@ -2600,8 +2612,8 @@ C2A_HD void load_tri(double* out, const MeshDev& M, int t) {
 // their parent is expanded, as in the reference.  The reference leaves
 // res->p1/p2 uninitialised on this branch; here they are the closest points
 // of the final triangle distance.  The models' last_tri are not updated.
-template <int K, int CAP>
-C2A_HD void translation_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
+template <int K, int CAP, bool ST>
+C2A_HD void translation_query(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
   const MeshDev M1 = mesh_of(g, 0);
   const MeshDev M2 = mesh_of(g, 1);
   node_ptr N1 = nodes_of(M1);
@@ -2744,9 +2756,51 @@ C2A_HD void translation_query(Wave<K, CAP>& g, Leader& L, const KArgs& a, int la
   finish_query(g, L, a, L.toc >= 1.0, lane);
 }
 
+// One of the states only a CCD query has; false: a round is needed or the
+// state is final.
+template <int K, int CAP, bool ST>
+C2A_HD bool run_ccd_state(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
+  switch (L.state) {
+    case ST_TRANS:
+      translation_query(g, L, a, lane);
+      break;
+    case ST_LAYOUT:
+      replay_layout(g, L, a, lane, nl);
+      start_scan(g, L, a, lane, nl);
+      L.state = ST_SCAN;
+      break;
+    case ST_SCAN:
+      if (scan(g, L, a, lane, nl)) {
+        L.state = ST_SUB;
+        break;
+      }
+      end_walk(g, L, a, lane, nl);
+      after_step(g, L, a, lane);
+      break;
+    case ST_SUB:
+      if (walk(g, L, a, lane, nl)) return false;
+      flush_log(g, L, arena_view(L.ab, a.logcap), lane, nl);
+      if (L.flags & C2A_FLAG_STACK_OVERFLOW) {
+        end_walk(g, L, a, lane, nl);
+        after_step(g, L, a, lane);
+      } else {
+        L.state = ST_SCAN;
+      }
+      break;
+    case ST_WALK:
+      if (walk(g, L, a, lane, nl)) return false;
+      end_walk(g, L, a, lane, nl);
+      after_step(g, L, a, lane);
+      break;
+    default:
+      return false;
+  }
+  return true;
+}
+
 // Advances the query state until a round is needed or no work is left.
-template <int K, int CAP>
-C2A_HD void leader_run(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int nl) {
+template <int K, int CAP, bool ST>
+C2A_HD void leader_run(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane, int nl) {
   L.need_round = 0;
   L.need_score = 0;
   for (;;) {
@@ -2756,7 +2810,7 @@ C2A_HD void leader_run(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
         break;
       case ST_STEP:
         begin_step(g, L, a, lane);
-        if (L.state == ST_CONTACT_WALK) break;   // distance query
+        if (ST || L.state == ST_CONTACT_WALK) break;   // distance query
         if (a.logcap > 0 && L.nlog_prev > 0) {
           replay(g, L, a, lane, nl);
           L.state = ST_LAYOUT;
@@ -2767,37 +2821,6 @@ C2A_HD void leader_run(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
         } else {
           L.state = ST_WALK;
         }
-        break;
-      case ST_TRANS:
-        translation_query(g, L, a, lane);
-        break;
-      case ST_LAYOUT:
-        replay_layout(g, L, a, lane, nl);
-        start_scan(g, L, a, lane, nl);
-        L.state = ST_SCAN;
-        break;
-      case ST_SCAN:
-        if (scan(g, L, a, lane, nl)) {
-          L.state = ST_SUB;
-          break;
-        }
-        end_walk(g, L, a, lane, nl);
-        after_step(g, L, a, lane);
-        break;
-      case ST_SUB:
-        if (walk(g, L, a, lane, nl)) return;
-        flush_log(g, L, arena_view(L.ab, a.logcap), lane, nl);
-        if (L.flags & C2A_FLAG_STACK_OVERFLOW) {
-          end_walk(g, L, a, lane, nl);
-          after_step(g, L, a, lane);
-        } else {
-          L.state = ST_SCAN;
-        }
-        break;
-      case ST_WALK:
-        if (walk(g, L, a, lane, nl)) return;
-        end_walk(g, L, a, lane, nl);
-        after_step(g, L, a, lane);
         break;
       case ST_CONTACT_WALK:
         if (walk(g, L, a, lane, nl)) return;
@@ -2826,7 +2849,11 @@ C2A_HD void leader_run(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane, int
         L.state = ST_FETCH;
         break;
       default:
-        return;
+        if constexpr (ST) {
+          return;
+        } else if (!run_ccd_state(g, L, a, lane, nl)) {
+          return;
+        }
     }
   }
 }

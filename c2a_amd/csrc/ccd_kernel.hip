@@ -22,22 +22,24 @@ namespace c2a {
 
 // Learned order: scores of the replayed records (features in the arena,
 // 64 records per matrix-core pass); the layout then orders siblings by them.
-template <int K, int CAP>
+template <int NW, int K, int CAP>
 __device__ void score_replay(Wave<K, CAP>& g, Leader& L, const KArgs& a, int lane) {
   const ArenaView av = arena_view(L.ab, a.logcap, true);
   const int nrec = 1 + 2 * L.nlog_prev;
-  for (int base = 1; base < nrec; base += 64) {
+  const int l = lane & 63;
+  for (int base = 1 + (lane & ~63); base < nrec; base += 64 * NW) {
     // rows up to base + 63 stay inside the feature array's 64-row slack
-    const float y = score64(a.scorer, av.feat + (int64_t)base * NF, lane);
-    if (base + lane < nrec) gp(av.hot)[base + lane].score = y;
+    const float y = score64(a.scorer, av.feat + (int64_t)base * NF, l);
+    if (base + l < nrec) gp(av.hot)[base + l].score = y;
   }
   mem_sync();
 }
 
-template <int K, int CAP, int NW, bool LRN>
-__global__ void __launch_bounds__(64 * NW) ccd_kernel(KArgs a) {
+template <int K, int CAP, int NW, int V>
+__global__ void __launch_bounds__(64 * NW, V == 2 ? 2 : 1) ccd_kernel(KArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  Wave<K, CAP>& g = *reinterpret_cast<Wave<K, CAP>*>(smem_raw);
+  using W = Wave<K, CAP, V == 2>;
+  W& g = *reinterpret_cast<W*>(smem_raw);
   const int lane = threadIdx.x;
   Leader L;
   L.state = ST_FETCH;
@@ -49,9 +51,9 @@ __global__ void __launch_bounds__(64 * NW) ccd_kernel(KArgs a) {
   for (;;) {
     leader_run(g, L, a, lane, 64 * NW);
     if (L.state == ST_DONE) break;
-    if constexpr (LRN) {
+    if constexpr (V == 1) {
       if (L.need_score) {
-        score_replay(g, L, a, lane);
+        score_replay<NW>(g, L, a, lane);
         continue;
       }
     }
@@ -63,10 +65,10 @@ __global__ void __launch_bounds__(64 * NW) ccd_kernel(KArgs a) {
 // ---------------------------------------------------------------------------
 // host-side launch of this unit's shape
 // ---------------------------------------------------------------------------
-template <int K, int CAP, int NW, bool LRN>
+template <int K, int CAP, int NW, int V>
 hipError_t launch_shape(const KArgs& a, int blocks, hipStream_t s) {
-  const size_t lds = sizeof(Wave<K, CAP>);
-  auto fn = ccd_kernel<K, CAP, NW, LRN>;
+  const size_t lds = sizeof(Wave<K, CAP, V == 2>);
+  auto fn = ccd_kernel<K, CAP, NW, V>;
   hipError_t e = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)lds);
   if (e != hipSuccess) return e;
@@ -74,10 +76,10 @@ hipError_t launch_shape(const KArgs& a, int blocks, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int K, int CAP, int NW, bool LRN>
+template <int K, int CAP, int NW, int V>
 int occupancy_shape() {
-  const size_t lds = sizeof(Wave<K, CAP>);
-  auto fn = ccd_kernel<K, CAP, NW, LRN>;
+  const size_t lds = sizeof(Wave<K, CAP, V == 2>);
+  auto fn = ccd_kernel<K, CAP, NW, V>;
   if (hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
       hipSuccess)
     return 0;
@@ -89,8 +91,8 @@ int occupancy_shape() {
 #if !defined(C2A_SK) || !defined(C2A_SCAP) || !defined(C2A_SNW) || !defined(C2A_SLRN)
 #error "ccd_kernel.hip is compiled once per shape: define C2A_SK, C2A_SCAP, C2A_SNW, C2A_SLRN"
 #endif
-template hipError_t launch_shape<C2A_SK, C2A_SCAP, C2A_SNW, (C2A_SLRN != 0)>(const KArgs&, int,
+template hipError_t launch_shape<C2A_SK, C2A_SCAP, C2A_SNW, C2A_SLRN>(const KArgs&, int,
                                                                             hipStream_t);
-template int occupancy_shape<C2A_SK, C2A_SCAP, C2A_SNW, (C2A_SLRN != 0)>();
+template int occupancy_shape<C2A_SK, C2A_SCAP, C2A_SNW, C2A_SLRN>();
 
 }  // namespace c2a

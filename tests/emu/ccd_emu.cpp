@@ -99,18 +99,18 @@ extern "C" int64_t emu_samples(float* rows, int64_t* keys, int64_t cap) {
 #ifdef C2A_EMU_SIMT
 // One wavefront of 64 lanes running the kernel's loop (ccd_kernel.hip), the
 // learned order's scores computed per lane by the scalar forward pass.
-template <int K, int CAP>
+template <int K, int CAP, bool ST>
 struct SimtCtx {
   const KArgs* a;
-  Wave<K, CAP>* g;
+  Wave<K, CAP, ST>* g;
   unsigned char* ab;
 };
 
-template <int K, int CAP>
+template <int K, int CAP, bool ST>
 static void simt_body(int lane, void* p) {
-  SimtCtx<K, CAP>& c = *(SimtCtx<K, CAP>*)p;
+  SimtCtx<K, CAP, ST>& c = *(SimtCtx<K, CAP, ST>*)p;
   const KArgs& a = *c.a;
-  Wave<K, CAP>& g = *c.g;
+  Wave<K, CAP, ST>& g = *c.g;
   Leader L;
   memset(&L, 0, sizeof(L));
   L.state = ST_FETCH;
@@ -132,22 +132,22 @@ static void simt_body(int lane, void* p) {
   }
 }
 
-template <int K, int CAP>
+template <int K, int CAP, bool ST = false>
 static int run(const KArgs& a) {
   // (the tail pass of tail_left goes on in the first run's arena)
   static std::vector<unsigned char> first, second;
   std::vector<unsigned char>& arena = a.tail_pass ? second : first;
   arena.assign(a.logcap > 0 ? arena_bytes(a.logcap, a.feats != 0) : 1, 0);
-  std::unique_ptr<Wave<K, CAP>> gp(new Wave<K, CAP>());
-  memset(gp.get(), 0, sizeof(Wave<K, CAP>));
+  std::unique_ptr<Wave<K, CAP, ST>> gp(new Wave<K, CAP, ST>());
+  memset(gp.get(), 0, sizeof(Wave<K, CAP, ST>));
   g_rounds = 0;
   memset(g_kind, 0, sizeof(g_kind));
   g_scount = 0;
-  SimtCtx<K, CAP> ctx{&a, gp.get(), a.logcap > 0 ? arena.data() : nullptr};
-  return simt::launch(simt_body<K, CAP>, &ctx) ? 10 : 0;
+  SimtCtx<K, CAP, ST> ctx{&a, gp.get(), a.logcap > 0 ? arena.data() : nullptr};
+  return simt::launch(simt_body<K, CAP, ST>, &ctx) ? 10 : 0;
 }
 #else
-template <int K, int CAP>
+template <int K, int CAP, bool ST = false>
 static int run(const KArgs& a) {
   // (the tail pass of tail_left goes on in the first run's arena)
   static std::vector<unsigned char> first, second;
@@ -316,7 +316,10 @@ extern "C" int emu_distance(const double* tris1, int64_t n1, const double* tris2
   a.nq = nq;
   a.mode = MODE_DISTANCE;
   const bool small = b1.max_depth + b2.max_depth + 2 <= 48;
-  if (emu_distance_k == 7) return small ? run<7, 48>(a) : run<7, 96>(a);
+#ifdef C2A_EMU_SIMT   // the variant the library runs distance queries on
+  if (emu_distance_k == 7) return small ? run<7, 48, true>(a) : run<7, 96, true>(a);
+  if (emu_arena_rounds == 0) return small ? run<5, 48, true>(a) : run<5, 96, true>(a);
+#endif
   return small ? run<5, 48>(a) : run<5, 96>(a);
 }
 
