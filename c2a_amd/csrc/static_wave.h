@@ -13,8 +13,8 @@
 // Why: with one thread per query (static_query.h) a batch takes as long as
 // its longest search on one lane, and the lanes of a wavefront wait for each
 // other in every branch.  MI355X, host to host, two 8192-triangle knots:
-// 2048 contact lists 217 ms with one thread and 10.3 ms with one wavefront
-// per query, 4096 tolerance queries 9.1 and 2.2 ms.
+// 2048 contact lists 217 ms with one thread and 9.7 ms with one wavefront per
+// query, 4096 tolerance queries 8.0 and 0.7 ms.
 //
 // Stack bound: a batch pops the stack's top, so pairs of depth d are pushed
 // only when every deeper one has been popped, by at most 32 parents of depth
