@@ -30,6 +30,7 @@
 #include "bvh.h"
 #include "bvh_fit.h"
 #include "bvh_gpu.h"
+#include "dev_mem.h"
 
 namespace c2a {
 
@@ -590,7 +591,7 @@ struct Dev {
   ~Dev() {
     if (p) (void)hipFree(p);
   }
-  hipError_t alloc(size_t n) { return hipMalloc(&p, n ? n : 1); }
+  hipError_t alloc(size_t n) { return device_malloc(&p, n); }
 };
 
 #define BVH_TRY(expr)                    \
@@ -619,7 +620,7 @@ hipError_t build_bvh_device(const double* xyz9, const int32_t* ids, const int32_
   for (int l = 0; l < 2; l++)
     for (int c = 0; c < 3; c++) BVH_TRY(lists[l][c].alloc((size_t)n * sizeof(BuildJob)));
   BVH_TRY(counts.alloc(4 * sizeof(int32_t)));
-  BVH_TRY(hipMalloc((void**)&nodes, (size_t)nn * sizeof(GpuNode)));
+  BVH_TRY(device_malloc((void**)&nodes, (size_t)nn * sizeof(GpuNode)));
   Dev nodes_guard;
   nodes_guard.p = nodes;
   BVH_TRY(hipMemcpyAsync(src.p, xyz9, (size_t)n * 9 * sizeof(double), hipMemcpyHostToDevice, s));

@@ -9,7 +9,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
 #include <fstream>
 #include <functional>
 #include <mutex>
@@ -24,6 +23,8 @@
 #include "c2a_math.h"
 #include "ccd_core.h"
 #include "ccd_kernel.h"
+#include "dev_mem.h"
+#include "kept_pool.h"
 #include "scorer.h"
 #include "static_kernel.h"
 #include "bvh_gpu.h"
@@ -62,6 +63,57 @@ int check_device() {
   return C2A_OK;
 }
 
+struct HipMem {
+  static int alloc(void** p, size_t n) {
+    const hipError_t e = hipMalloc(p, n ? n : 1);
+    if (e == hipSuccess) return 0;
+    *p = nullptr;
+    (void)hipGetLastError();   // reported here, not by the next launch
+    return (int)e;
+  }
+  static void free(void* p) { (void)hipFree(p); }
+};
+
+// One static-query workspace per device, kept between calls: mapping and
+// unmapping 240 MB took 5 of a 7.3 ms call (4096 tolerance queries on MI355X).
+// A call takes the buffer for itself and gives it back after it has
+// synchronised its stream, so calls on other threads or streams meanwhile
+// allocate their own.  At most kKeepBytes stay, nothing once the last mesh is
+// destroyed, and every allocation of the library that does not fit beside the
+// kept memory gets it.
+KeptPool<HipMem> g_pool;
+
+}  // namespace
+
+namespace c2a {
+hipError_t device_malloc(void** p, size_t n) { return (hipError_t)g_pool.alloc(p, n); }
+}  // namespace c2a
+
+namespace {
+
+// Memory an allocation can get: what is free and what is kept (0: unknown).
+size_t free_device_bytes() {
+  int dev = 0;
+  size_t free_b = 0, total_b = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipMemGetInfo(&free_b, &total_b) != hipSuccess) return 0;
+  return free_b ? free_b + g_pool.kept(dev) : 0;
+}
+
+struct KeptBuf {
+  void* p = nullptr;
+  size_t bytes = 0;
+  int dev = -1;
+  bool idle = false;   // no work that uses it is in flight
+  int alloc(size_t n) {
+    HIP_TRY(hipGetDevice(&dev));
+    const int e = g_pool.take(dev, n, &p, &bytes);
+    return e ? hip_fail((hipError_t)e, "hipMalloc") : C2A_OK;
+  }
+  ~KeptBuf() {
+    if (p) g_pool.give(dev, p, bytes, idle);
+  }
+};
+
 // A device allocation owned by the library.
 struct DevBuf {
   void* p = nullptr;
@@ -74,7 +126,7 @@ struct DevBuf {
     if (p) (void)hipFree(p);
     p = nullptr;
     bytes = 0;
-    hipError_t e = hipMalloc(&p, n ? n : 1);
+    hipError_t e = device_malloc(&p, n);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc");
     bytes = n;
     return C2A_OK;
@@ -93,79 +145,9 @@ namespace c2a {
 int set_error(int code, const char* msg) { return fail(code, msg); }
 }  // namespace c2a
 
-namespace {
-// One static-query workspace per device, kept between calls: mapping and
-// unmapping 240 MB took 5 of a 7.3 ms call (4096 tolerance queries on MI355X).
-// A call takes the buffer for itself and gives it back after it has
-// synchronised its stream, so calls on other threads or streams meanwhile
-// allocate their own.  At most kKeepBytes stay, and nothing once the last mesh
-// is destroyed.
-constexpr size_t kKeepBytes = (size_t)512 << 20;
-constexpr int kKeepDevices = 64;
-std::mutex g_keep_mu;
-struct {
-  void* p;
-  size_t bytes;
-} g_keep[kKeepDevices];
-std::atomic<int64_t> g_meshes{0};
-
-struct KeptBuf {
-  void* p = nullptr;
-  size_t bytes = 0;
-  int dev = -1;
-  bool idle = false;   // no work that uses it is in flight
-  int alloc(size_t n) {
-    HIP_TRY(hipGetDevice(&dev));
-    if (dev >= 0 && dev < kKeepDevices) {
-      std::lock_guard<std::mutex> lock(g_keep_mu);
-      if (g_keep[dev].p && g_keep[dev].bytes >= n) {
-        p = g_keep[dev].p;
-        bytes = g_keep[dev].bytes;
-        g_keep[dev].p = nullptr;
-        return C2A_OK;
-      }
-    }
-    const hipError_t e = hipMalloc(&p, n ? n : 1);
-    if (e != hipSuccess) {
-      p = nullptr;
-      return hip_fail(e, "hipMalloc");
-    }
-    bytes = n;
-    return C2A_OK;
-  }
-  ~KeptBuf() {
-    if (!p) return;
-    void* drop = p;
-    if (idle && bytes <= kKeepBytes && dev >= 0 && dev < kKeepDevices) {
-      std::lock_guard<std::mutex> lock(g_keep_mu);
-      if (g_meshes.load() > 0 && (!g_keep[dev].p || g_keep[dev].bytes < bytes)) {
-        drop = g_keep[dev].p;
-        g_keep[dev].p = p;
-        g_keep[dev].bytes = bytes;
-      }
-    }
-    if (drop) (void)hipFree(drop);
-  }
-};
-
-void release_kept() {
-  for (int d = 0; d < kKeepDevices; d++) {
-    void* p = nullptr;
-    {
-      std::lock_guard<std::mutex> lock(g_keep_mu);
-      p = g_keep[d].p;
-      g_keep[d].p = nullptr;
-    }
-    if (p) (void)hipFree(p);
-  }
-}
-}  // namespace
-
 struct c2a_mesh {
-  c2a_mesh() { g_meshes++; }
-  ~c2a_mesh() {
-    if (--g_meshes == 0) release_kept();
-  }
+  c2a_mesh() { g_pool.hold(); }
+  ~c2a_mesh() { g_pool.release(); }
   Bvh host;
   DevBuf nodes, tris;
   int64_t ntri = 0;
@@ -1030,8 +1012,8 @@ int c2a_batch_create(c2a_mesh* const* meshes, int32_t nmesh, const c2a_query* q,
     // one replay arena per resident workgroup: fewer workgroups when the
     // device has no room for all of them
     const size_t slice = arena_bytes(b->logcap, feats);
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b > 0) {
+    const size_t free_b = free_device_bytes();
+    if (free_b > 0) {
       const size_t fit = (size_t)(0.8 * (double)free_b) / slice;
       if (fit < (size_t)b->blocks) b->blocks = (int)std::max<size_t>(1, fit);
     }
@@ -1505,9 +1487,8 @@ int static_queries(c2a_mesh* const* meshes, int32_t nmesh, int32_t kind, const d
   // workspace of one workgroup: its wavefront's, or its threads'
   const size_t group_bytes = wave ? (size_t)static_wave_bytes(kind, pair_cap, depth_sum)
                                   : (size_t)kStaticBlock * per_thread * sizeof(SqEntry);
-  size_t free_b = 0, total_b = 0;
-  size_t budget = (size_t)1 << 30;
-  if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b > 0) budget = free_b / 4;
+  const size_t free_b = free_device_bytes();
+  const size_t budget = free_b > 0 ? free_b / 4 : (size_t)1 << 30;
   int64_t blocks = wave ? nq : (nq + kStaticBlock - 1) / kStaticBlock;
   blocks = std::min<int64_t>(blocks, wave ? 2048 : 4096);
   while (blocks > 1 && (size_t)blocks * group_bytes > budget) blocks /= 2;

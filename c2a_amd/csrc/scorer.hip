@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/c2a_amd.h"
+#include "dev_mem.h"
 #include "mlp_dev.h"
 #include "scorer.h"
 
@@ -198,7 +199,7 @@ struct DevArray {
   ~DevArray() {
     if (p) (void)hipFree(p);
   }
-  bool alloc(size_t n) { return hipMalloc(&p, (n ? n : 1) * sizeof(T)) == hipSuccess; }
+  bool alloc(size_t n) { return device_malloc((void**)&p, n * sizeof(T)) == hipSuccess; }
 };
 
 ScorerDev dev_view(const c2a_scorer* s, float b3) {
@@ -248,12 +249,12 @@ int c2a_scorer_create(uint64_t seed, c2a_scorer** out) {
   c2a_scorer* s = new (std::nothrow) c2a_scorer();
   if (!s) return oom("host allocation failed");
   const size_t pb = (NPARAM + 1) * sizeof(float);
-  if (hipMalloc(&s->p, pb) != hipSuccess || hipMalloc(&s->mom, pb) != hipSuccess ||
-      hipMalloc(&s->vel, pb) != hipSuccess ||
-      hipMalloc(&s->w1, NF * NH * sizeof(uint16_t)) != hipSuccess ||
-      hipMalloc(&s->w2, NH * NH * sizeof(uint16_t)) != hipSuccess ||
-      hipMalloc(&s->w1t, NF * NH * sizeof(uint16_t)) != hipSuccess ||
-      hipMalloc(&s->w2t, NH * NH * sizeof(uint16_t)) != hipSuccess) {
+  if (device_malloc((void**)&s->p, pb) != hipSuccess || device_malloc((void**)&s->mom, pb) != hipSuccess ||
+      device_malloc((void**)&s->vel, pb) != hipSuccess ||
+      device_malloc((void**)&s->w1, NF * NH * sizeof(uint16_t)) != hipSuccess ||
+      device_malloc((void**)&s->w2, NH * NH * sizeof(uint16_t)) != hipSuccess ||
+      device_malloc((void**)&s->w1t, NF * NH * sizeof(uint16_t)) != hipSuccess ||
+      device_malloc((void**)&s->w2t, NH * NH * sizeof(uint16_t)) != hipSuccess) {
     delete s;
     return oom("scorer parameter buffers");
   }

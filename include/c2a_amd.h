@@ -379,6 +379,11 @@ int c2a_distance_queue(c2a_mesh *const *meshes, int32_t nmesh, const double *pos
                        double abs_err, int32_t qsize, int64_t nq, c2a_distance_result *out,
                        void *stream);
 
+/* c2a_distance_queue and the static queries below keep their device workspace
+ * between calls while a mesh exists: one buffer per device, at most 512 MiB.
+ * An allocation of this library that does not fit beside it gets its memory;
+ * other users of the device get it back with the last mesh. */
+
 /* Result of the static queries below.  Triangles are build-order indices
  * (caller ids through c2a_mesh_tri_ids); p1 is in model 1's frame, p2 in
  * model 2's. */

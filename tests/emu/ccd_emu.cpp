@@ -433,3 +433,47 @@ extern "C" int emu_static_wave(const double* tris1, int64_t n1, const double* tr
   return 0;
 }
 #endif
+
+// The kept workspace (kept_pool.h) over a memory of emu_pool_reset's size.
+#include <map>
+
+#include "../../c2a_amd/csrc/kept_pool.h"
+namespace {
+size_t mem_total, mem_used;
+std::map<void*, size_t> mem_live;
+struct EmuMem {
+  static int alloc(void** p, size_t n) {
+    *p = nullptr;
+    if (n > mem_total - mem_used) return 2;
+    *p = malloc(1);
+    mem_live[*p] = n;
+    mem_used += n;
+    return 0;
+  }
+  static void free(void* p) {
+    mem_used -= mem_live.at(p);
+    mem_live.erase(p);
+    ::free(p);
+  }
+};
+KeptPool<EmuMem> emu_pool;
+}  // namespace
+extern "C" void emu_pool_reset(int64_t total) {
+  emu_pool.drop();
+  mem_total = (size_t)total;
+}
+extern "C" int64_t emu_pool_used() { return (int64_t)mem_used; }
+extern "C" int64_t emu_pool_kept(int dev) { return (int64_t)emu_pool.kept(dev); }
+extern "C" void emu_pool_hold() { emu_pool.hold(); }
+extern "C" void emu_pool_release() { emu_pool.release(); }
+extern "C" int emu_pool_alloc(int64_t n, void** p) { return emu_pool.alloc(p, (size_t)n); }
+extern "C" void emu_pool_free(void* p) { EmuMem::free(p); }
+extern "C" int emu_pool_take(int dev, int64_t n, void** p, int64_t* bytes) {
+  size_t b = 0;
+  const int rc = emu_pool.take(dev, (size_t)n, p, &b);
+  *bytes = (int64_t)b;
+  return rc;
+}
+extern "C" void emu_pool_give(int dev, void* p, int64_t bytes, int idle) {
+  emu_pool.give(dev, p, (size_t)bytes, idle != 0);
+}

@@ -6,6 +6,7 @@ import threading
 
 import numpy as np
 import pytest
+import torch
 
 import c2a_amd as G
 from c2a_amd import workloads as W
@@ -55,3 +56,22 @@ def test_workspace_is_shared_safely():
     gc.collect()
     meshes = [G.Mesh(t9), G.Mesh(t9)]   # the workspace went with the last mesh
     same(ref[0], run(0))
+
+
+def test_workspace_goes_with_the_last_mesh():
+    t9 = W.torus_knot(n_seg=64, n_ring=8)[0].reshape(-1, 9)
+    P = W.knot_queries(700, 51, 0.4)
+    poses, mp = np.concatenate([P[0], P[2]], axis=1), np.tile([0, 1], (700, 1))
+    gc.collect()
+    if any(type(o) is G.Mesh for o in gc.get_objects()):
+        pytest.skip("another test's mesh is alive: the workspace rightly stays")
+    print("workspace: kept while a mesh lives, then freed", flush=True)
+    for _ in range(2):
+        meshes = [G.Mesh(t9), G.Mesh(t9)]
+        G.tolerance(meshes, poses, mp, 0.05)
+        held = torch.cuda.mem_get_info()[0]
+        del meshes
+        gc.collect()
+        freed = torch.cuda.mem_get_info()[0]
+    # 700 wavefronts' stacks of 32 pairs a level and more
+    assert freed - held > 700 * 32 * 128
