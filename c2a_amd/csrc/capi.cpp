@@ -14,8 +14,6 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "../../include/c2a_amd.h"
@@ -24,6 +22,7 @@
 #include "ccd_core.h"
 #include "ccd_kernel.h"
 #include "dev_mem.h"
+#include "host_task.h"
 #include "kept_pool.h"
 #include "scorer.h"
 #include "static_kernel.h"
@@ -680,23 +679,6 @@ struct CacheHeader {
   uint64_t src_digest, payload_digest;
 };
 static_assert(sizeof(CacheHeader) == 48, "cache header layout");
-
-// Host work that runs beside the device's: one task on its own thread (in
-// place when no thread can be made), waited for on every path.
-struct HostTask {
-  std::thread t;
-  ~HostTask() { wait(); }
-  void start(const std::function<void()>& f) {
-    try {
-      t = std::thread(f);
-    } catch (const std::system_error&) {
-      f();
-    }
-  }
-  void wait() {
-    if (t.joinable()) t.join();
-  }
-};
 
 int check_mesh_input(const double* tri_xyz9, int64_t ntri) {
   if (ntri <= 0) return fail(C2A_ERR_EMPTY_MODEL, "model has no triangles");

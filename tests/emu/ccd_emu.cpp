@@ -477,3 +477,30 @@ extern "C" int emu_pool_take(int dev, int64_t n, void** p, int64_t* bytes) {
 extern "C" void emu_pool_give(int dev, void* p, int64_t bytes, int idle) {
   emu_pool.give(dev, p, (size_t)bytes, idle != 0);
 }
+
+// A task beside the device's work (host_task.h) whose callable cannot be
+// copied (`copies` left) to its thread.  Returns how often it ran, with 16
+// added when an exception came out.
+#include "../../c2a_amd/csrc/host_task.h"
+namespace {
+struct Work {
+  int* ran;
+  int* copies;
+  Work(int* r, int* c) : ran(r), copies(c) {}
+  Work(const Work& o) : ran(o.ran), copies(o.copies) {
+    if (--*copies < 0) throw std::bad_alloc();
+  }
+  void operator()() const { ++*ran; }
+};
+}  // namespace
+extern "C" int emu_host_task(int copies) {
+  int ran = 0;
+  try {
+    HostTask task;
+    task.start(Work(&ran, &copies));
+    task.wait();
+  } catch (...) {
+    return ran + 16;
+  }
+  return ran;
+}

@@ -92,3 +92,11 @@ def test_nothing_is_kept_without_a_mesh(pool):
     assert kept(pool) == 0 and pool.emu_pool_used() == 0
     assert call(pool, 300) == 0 and kept(pool) == 0
     pool.emu_pool_hold()
+
+
+@pytest.mark.parametrize("copies", [0, 1, 2, 3, 100])
+def test_host_task_runs_once_and_throws_nothing(copies):
+    """The task beside a device build runs in place when its thread cannot be
+    made, also for want of memory: nothing is thrown at the C entry."""
+    L = C.CDLL(os.environ.get("CCD_EMU", os.path.join(HERE, "emu", "libccd_emu.so")))
+    assert L.emu_host_task(copies) == 1
