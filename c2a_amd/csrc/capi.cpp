@@ -433,11 +433,12 @@ int run_batch(const c2a_batch* b, hipStream_t s) {
 
 // Sets up the tail pass when the batch can take it: no sample logging, a stack
 // the four-wavefront shapes cover.  With tail_budget (plain order), long
-// queries are handed over by their BV tests, without their replay log.  Without, a batch that is too
-// large for four wavefronts per query hands over the last unfinished ones, one
-// per compute unit at most: at that point they are the batch's longest queries
-// and three quarters of the chip has nothing left to do, and the step costs
-// nothing where it is not needed (two counters read per CA step).
+// queries are handed over by their BV tests, without their replay log.
+// Without, a batch that is too large for four wavefronts per query hands over
+// the last unfinished ones, one per compute unit at most: at that point they
+// are the batch's longest queries and three quarters of the chip has nothing
+// left to do, and the step costs nothing where it is not needed (two counters
+// read per CA step, records for one query per compute unit).
 // MI355X (256 compute units), ms without, with 64, 128, 256 and 512 queries
 // handed over: knot 4096 259, 237, 239, 227, 233; knot 1500 225, 187, 184, 180,
 // 176; uneven 8191 202, 183, 185, 180, 183.
@@ -448,8 +449,9 @@ int setup_tail(c2a_batch* b, const c2a_params* p) {
       !kernel_shape_ok(kWideK, b->CAP, kWideWaves, 0))
     return C2A_OK;
   int rc;
-  if ((rc = b->d_tail.alloc((size_t)b->nq * sizeof(TailRec))) ||
-      (rc = b->d_tlist.alloc((size_t)b->nq * sizeof(int32_t))) ||
+  const int64_t room = last ? std::min<int64_t>(b->nq, compute_units()) : b->nq;
+  if ((rc = b->d_tail.alloc((size_t)room * sizeof(TailRec))) ||
+      (rc = b->d_tlist.alloc((size_t)room * sizeof(int32_t))) ||
       (rc = b->d_tctr.alloc(16)))
     return rc;
   KArgs& a = b->args;
@@ -458,7 +460,7 @@ int setup_tail(c2a_batch* b, const c2a_params* p) {
   a.tail_list = (int32_t*)b->d_tlist.p;
   a.tail_count = (int32_t*)((char*)b->d_tctr.p + 8);
   a.finished = a.tail_count + 1;
-  if (last) a.tail_left = compute_units();
+  if (last) a.tail_left = (int32_t)room;
   b->args2 = a;
   b->args2.tail_pass = 1;
   b->args2.counter = (int64_t*)b->d_tctr.p;

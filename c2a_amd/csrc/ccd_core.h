@@ -2271,12 +2271,21 @@ C2A_HD void finish_query(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, bool co
 }
 
 // Saves the CA-loop state of a query about to start its next step and hands
-// the query to the tail pass (the next step starts there without a replay:
-// pair values do not depend on it).
+// the query to the tail pass.  The hand-over of the last queries (tail_left)
+// passes the replay log on as well; a query handed over by its tests starts
+// its next step there without a replay (pair values do not depend on it).
+// Records are numbered by hand-over: a wavefront hands over only what few_left
+// counted as unfinished, so tail_left records hold them all.
 template <int K, int CAP, bool ST>
 C2A_HD void hand_over(const Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
   if (lane == 0) {
-    TailRec& t = a.tail_rec[L.qi];
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int at = atomicAdd(a.tail_count, 1);
+#else
+    const int at = (*a.tail_count)++;
+#endif
+    a.tail_list[at] = (int32_t)L.qi;
+    TailRec& t = a.tail_rec[at];
     t.lamda = L.lamda;
     t.lastLamda = L.lastLamda;
     t.Up = L.Up;
@@ -2294,11 +2303,6 @@ C2A_HD void hand_over(const Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int 
     t.nmiss = L.nmiss;
     // a wavefront that takes further queries writes over its arena
     t.ab = (a.tail_left > 0 && a.logcap > 0) ? L.ab : nullptr;
-#if defined(__HIP_DEVICE_COMPILE__)
-    a.tail_list[atomicAdd(a.tail_count, 1)] = (int32_t)L.qi;
-#else
-    a.tail_list[(*a.tail_count)++] = (int32_t)L.qi;
-#endif
   }
   L.state = ST_FETCH;
 }
@@ -2407,13 +2411,14 @@ C2A_HD bool fetch(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
 #endif
   }
   L.fetched = 1;
-  int64_t qi = take_ticket(g, a.counter, lane);
+  const int64_t ticket = take_ticket(g, a.counter, lane);
+  int64_t qi = ticket;
   if (a.tail_pass) {   // the first launch's hand-overs
-    if (qi >= *a.tail_count) {
+    if (ticket >= *a.tail_count) {
       L.state = ST_DONE;
       return false;
     }
-    qi = a.tail_list[qi];
+    qi = a.tail_list[ticket];
   } else if (qi >= a.nq) {
     L.state = ST_DONE;
     return false;
@@ -2571,7 +2576,7 @@ C2A_HD bool fetch(Wave<K, CAP, ST>& g, Leader& L, const KArgs& a, int lane) {
     L.flags |= C2A_FLAG_TRANSLATION_ONLY;
   L.state = (a.translation && (L.flags & C2A_FLAG_TRANSLATION_ONLY)) ? ST_TRANS : ST_STEP;
   if (a.tail_pass) {   // continue where the first launch stopped
-    const TailRec& t = a.tail_rec[qi];
+    const TailRec& t = a.tail_rec[ticket];
     L.lamda = t.lamda;
     L.lastLamda = t.lastLamda;
     L.Up = t.Up;

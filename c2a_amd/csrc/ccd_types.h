@@ -244,7 +244,7 @@ struct KArgs {
   int32_t tail_left;
   int32_t pad3;
   int32_t* finished;       // queries done (tail_left > 0)
-  TailRec* tail_rec;       // per query
+  TailRec* tail_rec;       // per hand-over
   int32_t* tail_list;      // queries handed over, in hand-over order
   int32_t* tail_count;     // their number
 };

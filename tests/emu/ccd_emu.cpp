@@ -256,8 +256,13 @@ extern "C" int emu_ccd_batch(const double* tris1, int64_t n1, const double* tris
   emu_tail_handed = 0;
   if (emu_tail_budget <= 0 && emu_tail_left <= 0) return run_shape(a);
   // two runs, as the library's two launches
-  std::vector<TailRec> rec((size_t)nq);
-  std::vector<int32_t> list((size_t)nq + 1);
+  // the hand-over of the last queries has room for tail_left of them: anything
+  // written behind that is reported
+  const size_t room = emu_tail_budget > 0 ? (size_t)nq : (size_t)std::min<int64_t>(nq, emu_tail_left);
+  TailRec mark;
+  memset(&mark, 0x5a, sizeof(mark));
+  std::vector<TailRec> rec((size_t)nq, mark);
+  std::vector<int32_t> list((size_t)nq, -77);
   int32_t count = 0;
   int32_t finished = 0;
   a.tail_budget = emu_tail_budget;
@@ -269,6 +274,8 @@ extern "C" int emu_ccd_batch(const double* tris1, int64_t n1, const double* tris
   int rc = run_shape(a);
   if (rc) return rc;
   emu_tail_handed = count;
+  for (size_t i = room; i < (size_t)nq; i++)
+    if (list[i] != -77 || memcmp(&rec[i], &mark, sizeof(mark))) return 11;
   counter = 0;
   a.tail_pass = 1;
   return run_shape(a);
