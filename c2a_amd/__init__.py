@@ -328,7 +328,8 @@ class Batch:
         return ms.value
 
     def tail_count(self):
-        """Queries the last run handed to the tail pass (0: one launch)."""
+        """Queries the last run handed to the tail pass, by tail_budget or as the
+        batch's last ones (0: one launch, or no run yet)."""
         n = C.c_int64()
         _check(lib().c2a_batch_tail_count(self.handle, C.byref(n)))
         return n.value

@@ -1070,8 +1070,9 @@ int c2a_batch_run_graph(c2a_batch* b, void* stream) {
                 "graph replay takes batches without a scorer or sample logging");
   hipStream_t s = (hipStream_t)stream;
   if (!b->graph) {
-    // capture the launch sequence (counter reset by a kernel, then the CCD
-    // kernel: no memset node) on a private stream, once per batch
+    // capture the launch sequence (counters reset by kernels, the CCD kernel and,
+    // with a tail pass, its launch: no memset node) on a private stream, once
+    // per batch
     hipStream_t cs = nullptr;
     HIP_TRY(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
@@ -1105,7 +1106,7 @@ int c2a_batch_run_graph(c2a_batch* b, void* stream) {
 int c2a_batch_tail_count(c2a_batch* b, int64_t* n) {
   if (!b || !n) return fail(C2A_ERR_BAD_ARG, "null argument");
   *n = 0;
-  if (!b->tail || b->args.tail_budget <= 0) return C2A_OK;
+  if (!b->tail || !b->timed) return C2A_OK;   // no second launch, or no run yet
   int32_t v = 0;
   HIP_TRY(hipMemcpy(&v, b->args.tail_count, sizeof(v), hipMemcpyDeviceToHost));
   *n = v;

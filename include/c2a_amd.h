@@ -67,8 +67,9 @@ typedef struct {
   double contact_offset;
   int32_t spec_depth;       /* speculative subtree depth per round, 0 = auto */
   int32_t waves_per_query;  /* wavefronts cooperating on one query: 1, or
-                               0 (default) = chosen from the batch size.  No
-                               result depends on it. */
+                               0 (default) = four with spec_depth 0 and at
+                               most four queries per compute unit, else one.
+                               No result depends on it. */
   int32_t replay_log;       /* expansions logged per CA step for the next step's
                                replay; -1 (default) = from the largest mesh
                                (8192, or ntri / 8 rounded up to a power of
@@ -83,7 +84,10 @@ typedef struct {
   int64_t sample_cap;       /* rows of the sample buffer; 0 = no logging */
   int32_t miss_depth;       /* speculative depth of the first round below a
                                replayed pair the step must expand further
-                               than the last one (default 2; 0 = spec_depth) */
+                               than the last one (default 2; 0 = spec_depth).
+                               With spec_depth 0, in the allocation-free
+                               batch too, the size bucket's autotuned value
+                               is used instead. */
   int32_t ext_levels;       /* levels computed ahead, during the replay, below
                                replayed pairs that newly pass the descend test
                                at the step's initial bound; -1 (default) = the
@@ -117,11 +121,16 @@ typedef struct {
                                tests when a CA step ends continues, from
                                that step on, in a second launch with
                                tail_waves wavefronts per query.  Results are
-                               unchanged.  0 (default) = one launch.  Plain
-                               order without sample logging only (otherwise
-                               one launch).  It pays only when a few queries
-                               run far longer than all others: the second
-                               launch starts when the first one ends. */
+                               unchanged.  > 0: plain order without sample
+                               logging only (otherwise one launch).  It pays
+                               only when a few queries run far longer than
+                               all others: the second launch starts when the
+                               first one ends.  0 (default): with spec_depth
+                               and waves_per_query 0, a batch without sample
+                               logging that is too large for four wavefronts
+                               per query hands its last unfinished queries
+                               over, one per compute unit at most, in either
+                               order; otherwise one launch. */
 } c2a_params;
 
 enum { C2A_ORDER_PLAIN = 0, C2A_ORDER_LEARNED = 1 };
@@ -261,8 +270,9 @@ int c2a_batch_create(c2a_mesh *const *meshes, int32_t nmesh, const c2a_query *q,
                      const c2a_params *params, c2a_batch **out);
 int c2a_batch_run(c2a_batch *b, void *stream);
 /* c2a_batch_run through a HIP graph: the first call captures the batch's
- * launch sequence (the work-queue reset, a kernel, then the persistent CCD
- * kernel, which runs every query's whole CA loop) and later calls replay it.
+ * launch sequence (kernels that reset the work-queue counters, then the
+ * persistent CCD kernel, which runs every query's whole CA loop, and the tail
+ * pass of a batch that has one) and later calls replay it.
  * Results are those of c2a_batch_run.  Not for batches with a scorer or
  * sample logging. */
 int c2a_batch_run_graph(c2a_batch *b, void *stream);
@@ -271,9 +281,10 @@ int c2a_batch_destroy(c2a_batch *b);
 /* Kernel-only device time of the last c2a_batch_run, in milliseconds,
  * measured with HIP events on the stream the kernel was launched on. */
 int c2a_batch_last_ms(c2a_batch *b, float *ms);
-/* Queries the last run handed to the tail pass (c2a_params.tail_budget);
- * waits for the batch's stream.  0 when the batch runs in one launch.  No
- * counterpart in the reference (diagnostics of this build's launches). */
+/* Queries the last run handed to the tail pass, by c2a_params.tail_budget or
+ * as the batch's last ones; waits for the batch's stream.  0 when the batch
+ * runs in one launch or has not run.  No counterpart in the reference
+ * (diagnostics of this build's launches). */
 int c2a_batch_tail_count(c2a_batch *b, int64_t *n);
 /* Training samples logged by the last c2a_batch_run (params->sample_cap > 0;
  * replay_log > 0): every CA step after the first replays the previous
