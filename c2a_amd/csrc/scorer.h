@@ -23,10 +23,10 @@ constexpr int P_W3 = P_B2 + NH;
 constexpr int P_B3 = P_W3 + NH;
 constexpr int NPARAM = P_B3 + 1;   // 6337
 
-// Device copy of a scorer: BF16 weights (row-major [in][out], and transposed
-// [out][in] for the traversal's register-resident pass) and FP32 biases.
+// Device copy of a scorer: BF16 weights (transposed [out][in] for the forward
+// passes, the second layer's also row-major [in][out] for the backward one) and
+// FP32 biases.
 struct ScorerDev {
-  const uint16_t* w1;   // NF x NH
   const uint16_t* w2;   // NH x NH
   const uint16_t* w1t;  // NH x NF
   const uint16_t* w2t;  // NH x NH

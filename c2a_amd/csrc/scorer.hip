@@ -119,8 +119,7 @@ __global__ void reduce_kernel(const float* partial, int nblocks, float* grad) {
 __global__ void __launch_bounds__(64) adam_kernel(float* p, float* mom, float* vel,
                                                   const float* partial, int nblocks, float* loss,
                                                   float lr, float b1, float b2, float eps, int step,
-                                                  uint16_t* w1, uint16_t* w2, uint16_t* w1t,
-                                                  uint16_t* w2t) {
+                                                  uint16_t* w2, uint16_t* w1t, uint16_t* w2t) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > NPARAM) return;
   float g = 0.0f;
@@ -139,7 +138,7 @@ __global__ void __launch_bounds__(64) adam_kernel(float* p, float* mom, float* v
   p[i] = pi;
   if (i >= P_W1 && i < P_B1) {
     const int k = i - P_W1;
-    w1[k] = w1t[(k % NH) * NF + k / NH] = f32_to_bf16(pi);
+    w1t[(k % NH) * NF + k / NH] = f32_to_bf16(pi);
   }
   if (i >= P_W2 && i < P_B2) {
     const int k = i - P_W2;
@@ -147,10 +146,10 @@ __global__ void __launch_bounds__(64) adam_kernel(float* p, float* mom, float* v
   }
 }
 
-__global__ void to_bf16_kernel(const float* p, uint16_t* w1, uint16_t* w2, uint16_t* w1t,
+__global__ void to_bf16_kernel(const float* p, uint16_t* w2, uint16_t* w1t,
                                uint16_t* w2t) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < NF * NH) w1[i] = w1t[(i % NH) * NF + i / NH] = f32_to_bf16(p[P_W1 + i]);
+  if (i < NF * NH) w1t[(i % NH) * NF + i / NH] = f32_to_bf16(p[P_W1 + i]);
   if (i < NH * NH) w2[i] = w2t[(i % NH) * NH + i / NH] = f32_to_bf16(p[P_W2 + i]);
 }
 
@@ -164,7 +163,6 @@ struct c2a_scorer {
   float* p = nullptr;       // NPARAM + 1 (the last float is b3 mirrored for the kernels)
   float* mom = nullptr;
   float* vel = nullptr;
-  uint16_t* w1 = nullptr;
   uint16_t* w2 = nullptr;
   uint16_t* w1t = nullptr;
   uint16_t* w2t = nullptr;
@@ -173,7 +171,6 @@ struct c2a_scorer {
     if (p) (void)hipFree(p);
     if (mom) (void)hipFree(mom);
     if (vel) (void)hipFree(vel);
-    if (w1) (void)hipFree(w1);
     if (w2) (void)hipFree(w2);
     if (w1t) (void)hipFree(w1t);
     if (w2t) (void)hipFree(w2t);
@@ -204,7 +201,6 @@ struct DevArray {
 
 ScorerDev dev_view(const c2a_scorer* s, float b3) {
   ScorerDev d;
-  d.w1 = s->w1;
   d.w2 = s->w2;
   d.w1t = s->w1t;
   d.w2t = s->w2t;
@@ -251,7 +247,6 @@ int c2a_scorer_create(uint64_t seed, c2a_scorer** out) {
   const size_t pb = (NPARAM + 1) * sizeof(float);
   if (device_malloc((void**)&s->p, pb) != hipSuccess || device_malloc((void**)&s->mom, pb) != hipSuccess ||
       device_malloc((void**)&s->vel, pb) != hipSuccess ||
-      device_malloc((void**)&s->w1, NF * NH * sizeof(uint16_t)) != hipSuccess ||
       device_malloc((void**)&s->w2, NH * NH * sizeof(uint16_t)) != hipSuccess ||
       device_malloc((void**)&s->w1t, NF * NH * sizeof(uint16_t)) != hipSuccess ||
       device_malloc((void**)&s->w2t, NH * NH * sizeof(uint16_t)) != hipSuccess) {
@@ -289,8 +284,8 @@ int c2a_scorer_set_params(c2a_scorer* s, const float* params) {
   (void)hipMemset(s->mom, 0, (NPARAM + 1) * sizeof(float));
   (void)hipMemset(s->vel, 0, (NPARAM + 1) * sizeof(float));
   s->step = 0;
-  hipLaunchKernelGGL(to_bf16_kernel, dim3((NH * NH + 255) / 256), dim3(256), 0, 0, s->p, s->w1,
-                     s->w2, s->w1t, s->w2t);
+  hipLaunchKernelGGL(to_bf16_kernel, dim3((NH * NH + 255) / 256), dim3(256), 0, 0, s->p, s->w2,
+                     s->w1t, s->w2t);
   return hip_err(hipDeviceSynchronize());
 }
 
@@ -425,8 +420,8 @@ int c2a_scorer_train(c2a_scorer* s, const float* feats, const float* labels, int
                          dy, didx + b0, nb_rows, rows, (float)(2.0 / (double)nb_rows), part);
       s->step++;
       hipLaunchKernelGGL(adam_kernel, dim3((NPARAM + 64) / 64), dim3(64), 0, 0, s->p, s->mom,
-                         s->vel, part, nb, loss_.p + b, lr, 0.9f, 0.999f, 1e-8f, s->step, s->w1,
-                         s->w2, s->w1t, s->w2t);
+                         s->vel, part, nb, loss_.p + b, lr, 0.9f, 0.999f, 1e-8f, s->step, s->w2,
+                         s->w1t, s->w2t);
       e = hipGetLastError();
     }
     if (e == hipSuccess)
