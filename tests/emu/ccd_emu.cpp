@@ -20,8 +20,13 @@ static int64_t g_kind[2][4];
     }                                                                        \
   } while (0)   // rounds by reason, first step / later steps
 #ifdef C2A_EMU_SIMT
-// 64 lanes on fibers (simt.cpp); rounds are counted once, by lane 0
-namespace c2a { namespace simt { int lane_id(); int launch(void (*)(int, void*), void*); } }
+// wavefronts of 64 lanes on fibers (simt.cpp); rounds are counted once, by lane 0
+namespace c2a {
+namespace simt {
+int lane_id();
+int launch(void (*)(int, void*), void*, int waves, bool backward);
+}
+}
 #define C2A_EMU_COUNT(kind, L) \
   (c2a::simt::lane_id() == 0 ? (void)g_kind[(L).numCA > 1 ? 1 : 0][kind]++ : (void)0)
 #else
@@ -96,14 +101,27 @@ extern "C" int64_t emu_samples(float* rows, int64_t* keys, int64_t cap) {
   return (int64_t)g_scount;
 }
 
+// Wavefronts per query (the 64-lane build), their order between workgroup
+// barriers, and the tail pass's shape (0: the first run's).
+static int emu_waves = 1, emu_backward = 0, emu_tail_k = 0, emu_tail_waves = 0;
+extern "C" void emu_set_waves(int waves, int backward) {
+  emu_waves = waves;
+  emu_backward = backward;
+}
+extern "C" void emu_set_tail_shape(int k, int waves) {
+  emu_tail_k = k;
+  emu_tail_waves = waves;
+}
+
 #ifdef C2A_EMU_SIMT
-// One wavefront of 64 lanes running the kernel's loop (ccd_kernel.hip), the
+// Wavefronts of 64 lanes running the kernel's loop (ccd_kernel.hip), the
 // learned order's scores computed per lane by the scalar forward pass.
 template <int K, int CAP, bool ST>
 struct SimtCtx {
   const KArgs* a;
   Wave<K, CAP, ST>* g;
   unsigned char* ab;
+  int nl;
 };
 
 template <int K, int CAP, bool ST>
@@ -116,17 +134,17 @@ static void simt_body(int lane, void* p) {
   L.state = ST_FETCH;
   L.ab = L.own = c.ab;
   for (;;) {
-    leader_run(g, L, a, lane, 64);
+    leader_run(g, L, a, lane, c.nl);
     if (L.state == ST_DONE) break;
     if (L.need_score) {
       const ArenaView av = arena_view(L.ab, a.logcap, true);
-      for (int r = 1 + lane; r < 1 + 2 * L.nlog_prev; r += 64)
+      for (int r = 1 + lane; r < 1 + 2 * L.nlog_prev; r += c.nl)
         av.hot[r].score = score_dev_scalar(a.scorer, av.feat + (int64_t)r * NF);
       mem_sync();
       continue;
     }
     if (lane == 0) g_rounds++;
-    round_lane(g, L, lane, 64, a);
+    round_lane(g, L, lane, c.nl, a);
     if (g.rarena) mem_sync();
     else lane_sync();
   }
@@ -143,8 +161,9 @@ static int run(const KArgs& a) {
   g_rounds = 0;
   memset(g_kind, 0, sizeof(g_kind));
   g_scount = 0;
-  SimtCtx<K, CAP, ST> ctx{&a, gp.get(), a.logcap > 0 ? arena.data() : nullptr};
-  return simt::launch(simt_body<K, CAP, ST>, &ctx) ? 10 : 0;
+  const int waves = a.tail_pass && emu_tail_waves ? emu_tail_waves : emu_waves;
+  SimtCtx<K, CAP, ST> ctx{&a, gp.get(), a.logcap > 0 ? arena.data() : nullptr, 64 * waves};
+  return simt::launch(simt_body<K, CAP, ST>, &ctx, waves, emu_backward != 0) ? 10 : 0;
 }
 #else
 template <int K, int CAP, bool ST = false>
@@ -278,6 +297,7 @@ extern "C" int emu_ccd_batch(const double* tris1, int64_t n1, const double* tris
     if (list[i] != -77 || memcmp(&rec[i], &mark, sizeof(mark))) return 11;
   counter = 0;
   a.tail_pass = 1;
+  if (emu_tail_k && K) K = emu_tail_k;
   return run_shape(a);
 }
 
@@ -435,7 +455,7 @@ extern "C" int emu_static_wave(const double* tris1, int64_t n1, const double* tr
   for (int64_t i = 0; i < nq; i++) {
     memset(&g, 0, sizeof(g));
     SqCtx c{&a, &g, ws.data(), i};
-    if (simt::launch(sq_body, &c)) return 10;
+    if (simt::launch(sq_body, &c, 1, false)) return 10;
   }
   return 0;
 }

@@ -1,14 +1,17 @@
-// simt.cpp -- TEST HARNESS: 64 lanes of one wavefront on the CPU.
+// simt.cpp -- TEST HARNESS: one workgroup of 64-lane wavefronts on the CPU.
 //
 // Each lane runs the kernel's per-lane code on its own fiber (ucontext).
-// The wavefront primitives of ccd_core.h (lane_sync, mem_sync, ballot,
-// shuffles, cross-lane reductions) are barriers: a lane that reaches one
-// parks; when every live lane has parked, the barrier's results are
-// computed from all lanes' inputs and the lanes run on, in lane order, to
-// their next barrier.  Between barriers the lanes therefore run one after
-// another, not in lockstep, so code that passes data between lanes through
-// memory without a barrier reads stale values here; lanes that reach
-// different primitives, or finish while others wait, are reported.
+// The wavefront primitives of ccd_core.h (ballot, shuffles, cross-lane
+// reductions) are barriers of a wavefront: a lane that reaches one parks;
+// when the wavefront's lanes have parked, the results are computed from
+// their inputs and they run on, in lane order.  lane_sync and mem_sync are
+// barriers of the workgroup: a wavefront runs on until all its lanes wait
+// there, then the next one runs, in an order the caller picks, so that
+// wavefronts are as far apart as the barriers let them.  Between barriers
+// the lanes therefore run one after another, not in lockstep, so code that
+// passes data between lanes or wavefronts through memory without a barrier
+// reads stale values here; lanes that reach different primitives, or finish
+// while others wait, are reported.
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -20,7 +23,8 @@ namespace simt {
 
 namespace {
 
-constexpr int NL = 64;
+constexpr int NL = 64;       // lanes of a wavefront
+constexpr int NW_MAX = 4;    // wavefronts of a workgroup
 constexpr size_t kStack = 8u << 20;
 enum Kind : int { NONE = 0, SYNC, BALLOT, BCAST, BCASTD, PMAX, MIND, MAXI, LANE0, DONE };
 const char* const kName[] = {"none", "sync", "ballot", "bcast", "bcastd",
@@ -35,9 +39,10 @@ struct Lane {
   int src = 0;
 };
 
-Lane lanes[NL];
+Lane group[NW_MAX * NL];
+Lane* lanes = group;   // the wavefront that runs
 ucontext_t sched;
-int cur = -1;
+int cur = -1;          // its lane
 void (*g_body)(int, void*) = nullptr;
 void* g_arg = nullptr;
 int64_t g_barriers = 0;
@@ -50,7 +55,7 @@ void arrive(int k) {
 
 void trampoline(int lane) {
   g_body(lane, g_arg);
-  lanes[lane].kind = DONE;
+  group[lane].kind = DONE;
 }
 
 void resolve(int k) {
@@ -101,7 +106,7 @@ void resolve(int k) {
 
 }  // namespace
 
-int lane_id() { return cur; }
+int lane_id() { return (int)(lanes - group) + cur; }
 int64_t barriers() { return g_barriers; }
 
 void sync() { arrive(SYNC); }
@@ -143,14 +148,39 @@ long long lane0(long long v) {
   return (long long)lanes[cur].oi;
 }
 
-// Runs body(lane, arg) on 64 lanes; 0 when every lane finished together,
-// else the lanes diverged (the message names the primitives).
-int launch(void (*body)(int, void*), void* arg) {
+// Runs wavefront w until its lanes wait at a workgroup barrier or have
+// finished; the kind they wait at, or -1 when they diverged.
+static int run_wave(int w) {
+  lanes = group + w * NL;
+  for (;;) {
+    for (int i = 0; i < NL; i++) {
+      if (lanes[i].kind != NONE) continue;
+      cur = i;
+      swapcontext(&sched, &lanes[i].ctx);
+    }
+    cur = -1;
+    const int k = lanes[0].kind;
+    for (int i = 1; i < NL; i++)
+      if (lanes[i].kind != k) {
+        fprintf(stderr, "simt: wavefront %d: lane %d at %s while lane 0 is at %s (barrier %lld)\n",
+                w, i, kName[lanes[i].kind], kName[k], (long long)g_barriers);
+        return -1;
+      }
+    if (k == SYNC || k == DONE) return k;
+    resolve(k);
+  }
+}
+
+// Runs body(lane, arg) on `waves` wavefronts, the last one first when
+// `backward`; 0 when every lane finished together, else the lanes diverged
+// (the message names the primitives).
+int launch(void (*body)(int, void*), void* arg, int waves, bool backward) {
+  if (waves < 1 || waves > NW_MAX) return 4;
   g_body = body;
   g_arg = arg;
   g_barriers = 0;
-  for (int i = 0; i < NL; i++) {
-    Lane& l = lanes[i];
+  for (int i = 0; i < waves * NL; i++) {
+    Lane& l = group[i];
     if (!l.stack) l.stack = (char*)malloc(kStack);
     if (!l.stack) return 3;
     getcontext(&l.ctx);
@@ -161,32 +191,20 @@ int launch(void (*body)(int, void*), void* arg) {
     l.kind = NONE;
   }
   for (;;) {
-    for (int i = 0; i < NL; i++) {
-      if (lanes[i].kind != NONE) continue;
-      cur = i;
-      swapcontext(&sched, &lanes[i].ctx);
+    int ndone = 0;
+    for (int i = 0; i < waves; i++) {
+      const int k = run_wave(backward ? waves - 1 - i : i);
+      if (k < 0) return 1;
+      if (k == DONE) ndone++;
     }
-    cur = -1;
-    int ndone = 0, k = -1;
-    for (int i = 0; i < NL; i++) {
-      if (lanes[i].kind == DONE) {
-        ndone++;
-        continue;
-      }
-      if (k < 0) k = lanes[i].kind;
-      else if (lanes[i].kind != k) {
-        fprintf(stderr, "simt: lane %d at %s while lane 0.. wait at %s (barrier %lld)\n", i,
-                kName[lanes[i].kind], kName[k], (long long)g_barriers);
-        return 1;
-      }
-    }
-    if (ndone == NL) return 0;
+    if (ndone == waves) return 0;
     if (ndone > 0) {
-      fprintf(stderr, "simt: %d lanes finished while %d wait at %s (barrier %lld)\n", ndone,
-              NL - ndone, kName[k], (long long)g_barriers);
+      fprintf(stderr, "simt: %d wavefronts finished while %d wait (barrier %lld)\n", ndone,
+              waves - ndone, (long long)g_barriers);
       return 2;
     }
-    resolve(k);
+    g_barriers++;
+    for (int i = 0; i < waves * NL; i++) group[i].kind = NONE;
   }
 }
 
