@@ -19,8 +19,15 @@ triple), median of three kernel timings after a warm-up.  A larger log or
 more extension levels cost arena memory and traffic, so they are taken only
 when at least MARGIN faster than the best smaller setting.  Every
 setting gives the same results bit for bit; only the time differs.  The
-chosen knobs go to tuning.json, which c2a_amd/build.py compiles into the
-library: c2a_batch_create applies them per query when spec_depth is 0.
+chosen depth and log go to tuning.json, which c2a_amd/build.py compiles into
+the library: c2a_batch_create applies them per query when spec_depth is 0.
+
+A trial gives spec_depth, so it runs one wavefront per query in one launch.
+A default batch runs other launches (four wavefronts per query, or the
+hand-over of its last queries), in which a deeper first round below a miss
+and the extension pay more: the table's miss_depth and ext_levels were timed
+there (tuning.json, "default_launches") and are kept.  --all-knobs writes the
+one-launch choice of all four.
 
     python -m c2a_amd.autotune --out c2a_amd/tuning.json
 """
@@ -118,14 +125,23 @@ def tune_bucket(meshes, queries, tol_d, tol_t, max_ntri, depths, misses, logs, e
     return best, trials
 
 
+def keep_knobs(rows, table):
+    """rows with the miss_depth and ext_levels of the table's buckets, which were
+    timed with the launches of a default batch."""
+    old = {r["max_ntri"]: r for r in table}
+    keep = ("miss_depth", "ext_levels")
+    return [dict(r, **{k: old.get(r["max_ntri"], r)[k] for k in keep}) for r in rows]
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--out", default=DEFAULT_TABLE)
     ap.add_argument("--depths", default="3,4,5,6")
-    ap.add_argument("--misses", default="1,2,3")
+    ap.add_argument("--misses", default="1,2,3,4")
     ap.add_argument("--logs", default="2048,8192,32768")
     ap.add_argument("--exts", default="0,1,2")
     ap.add_argument("--no-grazing", action="store_true")
+    ap.add_argument("--all-knobs", action="store_true")
     a = ap.parse_args()
     depths = [int(v) for v in a.depths.split(",")]
     misses = [int(v) for v in a.misses.split(",")]
@@ -174,7 +190,7 @@ def main():
             % (best["spec_depth"], best["miss_depth"], best["replay_log"], best["ext_levels"],
                best["ms"]))
     doc = json.load(open(DEFAULT_TABLE)) if os.path.exists(DEFAULT_TABLE) else {}
-    doc["buckets"] = rows
+    doc["buckets"] = rows if a.all_knobs else keep_knobs(rows, doc.get("buckets", []))
     doc["measured"] = measured
     json.dump(doc, open(a.out, "w"), indent=1)
     log("wrote %s" % a.out)
