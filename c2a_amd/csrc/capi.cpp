@@ -273,12 +273,20 @@ constexpr int kWideWaves = 4;
 // Small batches run four wavefronts per query: with one, most of the chip
 // idles while the longest queries finish; with four, the replay and the
 // rounds (up to eight heaps of pending pairs each) take four times the lanes,
-// and a compute unit holds one query instead of four.  The lines are where
-// the two met on MI355X (256 compute units), ms with one -> four wavefronts.
-// CCD, 8192-triangle knots: 1 query 127 -> 96, 256 queries 154 -> 107, 1024
-// 162 -> 127, 1536 176 -> 183, 2048 193 -> 201 (a line at 4 per compute unit).
-// Distance queries: 64 14.2 -> 9.8, 512 21.8 -> 19.6, 1024 22.4 -> 25.4 (2 per
-// compute unit).
+// and a compute unit holds one query instead of four.  MI355X (256 compute
+// units), host to host, ms.
+// CCD, one wavefront and the hand-over of the last queries -> four, a line at 4
+// per compute unit: 512 queries: knots of 8192 triangles 118 -> 116, icospheres
+// of 20,480 176 -> 162; 1024: knots of 1024 triangles 35.3 -> 36.4, of 8192
+// 130 -> 119, icospheres 174 -> 161, the uneven table 74 -> 64 (learned order:
+// 40 -> 45, 132 -> 133, icospheres 180 -> 169); 1280: 43 -> 52, 190 -> 207, 178 -> 189;
+// 1536: 46 -> 52, 139 -> 170, 185 -> 219, uneven 82 -> 67; 2048: 51 -> 71,
+// 164 -> 188, 204 -> 230, uneven 140 -> 147.
+// Contact, distance and explicit-step queries, a line at 2 per compute unit.
+// Knots of 8192 triangles, 512 queries: distance 16.9 -> 12.6, overlap 1.20 ->
+// 0.96, contacts 43.2 -> 32.5, steps 19.2 -> 14.4.  Four are ahead at 768 too
+// (14.7 -> 11.8, 1.31 -> 1.15, 48.9 -> 39.5, 17.2 -> 13.2); at 1024 distances
+// meet (17.5 -> 15.7; icospheres of 20,480 triangles 11.9 -> 13.1).
 bool wide_batch(int64_t nq, int CAP, bool ccd) {
   return nq <= (int64_t)compute_units() * (ccd ? 4 : 2) &&
          kernel_shape_ok(kWideK, CAP, kWideWaves, 0);
@@ -338,8 +346,11 @@ void tune_args(KArgs& t, int replay_log, int ext_levels, bool ext) {
   for (int r = 0; r < rows; r++) {
     t.tune_ntri[r] = kTune[r][0];
     t.tune_depth[r] = std::min(6, std::max(1, kTune[r][1]));
-    // the learned order's replays hold fewer misses: three levels below one
-    // (2048 knot queries, MI355X: 206 ms; four levels 214)
+    // The learned order takes at most three levels below a miss; four are about
+    // even.  MI355X, ms with three and four levels: knots of 8192 triangles, 2048
+    // queries 164.4 and 167.1, 512 queries 105.1 and 100.4; icospheres of 20,480
+    // triangles, 2048 queries 169.3 and 164.4; the uneven table, 8191 queries
+    // 150.4 and 144.7.
     t.tune_miss[r] = std::max(0, ext ? kTune[r][2] : std::min(3, kTune[r][2]));
     t.tune_log[r] = replay_log >= 0 ? replay_log : kTune[r][3];
     t.tune_ext[r] = ext_levels >= 0 ? std::min(8, ext_levels)

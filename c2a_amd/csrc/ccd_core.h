@@ -2,16 +2,18 @@
 // gfx950 kernel (ccd_kernel.hip) and the host-side test harness that runs the
 // same code with a single lane.
 //
-// One wavefront per query.  All lanes run the walk of the reference's DFS
-// (TOCStepRecurse_Dis, C2A.cpp:1113-1354) in lockstep over a stack in LDS, so
-// every prune/descend/leaf decision is made in reference order with uniform
-// control flow; stack entries are copied one 8-byte word per lane.  When the
-// walk needs pair values it does not have, the lanes compute a speculative
-// depth-K subtree below that pair in one round (round_lane): lane j chains the
-// child transforms down to heap slot j+1 and evaluates the RSS distance, the
-// directional motion bound and, for leaf pairs, the triangle distance.  Pair
-// values never depend on the traversal state, so speculation cannot change a
-// result; it only lets one round feed up to K levels of the walk.
+// One workgroup per query, of one wavefront (large batches) or four (small
+// ones, a batch's last queries); with four, every wavefront makes the same
+// decisions, and the lanes of all of them share a round's slots and the replay.
+// Every prune/descend/leaf decision of the reference's DFS
+// (TOCStepRecurse_Dis, C2A.cpp:1113-1354) is made in reference order with
+// uniform control flow over a stack in LDS.  When the walk needs pair values it
+// does not have, the lanes compute a speculative subtree (a heap) below that
+// pair, and below other pending pairs, in one round (round_lane): a lane chains
+// the child transforms down to its heap slot and evaluates the RSS distance, the
+// directional motion bound and, for leaf pairs, the triangle distance; then
+// the lanes decide a heap at once (heap_scan).  Pair values never depend on the
+// traversal state, so speculation cannot change a result.
 //
 // Replay: the walk logs every expansion of a CA step.  At the next step the
 // lanes first recompute the logged subtree at the new poses, one BVTT level
@@ -39,8 +41,8 @@
 namespace c2a {
 
 #if !defined(__HIP_DEVICE_COMPILE__) && defined(C2A_EMU_SIMT)
-// Host-side test harness with 64 lanes (tests/emu/ccd_emu64.cpp): each lane
-// runs on its own fiber and the wavefront primitives below are barriers
+// Host-side test harness with wavefronts of 64 lanes (tests/emu/simt.cpp): each
+// lane runs on its own fiber and the wavefront primitives below are barriers
 // that exchange the lanes' values.
 namespace simt {
 void sync();

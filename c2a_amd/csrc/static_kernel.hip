@@ -1,6 +1,7 @@
-// static_kernel.hip -- the static proximity queries of static_query.h on
-// gfx950: one thread per query, threads take queries from a device work
-// queue until it drains, each with its own slice of the workspace.
+// static_kernel.hip -- the static proximity queries on gfx950: one wavefront
+// per query where static_wave.h takes the search, else one thread per query
+// (static_query.h).  Both take queries from a device work queue until it
+// drains, each wavefront or thread with its own slice of the workspace.
 #include <hip/hip_runtime.h>
 
 #include "static_query.h"

@@ -13,8 +13,11 @@
 // Why: with one thread per query (static_query.h) a batch takes as long as
 // its longest search on one lane, and the lanes of a wavefront wait for each
 // other in every branch.  MI355X, host to host, two 8192-triangle knots:
-// 2048 contact lists 217 ms with one thread and 9.7 ms with one wavefront per
-// query, 4096 tolerance queries 8.0 and 0.7 ms.
+// 2048 contact lists 194 ms with one thread and 8.9 ms with one wavefront per
+// query, 4096 tolerance queries 8.0 and 0.7 ms (with the workspace kept
+// between calls).  A single query is one lane's search against 32 pairs a turn
+// and a second pass for the counts: 24 contact-space queries one by one 0.87
+// and 0.27 ms on average, the shortest 0.16 and 0.22.
 //
 // Stack bound: a batch pops the stack's top, so pairs of depth d are pushed
 // only when every deeper one has been popped, by at most 32 parents of depth
@@ -118,7 +121,7 @@ C2A_HD void sq_wave_search(const StaticArgs& a, SqWaveLds& g, const MeshDev& M1,
     if (!root) {
       const int np = n < 32 ? n : 32;
       act = (lane >> 1) < np;
-      C2A_CHECK(n <= sq_wave_stack(kSqWaveDepth));
+      C2A_CHECK(n <= sq_wave_stack(a.depth_sum));
       const SqWaveEntry C2A_GLOBAL* e = gp(st) + (n - 1 - (act ? lane >> 1 : 0));
       for (int i = 0; i < 9; i++) R[i] = e->R[i];
       for (int i = 0; i < 3; i++) T[i] = e->T[i];
