@@ -1,7 +1,8 @@
 """Benchmark: batched conservative-advancement CCD on one MI355X.
 
-One step = one launch of the CCD kernel over the whole query batch (every
-query runs its full CA loop: the reference's C2A_QueryTimeOfContact).  The
+One step = one run of the whole query batch (every query runs its full CA loop:
+the reference's C2A_QueryTimeOfContact; the CCD kernel's launch, then a second
+one over the batch's last queries).  The
 workload is the knot-pair batch: two (2,3) torus-knot tubes of 8192 FP64
 triangles each, 4096 independent queries with seeded poses (translation
 U[-2,2]^3, uniform random rotation), about 30% of them colliding (end poses
