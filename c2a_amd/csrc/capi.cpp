@@ -9,6 +9,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <exception>
 #include <fstream>
 #include <functional>
 #include <mutex>
@@ -855,7 +856,7 @@ int c2a_mesh_load(const char* path, const double* tri_xyz9, const int32_t* tri_i
   return C2A_OK;
 }
 
-int c2a_mesh_refit(c2a_mesh* m, const double* tri_xyz9, int32_t on_device, void* stream) {
+int c2a_mesh_refit(c2a_mesh* m, const double* tri_xyz9, int32_t on_device, void* stream) try {
   if (!m || !tri_xyz9) return fail(C2A_ERR_BAD_ARG, "null argument");
   if ((int64_t)m->host.src_index.size() != m->ntri)
     return fail(C2A_ERR_BAD_ARG, "mesh has no source order");
@@ -892,6 +893,8 @@ int c2a_mesh_refit(c2a_mesh* m, const double* tri_xyz9, int32_t on_device, void*
   task.wait();
   m->src_digest = on_device ? digest : digest_bytes(d0, tri_xyz9, bytes);
   return C2A_OK;
+} catch (const std::exception&) {   // a host array of this size cannot be had
+  return fail(C2A_ERR_OOM, "host allocation failed");
 }
 
 int c2a_mesh_destroy(c2a_mesh* m) {
@@ -961,7 +964,7 @@ int c2a_batch_create(c2a_mesh* const* meshes, int32_t nmesh, const c2a_query* q,
       delete b;
       return rc;
     }
-  } catch (const std::bad_alloc&) {
+  } catch (const std::exception&) {
     delete b;
     return fail(C2A_ERR_OOM, "host allocation failed");
   }
@@ -1143,7 +1146,7 @@ int c2a_batch_last_ms(c2a_batch* b, float* ms) {
 }
 
 int c2a_batch_samples(c2a_batch* b, float* feats, float* labels, int64_t* keys, int64_t cap,
-                      int64_t* n_out, int64_t* n_written) {
+                      int64_t* n_out, int64_t* n_written) try {
   if (!b || cap < 0 || (cap > 0 && (!feats || !labels || !keys)))
     return fail(C2A_ERR_BAD_ARG, "bad sample buffers");
   if (b->sample_cap <= 0) return fail(C2A_ERR_BAD_ARG, "the batch logs no samples");
@@ -1177,6 +1180,8 @@ int c2a_batch_samples(c2a_batch* b, float* feats, float* labels, int64_t* keys, 
   if (n_out) *n_out = (int64_t)cnt;
   if (n_written) *n_written = w;
   return C2A_OK;
+} catch (const std::exception&) {   // a host array of this size cannot be had
+  return fail(C2A_ERR_OOM, "host allocation failed");
 }
 
 int c2a_batch_destroy(c2a_batch* b) {
@@ -1197,7 +1202,7 @@ int c2a_ccd_batch(c2a_mesh* const* meshes, int32_t nmesh, const c2a_query* q, in
 }
 
 int c2a_ccd_step(c2a_mesh* const* meshes, int32_t nmesh, const c2a_step_query* q, int64_t nq,
-                 c2a_step_result* out, void* stream) {
+                 c2a_step_result* out, void* stream) try {
   if (nq < 0 || (nq > 0 && (!q || !out))) return fail(C2A_ERR_BAD_ARG, "bad arrays");
   if (nq == 0) return C2A_OK;
   int rc = check_device();
@@ -1258,11 +1263,13 @@ int c2a_ccd_step(c2a_mesh* const* meshes, int32_t nmesh, const c2a_step_query* q
   HIP_TRY(hipMemcpyAsync(out, dout.p, (size_t)nq * sizeof(c2a_step_result), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   return C2A_OK;
+} catch (const std::exception&) {   // a host array of this size cannot be had
+  return fail(C2A_ERR_OOM, "host allocation failed");
 }
 
 static int contact_queries(c2a_mesh* const* meshes, int32_t nmesh, const double* poses,
                            const int32_t* mesh_pairs, const double* thresholds, int64_t nq,
-                           int32_t cap, c2a_contact* out, int32_t* counts_out, void* stream) {
+                           int32_t cap, c2a_contact* out, int32_t* counts_out, void* stream) try {
   if (nq < 0 || (nq > 0 && (!poses || !mesh_pairs || !thresholds || !counts_out)))
     return fail(C2A_ERR_BAD_ARG, "bad arrays");
   if (cap < 0 || (cap > 0 && !out)) return fail(C2A_ERR_BAD_ARG, "bad contact buffer");
@@ -1335,6 +1342,8 @@ static int contact_queries(c2a_mesh* const* meshes, int32_t nmesh, const double*
     }
   }
   return C2A_OK;
+} catch (const std::exception&) {   // a host array of this size cannot be had
+  return fail(C2A_ERR_OOM, "host allocation failed");
 }
 
 int c2a_contact_count(c2a_mesh* const* meshes, int32_t nmesh, const double* poses,
@@ -1354,7 +1363,7 @@ int c2a_contact_list(c2a_mesh* const* meshes, int32_t nmesh, const double* poses
 static int distance_queries(c2a_mesh* const* meshes, int32_t nmesh, const double* poses,
                             const int32_t* mesh_pairs, const int32_t* seed_tris, double rel_err,
                             double abs_err, int64_t nq, c2a_distance_result* out, void* stream,
-                            int overlap_only) {
+                            int overlap_only) try {
   if (nq < 0 || (nq > 0 && (!poses || !mesh_pairs || !out)))
     return fail(C2A_ERR_BAD_ARG, "bad arrays");
   if (!(rel_err >= 0) || !(abs_err >= 0))
@@ -1415,6 +1424,8 @@ static int distance_queries(c2a_mesh* const* meshes, int32_t nmesh, const double
                          hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   return C2A_OK;
+} catch (const std::exception&) {   // a host array of this size cannot be had
+  return fail(C2A_ERR_OOM, "host allocation failed");
 }
 
 int c2a_distance(c2a_mesh* const* meshes, int32_t nmesh, const double* poses,
@@ -1441,7 +1452,7 @@ static_assert(sizeof(StaticOut) == sizeof(c2a_static_result), "static result lay
 int static_queries(c2a_mesh* const* meshes, int32_t nmesh, int32_t kind, const double* poses,
                    const int32_t* mesh_pairs, const int32_t* seed_tris, const double* params,
                    double rel_err, double abs_err, int32_t qsize, int32_t flag, int64_t nq,
-                   int32_t pair_cap, int32_t* pairs_out, void* out, void* stream) {
+                   int32_t pair_cap, int32_t* pairs_out, void* out, void* stream) try {
   if (nq < 0 || (nq > 0 && (!poses || !mesh_pairs || !out)))
     return fail(C2A_ERR_BAD_ARG, "bad arrays");
   if (nq > 0 && (kind == SQ_DISTANCE_CS || kind == SQ_TOLERANCE) && !params)
@@ -1556,6 +1567,8 @@ int static_queries(c2a_mesh* const* meshes, int32_t nmesh, int32_t kind, const d
   HIP_TRY(hipStreamSynchronize(s));
   dws.idle = true;
   return C2A_OK;
+} catch (const std::exception&) {   // a host array of this size cannot be had
+  return fail(C2A_ERR_OOM, "host allocation failed");
 }
 
 }  // namespace
